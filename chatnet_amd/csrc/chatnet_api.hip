@@ -121,13 +121,19 @@ std::vector<char*> g_ws_retired;
 // every launch leaves them zero.
 constexpr size_t kMatmulCounterBytes = (size_t)kGemmTileCounters * sizeof(unsigned);
 
-int matmul_workspace(int dev, hipStream_t st, size_t bytes, char** out) {
+// With `grown`, a capturing stream whose workspace is too small is no error:
+// *grown is false and the caller runs a path without one.
+int matmul_workspace(int dev, hipStream_t st, size_t bytes, char** out, bool* grown = nullptr) {
   std::lock_guard<std::mutex> lk(g_ws_mu);
   auto& e = g_ws[{dev, st}];
   bytes = std::max(bytes, kMatmulCounterBytes);
   if (e.second < bytes) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     HIP_TRY(hipStreamIsCapturing(st, &cs));
+    if (cs != hipStreamCaptureStatusNone && grown) {
+      *grown = false;
+      return CHATNET_OK;
+    }
     if (cs != hipStreamCaptureStatusNone)
       return fail(CHATNET_ERR_INVALID_ARG,
                   "chatnet_matmul: the stream is capturing and its workspace (%zu bytes) is smaller than the %zu "
@@ -1106,6 +1112,60 @@ int run_prompt(chatnet_model* m, const int32_t* tokens, int n, int position) {
   return CHATNET_OK;
 }
 
+// F32 / F16 rows with several columns.  One launch of the multi-column GEMV takes
+// the columns whose fp32 x fits in LDS (8 up to K = 4864, 3 at 11008); F16 with
+// more of them runs the span kernel's exact-weight F16 product (W * xh + W *
+// xl, x as two fp16 planes, fp32 sums) out of the stream's workspace, three
+// launches whatever N is: F16 4096 x 4096 at 8 columns 20.5 us in one GEMV
+// launch and 25.1 us as a product, at 24 columns 140 us column by column and
+// 26 us; 2048 x 11008 at 7 columns 44 us in three GEMV launches.  F32, a
+// capturing stream whose workspace is too small and the no-allocation variant
+// (which takes these types without scratch, so overlapping calls are safe) run
+// the multi-column GEMV for any N.
+int matmul_float(int type, const void* w, const float* x, float* y, int M, int K, int N, int dev, int cus,
+                 hipStream_t st, bool noalloc) {
+  if (type == CHATNET_GGML_F16 && N >= 4 && N > gemv_float_cols_max(K) && !noalloc) {
+    const size_t plane = ((size_t)N * K * sizeof(uint16_t) + 255) & ~(size_t)255;
+    const size_t scales = ((size_t)N * sizeof(float) + 255) & ~(size_t)255;
+    const size_t part = gemm_workspace_bytes(M, N, K, cus, true, GEMM_W_F16);
+    char* ws = nullptr;
+    bool ok = true;
+    const int rc = matmul_workspace(dev, st, kMatmulCounterBytes + 2 * plane + scales + part, &ws, &ok);
+    if (rc) return rc;
+    if (ok) {
+      uint16_t* xh = (uint16_t*)(ws + kMatmulCounterBytes);
+      uint16_t* xl = (uint16_t*)((char*)xh + plane);
+      float* xinv = (float*)((char*)xl + plane);
+      HIP_TRY(to_f16_planes_launch(x, xh, xl, xinv, N, K, st));
+      GemmArgs g;
+      memset(&g, 0, sizeof(g));
+      g.qtype = type;
+      g.packed = GEMM_W_F16;
+      g.precise = 1;
+      g.w[0] = g.w[1] = g.w[2] = (const uint8_t*)w;
+      g.seg_rows[0] = M;
+      g.seg_mode = GEMM_SEG_SINGLE;
+      g.M = M;
+      g.K = K;
+      g.N = N;
+      g.xb = xh;
+      g.xb_lo = xl;
+      g.xinv = xinv;
+      g.x32 = x;
+      g.epi = GEMV_EPI_STORE;
+      g.y = y;
+      g.ldy = M;
+      g.part = part ? (float*)((char*)xinv + scales) : nullptr;
+      HIP_TRY(gemm_launch(g, cus, st));
+      g_err.clear();
+      return CHATNET_OK;
+    }
+  }
+  HIP_TRY(gemv_float_cols_launch(type, w, x, y, M, K, N, cus, st));
+  g_err.clear();
+  return CHATNET_OK;
+}
+
 // chatnet_matmul and chatnet_matmul_noalloc: the same kernels; the batched
 // path's scratch (fp16 x and its column scales, then the K-split partials) comes from the per-stream
 // workspace, or with `noalloc` from the fixed per-device scratch array.
@@ -1137,6 +1197,8 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
     g_err.clear();
     return CHATNET_OK;
   }
+  if ((type == CHATNET_GGML_F32 || type == CHATNET_GGML_F16) && N >= 2)
+    return matmul_float((int)type, w_dev, x_dev, y_dev, M, K, N, dev, cus, st, noalloc);
   const bool raw = gemm_supports((int)type, K);
   const bool must_pack = gemv_needs_pack((int)type);
   const bool batched = N >= 8 && (raw || must_pack || (!noalloc && gemm_pack_supports((int)type, K)));

@@ -28,6 +28,15 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// s += v element by element, the rounding error of the sum so far carried in c.
+template <class V>
+__device__ __forceinline__ void add_compensated(V& s, V& c, const V& v) {
+  const V y = v - c;
+  const V t = s + y;
+  c = (t - s) - y;
+  s = t;
+}
+
 // W rows of the virtual row `vr`: single matrix, three concatenated (q|k|v)
 // or two interleaved (gate even, up odd).
 __device__ __forceinline__ const uint32_t* gemm_row_ptr(const GemmArgs& a, int vr, int row_dw) {
@@ -69,6 +78,18 @@ __device__ __forceinline__ void write_h(const GemmArgs& a, int n, int j, float v
   a.hb_lo[i] = (uint16_t)lo;
 }
 
+// An output of chatnet_matmul's F16 rows that came out NaN, summed again from
+// the fp32 x: in two planes an infinite weight meets x's low part too (inf * 0
+// or inf - inf), where the plain product is infinite.  Never taken for finite
+// operands.
+__device__ __attribute__((noinline)) float f16_dot_again(const GemmArgs& a, int n, int m) {
+  const _Float16* w = reinterpret_cast<const _Float16*>(a.w[0]) + (size_t)m * a.K;
+  const float* x = a.x32 + (size_t)n * a.K;
+  float s = 0.f;
+  for (int k = 0; k < a.K; k++) s = fmaf((float)w[k], x[k], s);
+  return s;
+}
+
 // Final write of 4 consecutive rows m..m+3 of column n.
 __device__ __forceinline__ void write_out4(const GemmArgs& a, int epi, int n, int m, f32x4 v) {
   if (n >= a.N || m >= a.M) return;
@@ -87,6 +108,13 @@ __device__ __forceinline__ void write_out4(const GemmArgs& a, int epi, int n, in
       write_h(a, n, m >> 1, silu_mul(v[0], v[1]));
     }
     return;
+  }
+  if (a.x32) {
+    const float t = (v[0] + v[1]) + (v[2] + v[3]);
+    if (!(t == t)) {
+      for (int i = 0; i < 4 && m + i < a.M; i++)
+        if (!(v[i] == v[i])) v[i] = f16_dot_again(a, n, m + i);
+    }
   }
   float* y = a.y + (size_t)n * a.ldy + m;
   if (full) {
@@ -753,7 +781,13 @@ __global__ __launch_bounds__(CN_BLOCK) __attribute__((amdgpu_waves_per_eu(SK ? 2
 // fp16 MFMAs per step: Wa*xh + Wa*xl + Wb*xh, W = Wa + Wb exact for Q4_0 (~22
 // bits for packed units), x = xh + xl to ~2^-22; the dropped Wb*xl term is
 // below 2^-19 relative.
-template <int TN, int S, int WF>
+//
+// COMP (chatnet_matmul's F16 rows): every chunk's eight MFMA steps start from
+// zero and the chunk sums are added with a running compensation (Kahan), so
+// the product rounds no worse than the fp32 GEMV whose place it takes
+// (relative error against float64 at K = 4096: GEMV 1.0e-7, one accumulator
+// 5.9e-7, this 0.8e-7).
+template <int TN, int S, int WF, bool COMP = false>
 __global__ __launch_bounds__(CN_BLOCK) void gemm_s_kernel(GemmArgs a) {
   using C = PipeCfg<true, TN, S, WF>;
   constexpr bool PK = C::PK;
@@ -766,6 +800,11 @@ __global__ __launch_bounds__(CN_BLOCK) void gemm_s_kernel(GemmArgs a) {
   for (int cc = 0; cc < TN; cc++)
 #pragma unroll
     for (int v = 0; v < 16; v++) acc[cc][v] = 0.f;
+  f32x16 sum[COMP ? TN : 1], com[COMP ? TN : 1];
+  if constexpr (COMP) {
+#pragma unroll
+    for (int cc = 0; cc < TN; cc++) sum[cc] = com[cc] = acc[cc];
+  }
 
   // v_perm_b32 selectors: qs dword s of the lane's block (2 bytes into the
   // unit for block A) as bytes b0 b2 b1 b3; 0x64006400 kept in a register
@@ -825,6 +864,26 @@ __global__ __launch_bounds__(CN_BLOCK) void gemm_s_kernel(GemmArgs a) {
           xl[b][cc] = __builtin_bit_cast(f16x8, io.xfrag(st, 1, s, cc));
         }
       };
+      if constexpr (COMP) {
+        // the low plane's four products first, while the sum is still 2^-12 of
+        // the chunk's: their rounding then does not count
+#pragma unroll
+        for (int p = 1; p >= 0; p--)
+#pragma unroll
+          for (int s = 0; s < 4; s++) {
+            const f16x8 wa =
+                __builtin_bit_cast(f16x8, (cn_u32x4){w[2 * s], w[2 * s + 1], w[8 + 2 * s], w[9 + 2 * s]});
+#pragma unroll
+            for (int cc = 0; cc < TN; cc++)
+              acc[cc] = mma32(wa, __builtin_bit_cast(f16x8, io.xfrag(st, p, s, cc)), acc[cc]);
+          }
+#pragma unroll
+        for (int cc = 0; cc < TN; cc++) {
+          add_compensated(sum[cc], com[cc], acc[cc]);
+          acc[cc] = f32x16{};
+        }
+        continue;
+      }
       load_x(0, 0);
 #pragma unroll
       for (int s = 0; s < 4; s++) {
@@ -870,7 +929,8 @@ __global__ __launch_bounds__(CN_BLOCK) void gemm_s_kernel(GemmArgs a) {
   }
   float sc[TN];
   io.template load_scales<TN>(a, sc);
-  io.template store<TN>(a, acc, sc);
+  if constexpr (COMP) io.template store<TN>(a, sum, sc);
+  else io.template store<TN>(a, acc, sc);
 }
 
 // Sums the K-split partials [splits][N][M] and applies the epilogue; one
@@ -880,14 +940,17 @@ __global__ __launch_bounds__(CN_BLOCK) void gemm_reduce_kernel(GemmArgs a) {
   const long long t = (long long)blockIdx.x * CN_BLOCK + threadIdx.x;
   if (t >= (long long)m4 * a.N) return;
   const int n = (int)(t / m4), m = (int)(t % m4) * 4;
-  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+  f32x4 s = {0.f, 0.f, 0.f, 0.f}, c = s;
   for (int k = 0; k < a.splits; k++) {
     const float* p = a.part + ((size_t)k * a.N + n) * a.M + m;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
     if (m + 3 < a.M && (a.M & 3) == 0) {
-      s += *reinterpret_cast<const f32x4*>(p);
+      v = *reinterpret_cast<const f32x4*>(p);
     } else {
-      for (int i = 0; i < 4 && m + i < a.M; i++) s[i] += p[i];
+      for (int i = 0; i < 4 && m + i < a.M; i++) v[i] = p[i];
     }
+    if (a.x32) add_compensated(s, c, v);
+    else s += v;
   }
   write_out4(a, a.epi, n, m, s);
 }
@@ -933,6 +996,58 @@ __global__ __launch_bounds__(CN_BLOCK) void to_f16_scaled_kernel(const float* __
     const cn_half2 b = __builtin_convertvector((cn_float2){y[2], y[3]}, cn_half2);
     *reinterpret_cast<uint2*>(o + cn_span_pos(i)) =
         make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
+  }
+}
+
+// x [N][K] fp32 -> the span kernel's two planes with the per-column scaling of
+// to_f16_scaled_kernel (the largest finite |x| in [2^14, 2^15)): hi = fp16(x *
+// 2^e), lo = fp16(x * 2^e - hi), together within 2^-24 of the element (lo's own
+// subnormals start 2^-39 below the column's largest).  An infinity keeps lo = 0.
+template <int V>
+__global__ __launch_bounds__(CN_BLOCK) void to_f16_planes_kernel(const float* __restrict__ x,
+                                                                uint16_t* __restrict__ xh, uint16_t* __restrict__ xl,
+                                                                float* __restrict__ xinv, int K) {
+  __shared__ float red[4];
+  const size_t n = blockIdx.x;
+  const float* xr = x + n * K;
+  f32x4 v[V];
+  float mx = 0.f;
+#pragma unroll
+  for (int j = 0; j < V; j++) {
+    const int i = (threadIdx.x + CN_BLOCK * j) * 4;
+    v[j] = i < K ? *reinterpret_cast<const f32x4*>(xr + i) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const float m = fabsf(v[j][q]);
+      mx = m <= 3.402823466e38f ? fmaxf(mx, m) : mx;  // finite elements only
+    }
+  }
+  mx = cn_block_max(mx, red);
+  int e = 0;
+  if (mx > 0.f) {
+    int E;
+    (void)frexpf(mx, &E);  // mx = f * 2^E, f in [0.5, 1)
+    e = min(125, max(-125, 15 - E));
+  }
+  if (threadIdx.x == 0) xinv[n] = ldexpf(1.0f, -e);
+  const float sc = ldexpf(1.0f, e);
+#pragma unroll
+  for (int j = 0; j < V; j++) {
+    const int i = (threadIdx.x + CN_BLOCK * j) * 4;
+    if (i >= K) continue;
+    const f32x4 y = v[j] * sc;  // 2^e is a normal float for e in [-125, 125]
+    _Float16 hi[4], lo[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      hi[q] = (_Float16)y[q];
+      const float r = y[q] - (float)hi[q];
+      lo[q] = fabsf(y[q]) <= 3.402823466e38f ? (_Float16)r : (_Float16)0.f;
+    }
+    const size_t o = n * K + cn_span_pos(i);  // four adjacent elements stay adjacent
+    *reinterpret_cast<uint2*>(xh + o) = make_uint2(__builtin_bit_cast(uint32_t, (cn_half2){hi[0], hi[1]}),
+                                                   __builtin_bit_cast(uint32_t, (cn_half2){hi[2], hi[3]}));
+    *reinterpret_cast<uint2*>(xl + o) = make_uint2(__builtin_bit_cast(uint32_t, (cn_half2){lo[0], lo[1]}),
+                                                   __builtin_bit_cast(uint32_t, (cn_half2){lo[2], lo[3]}));
   }
 }
 
@@ -1428,16 +1543,19 @@ hipError_t launch_p_ring(const GemmArgs& a, int mt, int grid, hipStream_t st) {
   return launch_p<TN, S, PK, 1>(a, grid, st);
 }
 
-template <int TN, int S, int WF>
+template <int TN, int S, int WF, bool COMP = false>
 hipError_t launch_s(const GemmArgs& a, int grid, hipStream_t st) {
+  if constexpr (WF == GEMM_W_F16 && !COMP) {
+    if (a.x32) return launch_s<TN, S, WF, true>(a, grid, st);
+  }
   constexpr int lds = PipeCfg<true, TN, S, WF>::LDS;
   static_assert(lds <= 160 * 1024, "LDS ring exceeds the CU's 160 KB");
   static std::atomic<uint64_t> lds_done{0};
   if (lds > 64 * 1024) {
-    const hipError_t e = allow_full_lds(reinterpret_cast<const void*>(&gemm_s_kernel<TN, S, WF>), lds_done);
+    const hipError_t e = allow_full_lds(reinterpret_cast<const void*>(&gemm_s_kernel<TN, S, WF, COMP>), lds_done);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((gemm_s_kernel<TN, S, WF>), dim3(grid), dim3(CN_BLOCK), lds, st, a);
+  hipLaunchKernelGGL((gemm_s_kernel<TN, S, WF, COMP>), dim3(grid), dim3(CN_BLOCK), lds, st, a);
   return hipGetLastError();
 }
 
@@ -1564,6 +1682,17 @@ hipError_t to_f16_scaled_launch(const float* x, uint16_t* xh, float* xinv, int N
   else if (v <= 4) hipLaunchKernelGGL((to_f16_scaled_kernel<4>), grid, block, 0, st, x, xh, xinv, K);
   else if (v <= 8) hipLaunchKernelGGL((to_f16_scaled_kernel<8>), grid, block, 0, st, x, xh, xinv, K);
   else hipLaunchKernelGGL((to_f16_scaled_kernel<16>), grid, block, 0, st, x, xh, xinv, K);
+  return hipGetLastError();
+}
+
+hipError_t to_f16_planes_launch(const float* x, uint16_t* xh, uint16_t* xl, float* xinv, int N, int K, hipStream_t st) {
+  if (N <= 0 || K <= 0 || K % 32 || K > 16384) return hipErrorInvalidValue;
+  const int v = (K + 4 * CN_BLOCK - 1) / (4 * CN_BLOCK);  // float4 per thread
+  const dim3 grid(N), block(CN_BLOCK);
+  if (v <= 2) hipLaunchKernelGGL((to_f16_planes_kernel<2>), grid, block, 0, st, x, xh, xl, xinv, K);
+  else if (v <= 4) hipLaunchKernelGGL((to_f16_planes_kernel<4>), grid, block, 0, st, x, xh, xl, xinv, K);
+  else if (v <= 8) hipLaunchKernelGGL((to_f16_planes_kernel<8>), grid, block, 0, st, x, xh, xl, xinv, K);
+  else hipLaunchKernelGGL((to_f16_planes_kernel<16>), grid, block, 0, st, x, xh, xl, xinv, K);
   return hipGetLastError();
 }
 

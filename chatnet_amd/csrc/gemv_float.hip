@@ -18,6 +18,8 @@
 // GEMV's (gemv_common.h): store, residual add, QKV + RoPE + KV-cache write,
 // SiLU(gate)*up on interleaved rows, LM head, and the attention merge folded
 // into the O projection's x staging.
+#include <cstring>
+
 #include "device_common.h"
 #include "gemv_common.h"
 #include "kernels.h"
@@ -141,6 +143,110 @@ __global__ __launch_bounds__(CN_BLOCK) void gemv_f_kernel(GemvArgs a) {
     for (int i = 0; i < RPW; i++) acc[i] = cn_wave_sum(acc[i]) * rms;
     if (lane == 0) epilogue<EPI, RPW>(a, vr0, acc, res, pos);
   }
+}
+
+// Several columns of x (2 .. NC) against the same float rows: chatnet_matmul
+// with a few columns ran gemv_f_kernel once per column, each launch reading W
+// again (F16 4096 x 4096: 5.9 us a column).  Here ncols columns are staged in
+// LDS as fp32 ([ncols][K]) and every 16-byte piece of W, loaded once, meets
+// all of them.  Lane l takes pieces l, l + 64, ... of a row in order and the
+// row sums meet in cn_wave_sum, as in gemv_f_kernel, so a column's result is
+// the single-column launch's bit for bit.  Bound by the LDS reads of x (32
+// bytes per piece, row group and column), which RPW = 4 rows share: 512
+// threads, one or two workgroups per CU by LDS.
+template <int WT, int NC, int RPW>
+__global__ __launch_bounds__(512) void gemv_fcols_kernel(GemvArgs a, int ncols) {
+  constexpr int BS = 512, NWV = BS / CN_WAVE, U = 8 / RPW;
+  constexpr int PE = piece_elems<WT>();
+  extern __shared__ float smem[];
+  const int K = a.K, M = a.n_vrows;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const size_t row_bytes = (size_t)K * (WT == WT_F32 ? 4 : 2);
+  const int npieces = K / PE;
+  const int n_iters = (M + RPW - 1) / RPW;
+  int it = blockIdx.x * NWV + wave;
+  // U steps of pieces of a row group; rows past the end re-read the last row,
+  // pieces past its end the last piece (neither is used)
+  cn_u32x4 w[U][RPW];
+  auto load = [&](int itn, int p0) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int p = min(p0 + CN_WAVE * u + lane, npieces - 1);
+#pragma unroll
+      for (int i = 0; i < RPW; i++)
+        w[u][i] = *(const CN_GLOBAL cn_u32x4*)((const cn_gbyte*)a.w[0] +
+                                               (size_t)min(itn * RPW + i, M - 1) * row_bytes + (size_t)p * 16);
+    }
+  };
+  load(it, 0);  // the first weights travel while x is staged
+  for (int c = threadIdx.x; c < ncols * (K >> 2); c += BS)
+    reinterpret_cast<float4*>(smem)[c] = reinterpret_cast<const float4*>(a.x)[c];
+  __syncthreads();
+  while (it < n_iters) {
+    const int r0 = it * RPW;
+    it += gridDim.x * NWV;
+    float acc[NC][RPW];
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+#pragma unroll
+      for (int i = 0; i < RPW; i++) acc[c][i] = 0.f;
+    for (int p0 = 0; p0 < npieces; p0 += CN_WAVE * U) {
+      cn_u32x4 cur[U][RPW];
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int i = 0; i < RPW; i++) cur[u][i] = w[u][i];
+      if (p0 + CN_WAVE * U < npieces) load(r0 / RPW, p0 + CN_WAVE * U);
+      else if (it < n_iters) load(it, 0);
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int p = p0 + CN_WAVE * u + lane;
+        if (p < npieces) {
+#pragma unroll
+          for (int c = 0; c < NC; c++)
+            if (c < ncols) {
+#pragma unroll
+              for (int i = 0; i < RPW; i++)
+                acc[c][i] += piece_dot<WT>(cur[u][i], smem + (size_t)c * K + (size_t)p * PE);
+            }
+        }
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+      if (c < ncols) {
+#pragma unroll
+        for (int i = 0; i < RPW; i++) {
+          const float v = cn_wave_sum(acc[c][i]);
+          if (lane == 0 && r0 + i < M) a.out[0][(size_t)c * M + r0 + i] = v;
+        }
+      }
+  }
+}
+
+template <int WT, int NC, int RPW>
+hipError_t launch_fcols_rows(const GemvArgs& a, int ncols, int num_cus, hipStream_t st) {
+  const size_t smem = sizeof(float) * (size_t)ncols * a.K;
+  const auto kern = &gemv_fcols_kernel<WT, NC, RPW>;
+  if (smem > 65536) {  // more than 64 KB of dynamic LDS must be allowed (once per device)
+    static std::atomic<uint64_t> lds_done{0};
+    const hipError_t e = allow_full_lds(reinterpret_cast<const void*>(kern), lds_done);
+    if (e != hipSuccess) return e;
+  }
+  const int n_iters = (a.n_vrows + RPW - 1) / RPW;
+  int grid = (n_iters + 7) / 8;
+  const int per_cu = smem * 2 > (size_t)kCuLdsBytes ? 1 : 2;
+  if (grid > per_cu * num_cus) grid = per_cu * num_cus;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(512), smem, st, a, ncols);
+  return hipGetLastError();
+}
+
+// Four rows per wave while that still gives every CU a workgroup, else one.
+template <int WT, int NC>
+hipError_t launch_fcols(const GemvArgs& a, int ncols, int num_cus, hipStream_t st) {
+  if (a.n_vrows >= 32 * num_cus) return launch_fcols_rows<WT, NC, 4>(a, ncols, num_cus, st);
+  if (a.n_vrows >= 16 * num_cus) return launch_fcols_rows<WT, NC, 2>(a, ncols, num_cus, st);
+  return launch_fcols_rows<WT, NC, 1>(a, ncols, num_cus, st);
 }
 
 size_t gemv_f_smem(int K) { return sizeof(float) * ((size_t)K + 16); }
@@ -335,4 +441,34 @@ hipError_t gemv_float_launch(int qtype, int epi, const GemvArgs& a, int num_cus,
       return launch_f_epi<GEMV_EPI_ADD_MERGE>(qtype, a, num_cus, st);
     default: return hipErrorInvalidValue;
   }
+}
+
+// Columns per launch: 8, or as many as leave their fp32 x in 152 KB of LDS (2 at K = 16384).
+int gemv_float_cols_max(int K) {
+  const int fit = (int)((152 * 1024) / (sizeof(float) * (size_t)K));
+  return fit < 8 ? fit : 8;
+}
+
+hipError_t gemv_float_cols_launch(int qtype, const void* w, const float* x, float* y, int M, int K, int N, int num_cus,
+                                  hipStream_t st) {
+  if ((qtype != 0 && qtype != 1) || K <= 0 || K % 64 != 0 || K > 16384 || M <= 0 || N < 1 || !w || !x || !y)
+    return hipErrorInvalidValue;
+  const int g = gemv_float_cols_max(K);
+  for (int c0 = 0; c0 < N; c0 += g) {
+    const int nc = N - c0 < g ? N - c0 : g;
+    GemvArgs a;
+    memset(&a, 0, sizeof(a));
+    a.w[0] = a.w[1] = a.w[2] = static_cast<const uint8_t*>(w);
+    a.seg_rows[0] = M;
+    a.n_vrows = M;
+    a.K = K;
+    a.x = x + (size_t)c0 * K;
+    a.out[0] = y + (size_t)c0 * M;
+    hipError_t e;
+    if (nc <= 2) e = qtype == 0 ? launch_fcols<WT_F32, 2>(a, nc, num_cus, st) : launch_fcols<WT_F16, 2>(a, nc, num_cus, st);
+    else if (nc <= 4) e = qtype == 0 ? launch_fcols<WT_F32, 4>(a, nc, num_cus, st) : launch_fcols<WT_F16, 4>(a, nc, num_cus, st);
+    else e = qtype == 0 ? launch_fcols<WT_F32, 8>(a, nc, num_cus, st) : launch_fcols<WT_F16, 8>(a, nc, num_cus, st);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }

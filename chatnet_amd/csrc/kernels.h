@@ -81,6 +81,12 @@ bool gemv_needs_pack(int qtype);
 int gemv_cols_max(int K);
 hipError_t gemv_cols_launch(const void* w, const float* x, float* y, int M, int K, int N, int num_cus,
                             hipStream_t st);
+// F32 (0) / F16 (1) rows against N columns of x, gemv_float_cols_max(K) (2 to 8)
+// per launch: column c = the single-column GEMV of x[c] bit for bit.  K % 64 ==
+// 0, K <= 16384.
+int gemv_float_cols_max(int K);
+hipError_t gemv_float_cols_launch(int qtype, const void* w, const float* x, float* y, int M, int K, int N, int num_cus,
+                                  hipStream_t st);
 size_t gemv_lds_bytes(int qtype, int K);
 hipError_t gemv_launch(int qtype, int epi, const GemvArgs& a, int num_cus, hipStream_t st);
 hipError_t gemv_float_launch(int qtype, int epi, const GemvArgs& a, int num_cus, hipStream_t st);
@@ -107,6 +113,7 @@ struct GemmArgs {
   const uint16_t* xb_lo;  // precise: fp16 low parts, x = xb + xb_lo
   const float* xinv;      // one-plane kernel: per-column 2^-e undoing the scale of xb (nullptr: 1)
   int precise;            // exact-weight two-plane kernel
+  const float* x32;       // F16 rows from chatnet_matmul: the fp32 x, read to redo an output that came out NaN
   int epi;
   float* y;               // STORE / ADD target
   int ldy;
@@ -145,6 +152,10 @@ hipError_t gemm_launch(const GemmArgs& a, int num_cus, hipStream_t st, int* spli
 // the cn_span_pos order, 2^e_n bringing max|x[n]| into [2^14, 2^15), and
 // xinv[n] = 2^-e_n.  K % 32 == 0, K <= 16384.
 hipError_t to_f16_scaled_launch(const float* x, uint16_t* xh, float* xinv, int N, int K, hipStream_t st);
+// x [N][K] fp32 -> the span kernel's input scaled per column as above: hi + lo
+// fp16 planes of x[n] * 2^e_n (max over the finite |x[n]|), about 2^-24 of each
+// element, and xinv[n] = 2^-e_n.  Infinities stay infinite with lo = 0.
+hipError_t to_f16_planes_launch(const float* x, uint16_t* xh, uint16_t* xl, float* xinv, int N, int K, hipStream_t st);
 // x[r] += the K-split partials part[0..splits)[r] (summed as the GEMM's reduce
 // does), then xb / xb_lo = RMSNorm(x[r]) * g as the span GEMM's input (fp16 hi
 // + lo planes in the cn_span_pos order); splits 0: the norm alone.  dim % 32

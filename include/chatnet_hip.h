@@ -250,8 +250,13 @@ CHATNET_API int chatnet_get_logits(chatnet_model* m, float* logits_host);
  * inside fp16's range, each weight rounded once to fp16; Q4_0 read as raw
  * blocks, the other types first re-encoded
  * into the workspace as u8 codes with an fp32 scale and offset per 16 weights,
- * M*(K/64)*96 bytes, giving the same dequantized values); any other call
- * (N < 8, F32, F16) runs the fused GEMV once per column, which reads Q4_1,
+ * M*(K/64)*96 bytes, giving the same dequantized values).  F32 and F16 rows
+ * with several columns run a multi-column GEMV (each column the N = 1
+ * product's exact arithmetic), F16 with more columns than one launch of it
+ * holds (8 up to K = 4864, fewer above) an MFMA product of the exact weights
+ * with x as two fp16 planes, summed with compensation in fp32 (its error
+ * against float64 is the GEMV's, 1e-7).  Any other call (block types at N < 8)
+ * runs the fused GEMV once per column, which reads Q4_1,
  * Q5_0, Q5_1, Q2_K, Q8_K and the IQ types from that same re-encoded
  * copy, made in the workspace first.  A GEMM whose grid of 128 x 128 tiles
  * is just over one tile per CU (e.g. 11008 x 4096 at N = 512) runs as a
@@ -265,7 +270,8 @@ CHATNET_API int chatnet_get_logits(chatnet_model* m, float* logits_host);
  * CHATNET_ERR_INVALID_ARG if the stream's workspace is too small, so a
  * capturing caller first makes one uncaptured call of the largest size, or
  * uses chatnet_matmul_noalloc.  `stream` is a hipStream_t (NULL = default
- * stream).  Asynchronous on `stream`. */
+ * stream).  F16 rows need no workspace there: their
+ * calls then run the multi-column GEMV.  Asynchronous on `stream`. */
 CHATNET_API int chatnet_matmul(uint32_t ggml_type, const void* w_dev, const float* x_dev,
                    float* y_dev, int M, int K, int N, void* stream);
 
@@ -278,7 +284,7 @@ CHATNET_API int chatnet_matmul(uint32_t ggml_type, const void* w_dev, const floa
  * that it runs no stream-K launch: where chatnet_matmul shares tiles it runs
  * the plain tile grid, the same product summed in another order.  Q8_0,
  * Q3_K, Q4_K, Q5_K and Q6_K run the fused GEMV once per column on their stored
- * blocks.  The scratch (fp16 x, its per-column scales, the K-split partials
+ * blocks, F32 and F16 the multi-column GEMV, without scratch.  The scratch (fp16 x, its per-column scales, the K-split partials
  * and the packed W) lives
  * in a fixed 64 MiB array per device, held by the library from load to
  * process exit, instead of a per-stream workspace.  Calls needing more

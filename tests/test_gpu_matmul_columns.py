@@ -1,0 +1,95 @@
+"""chatnet_matmul with several columns against float64 products of the oracle's
+dequantized weights, at the edges of each path: a few columns in one launch
+(multi-column GEMV), the matrix-core paths from 8 columns on, non-finite
+values, a capturing stream and the no-allocation variant."""
+import numpy as np
+import pytest
+
+from chatnet_amd import _native, hiprt, ops, synth
+from gpu_util import announce, gpu_matmul, normwise
+
+pytestmark = pytest.mark.gpu
+
+F32, F16 = 0, 1
+
+
+def float_weights(qtype, M, K, seed):
+    w = synth.normal(seed, f"fc{M}x{K}", M * K, 0.05).reshape(M, K)
+    return w.astype(np.float16) if qtype == F16 else w
+
+
+# Groups of columns whose fp32 x fits in LDS: 8 up to K = 4864, 3 at 11008, 2 at
+# 16384; tiles of 32 and 64 columns and ragged rows for the F16 product.
+@pytest.mark.parametrize("M,K,N", [
+    (1, 64, 2), (3, 192, 7), (130, 4096, 5), (37, 11008, 7), (65, 16384, 3), (5, 64, 8), (129, 4096, 33), (200, 320, 64),
+    (4096, 4096, 24), (66, 16384, 12), (1000, 2048, 300),
+])
+@pytest.mark.parametrize("qtype", [F32, F16])
+def test_float_columns_match_float64(qtype, M, K, N):
+    """Bar: 32-bit sums in any order, |error| <= K * 2^-24 of sum |w x| at worst
+    (the F16 product's x carries 2^-24 of each element besides); measured about
+    1e-7 of the largest output."""
+    announce(f"float columns type={qtype} M={M} K={K} N={N}")
+    w = float_weights(qtype, M, K, 5)
+    x = synth.normal(6, f"fcx{N}x{K}", N * K, 1.0).reshape(N, K)
+    x[:, 0] *= 300.0
+    y = gpu_matmul(qtype, w.view(np.uint8).ravel(), x, M, K)
+    r = x.astype(np.float64) @ w.astype(np.float64).T
+    scale = np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T
+    assert np.all(np.abs(y - r) <= 2e-6 * scale), float(np.max(np.abs(y - r) / scale))
+    if qtype == F32 or N * K * 4 <= 152 * 1024 and N <= 8:  # one GEMV launch: each column the single-column result
+        for n in range(N):
+            assert np.array_equal(y[n], gpu_matmul(qtype, w.view(np.uint8).ravel(), x[n], M, K)[0])
+
+
+def test_f16_columns_of_other_magnitudes_and_non_finite_values():
+    """Columns far outside fp16's range keep their accuracy; infinities and NaN in
+    x or W give what the single-column product gives."""
+    M, K, N = 70, 256, 12
+    w = float_weights(F16, M, K, 7)
+    w[3, 5], w[4, 6], w[5, 7] = np.inf, -np.inf, np.nan
+    x = synth.normal(8, "fcx-mag", N * K, 1.0).reshape(N, K).astype(np.float64)
+    x *= np.array([1e-30, 1e-12, 3e-5, 1e-3, 0.5, 1.0, 7.0, 6e4, 1e8, 1e20, 1e30, 0.0])[:, None]
+    x = x.astype(np.float32)
+    x[5, 9], x[6, 10], x[7, 11] = np.inf, -np.inf, np.nan
+    x[4, 5] = 0.25  # an exact fp16 value against the infinite weight: its low part is zero
+    announce("f16 columns, magnitudes and non-finite values")
+    y = gpu_matmul(F16, w.view(np.uint8).ravel(), x, M, K)
+    for n in range(N):
+        one = gpu_matmul(F16, w.view(np.uint8).ravel(), x[n], M, K)[0]
+        fin = np.isfinite(one)
+        assert np.array_equal(fin, np.isfinite(y[n])), n
+        assert np.array_equal(np.isnan(one), np.isnan(y[n])), n
+        assert np.array_equal(one[~fin & ~np.isnan(one)], y[n][~fin & ~np.isnan(one)]), n
+        if fin.any():
+            assert normwise(y[n][fin], one[fin]) <= 2e-6, n
+
+
+@pytest.mark.parametrize("M,K,N", [(96, 512, 16), (96, 512, 3)])
+def test_f16_columns_captured_without_a_workspace_and_noalloc(M, K, N):
+    """F16 rows take no workspace they cannot have: captured on a fresh stream
+    (no earlier call grew one) and in the no-allocation variant they run the
+    multi-column GEMV, each column the single-column result."""
+    announce(f"f16 captured M={M} K={K} N={N}")
+    w = float_weights(F16, M, K, 9)
+    x = synth.normal(9, "fcx-cap", N * K, 1.0).reshape(N, K)
+    ref = np.stack([gpu_matmul(F16, w.view(np.uint8).ravel(), x[n], M, K)[0] for n in range(N)])
+    w_d = hiprt.DeviceBuffer.from_numpy(w.view(np.uint8).ravel(), pad=256)
+    x_d, y_d = hiprt.DeviceBuffer.from_numpy(x), hiprt.DeviceBuffer(4 * N * M)
+    stream = hiprt.Stream()
+    graph = hiprt.Graph(stream, lambda: ops.matmul_ptr(F16, w_d.ptr, x_d.ptr, y_d.ptr, M, K, N, stream.h))
+    for _ in range(2):
+        y_d.fill(0xFF)
+        hiprt.synchronize()
+        graph.launch()
+        stream.synchronize()
+        assert np.array_equal(y_d.to_numpy(np.float32, N * M).reshape(N, M), ref)
+    y_d.fill(0xFF)
+    hiprt.synchronize()
+    lib = _native.hip_lib()
+    _native.check(lib.chatnet_matmul_noalloc(F16, w_d.ptr, x_d.ptr, y_d.ptr, M, K, N, stream.h))
+    stream.synchronize()
+    assert np.array_equal(y_d.to_numpy(np.float32, N * M).reshape(N, M), ref)
+    del graph
+    for b in (w_d, x_d, y_d):
+        b.free()
