@@ -17,8 +17,10 @@ CSRC = os.path.join(PKG, "csrc")
 LIBDIR = os.path.join(PKG, "lib")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
-HIP_SOURCES = ["chatnet_api.hip", "gemv.hip", "gemv_float.hip", "gemm.hip", "prefill.hip", "decode_ops.hip", "sample.hip"]
-HIP_HEADERS = ["device_common.h", "gemv_common.h", "kernels.h"]
+HIP_SOURCES = ["gemv_q4_0.hip", "gemm.hip", "gemv_q8_0.hip", "gemv_q6_k.hip", "gemv_q5_k.hip", "gemv_q4_k.hip", "gemv_q3_k.hip",
+               "gemv_q5_0.hip", "gemv_q5_1.hip", "gemv_q4_1.hip", "gemv_iq4_nl.hip", "gemv_iq4_xs.hip", "gemv_q2_k.hip",
+               "chatnet_api.hip", "gemv.hip", "gemv_float.hip", "prefill.hip", "decode_ops.hip", "sample.hip"]
+HIP_HEADERS = ["device_common.h", "gemv_common.h", "gemv_mcol.h", "gemv_quant.h", "kernels.h"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

@@ -80,14 +80,17 @@ int device_cus(int dev) {
 }
 
 // Weight types the GEMV serves (LlamaModel.MatVecMulByType, LlamaModel.cs:470-567):
-// F32, F16, Q4_0, Q8_0, Q3_K, Q4_K, Q5_K, Q6_K from the stored blocks, and
-// Q4_1, Q5_0, Q5_1, Q2_K, Q8_K and the nine IQ types (the reference's
-// MatVecMulGeneric branches, LlamaModel.cs:488-562) from packed units made at
-// upload.
-bool is_matrix_type(uint32_t t) {
-  return t == CHATNET_GGML_F32 || t == CHATNET_GGML_F16 || t == CHATNET_GGML_Q4_0 || t == CHATNET_GGML_Q8_0 ||
-         t == CHATNET_GGML_Q3_K || t == CHATNET_GGML_Q4_K || t == CHATNET_GGML_Q5_K || t == CHATNET_GGML_Q6_K ||
-         gemv_needs_pack((int)t);
+// F32, F16, Q4_0, Q4_1, Q5_0, Q5_1, Q8_0, Q2_K .. Q6_K, IQ4_NL and IQ4_XS from
+// the stored blocks, Q8_K and the other IQ types (reference branches
+// LlamaModel.cs:488-562) from packed units made at upload.
+bool is_matrix_type(uint32_t t) { return gemv_supports((int)t, 256); }
+
+// The types that spans and wide products read as packed units made ahead
+// (a model's at upload) and that chatnet_matmul_noalloc takes only while
+// their packed copy fits its scratch.
+bool packed_ahead(uint32_t t) {
+  return gemv_needs_pack((int)t) || t == CHATNET_GGML_Q4_1 || t == CHATNET_GGML_Q5_0 || t == CHATNET_GGML_Q5_1 ||
+         t == CHATNET_GGML_Q2_K || t == CHATNET_GGML_IQ4_NL || t == CHATNET_GGML_IQ4_XS;
 }
 
 // Embedding rows read in their stored form; every other block type is
@@ -115,6 +118,9 @@ const void* embed_w(const DevTensor& t) { return embed_raw_type(t.type) ? t.ptr 
 std::mutex g_ws_mu;
 std::map<std::pair<int, hipStream_t>, std::pair<char*, size_t>> g_ws;
 std::vector<char*> g_ws_retired;
+// Held while a call enqueues the launches that share its stream's workspace, so
+// that calls from several threads on one stream do not interleave them.
+std::mutex g_enqueue_mu;
 
 // The first kMatmulCounterBytes of a stream's workspace are the one-plane
 // GEMM's stream-K tile counters: zeroed when the workspace is allocated, and
@@ -570,13 +576,15 @@ int chatnet_upload_tensor(chatnet_model* m, const char* name, uint32_t type, con
     return fail(CHATNET_ERR_OUT_OF_MEMORY, "hipMalloc of %llu bytes for %s failed", (unsigned long long)nbytes, name);
   const bool neox_rows = c.arch == CHATNET_ARCH_QWEN2 && layer >= 0 &&
                          (slot == &m->layers[layer].wq || slot == &m->layers[layer].wk);
-  // Types the GEMV (or the embedding gather) reads only as packed units are
+  // Types that spans (or the embedding gather) read as packed units are
   // packed below, one pass over the uploaded rows; the stored blocks stay for
-  // the other readers.  Their stored rows keep the file's order even where the
-  // Qwen2 row order applies (an IQ3_S row reads into the row after it in the
-  // file, DequantIQ.cs:255-283): the packed rows are put in that order instead.
-  const bool pack_now = (matrix && gemv_needs_pack((int)type)) || (slot == &m->emb && !embed_raw_type(type));
-  if (neox_rows && !pack_now) {
+  // the other readers.  The types the GEMV reads only packed keep the file's
+  // row order even where the Qwen2 row order applies (an IQ3_S row reads into
+  // the row after it in the file, DequantIQ.cs:255-283): their packed rows are
+  // put in that order instead.
+  const bool pack_now = (matrix && packed_ahead(type)) || (slot == &m->emb && !embed_raw_type(type));
+  const bool file_rows = gemv_needs_pack((int)type);
+  if (neox_rows && !file_rows) {
     const size_t bpr = (size_t)(nbytes / ne1);
     std::vector<uint8_t> rows(nbytes);
     for (uint64_t r = 0; r < ne1; r++)
@@ -596,7 +604,7 @@ int chatnet_upload_tensor(chatnet_model* m, const char* name, uint32_t type, con
       slot->pk = nullptr;
       return fail(CHATNET_ERR_OUT_OF_MEMORY, "hipMalloc of %zu bytes (packed %s) failed", pk_bytes, name);
     }
-    if (neox_rows) {
+    if (neox_rows && file_rows) {
       void* tmp = nullptr;
       if (hipMalloc(&tmp, pk_bytes) != hipSuccess)
         return fail(CHATNET_ERR_OUT_OF_MEMORY, "hipMalloc of %zu bytes (packed %s) failed", pk_bytes, name);
@@ -1125,6 +1133,7 @@ int run_prompt(chatnet_model* m, const int32_t* tokens, int n, int position) {
 int matmul_float(int type, const void* w, const float* x, float* y, int M, int K, int N, int dev, int cus,
                  hipStream_t st, bool noalloc) {
   if (type == CHATNET_GGML_F16 && N >= 4 && N > gemv_float_cols_max(K) && !noalloc) {
+    std::lock_guard<std::mutex> lk(g_enqueue_mu);
     const size_t plane = ((size_t)N * K * sizeof(uint16_t) + 255) & ~(size_t)255;
     const size_t scales = ((size_t)N * sizeof(float) + 255) & ~(size_t)255;
     const size_t part = gemm_workspace_bytes(M, N, K, cus, true, GEMM_W_F16);
@@ -1182,10 +1191,6 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
   HIP_TRY(hipGetDevice(&dev));
   const int cus = device_cus(dev);
   hipStream_t st = (hipStream_t)stream;
-  // Q4_0 reads its raw blocks; the other block types (not in the no-allocation
-  // variant) are packed into the workspace first, one pass over W.  The types
-  // the GEMV reads only as packed units are packed for every N, in both
-  // variants.
   // Q4_0 with a few columns: the GEMV over all of them at once, one pass over W.
   // Its digit dots cost ALU and LDS time per column, so from 8 columns on it
   // is taken only up to the size where it measured faster than the MFMA GEMM
@@ -1199,12 +1204,28 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
   }
   if ((type == CHATNET_GGML_F32 || type == CHATNET_GGML_F16) && N >= 2)
     return matmul_float((int)type, w_dev, x_dev, y_dev, M, K, N, dev, cus, st, noalloc);
+  // The other block types up to kColsGemv columns: all columns at once on the
+  // stored blocks (gemv_qcols_launch), more precise and faster than the MFMA
+  // GEMM behind its packing pass (Q4_K 4096 x 4096 at 16 columns 14.7 against
+  // 38.4 us, 11008 x 4096 26.3 against 68.0, Q3_K 2048 x 11008 45.4 against
+  // 61.2).  Two columns (Q3_K, whose unpacking costs the most: three) of a
+  // matrix of at least kTwoGemvs weights run the single-column GEMV for each
+  // (11008 x 4096: Q4_K at 2 columns 13.1 against 16.6 us, Q3_K at 3 24.7
+  // against 29.0).  More columns run the GEMM: Q4_0 reads its
+  // raw blocks, the other types are packed into the workspace first, one pass
+  // over W (in the no-allocation variant only the packed_ahead types).  The
+  // types the GEMV reads only as packed units are packed for every N.
+  constexpr int kColsGemv = 16;
+  constexpr long long kTwoGemvs = 32LL << 20;
   const bool raw = gemm_supports((int)type, K);
   const bool must_pack = gemv_needs_pack((int)type);
-  const bool batched = N >= 8 && (raw || must_pack || (!noalloc && gemm_pack_supports((int)type, K)));
+  const bool ahead = packed_ahead(type);
+  const bool batched = N >= 8 && !(N <= kColsGemv && gemv_qcols_supports((int)type)) &&
+                       (raw || ahead || (!noalloc && gemm_pack_supports((int)type, K)));
   const bool pack = must_pack || (batched && !raw);
   const uint8_t* wp = (const uint8_t*)w_dev;
-  if (batched || pack) {
+  std::unique_lock<std::mutex> lk(g_enqueue_mu, std::defer_lock);
+  if (batched || pack || (noalloc && ahead)) {
     // [stream-K tile counters | fp16 x | per-column x scales | K-split or
     // stream-K partials | packed W]: the counters in the per-stream workspace
     // only (the no-allocation variant runs no stream-K launch), the next
@@ -1214,10 +1235,11 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
     const size_t xb_bytes = batched ? xh_bytes + (((size_t)N * sizeof(float) + 255) & ~(size_t)255) : cnt_bytes;
     const size_t part_bytes =
         batched ? (gemm_workspace_bytes(M, N, K, cus, false, pack, !noalloc) + 255) & ~(size_t)255 : 0;
-    const size_t pack_bytes = pack ? gemm_pack_bytes(M, K) : 0;
+    const size_t pack_bytes = pack || (noalloc && ahead) ? gemm_pack_bytes(M, K) : 0;
     const size_t need = xb_bytes + part_bytes + pack_bytes;
     char* ws = nullptr;
     int rc;
+    if (batched || pack) lk.lock();
     if (noalloc) {
       if (need > kNoAllocScratchBytes)
         return fail(CHATNET_ERR_INVALID_ARG,
@@ -1256,6 +1278,21 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
       g_err.clear();
       return CHATNET_OK;
     }
+  }
+  if (N >= 2 && !pack && gemv_qcols_supports((int)type) && !(N <= (type == CHATNET_GGML_Q3_K ? 3 : 2) && (long long)M * K >= kTwoGemvs)) {
+    // x staged once in the stream's workspace where there is one and it pays
+    const size_t need = noalloc ? 0 : gemv_qcols_workspace(M, K, N, cus);
+    char* ws = nullptr;
+    if (need) {
+      lk.lock();
+      bool ok = true;
+      const int rc = matmul_workspace(dev, st, kMatmulCounterBytes + need, &ws, &ok);
+      if (rc) return rc;
+      ws = ok ? ws + kMatmulCounterBytes : nullptr;
+    }
+    HIP_TRY(gemv_qcols_launch((int)type, w_dev, x_dev, y_dev, M, K, N, cus, ws, st));
+    g_err.clear();
+    return CHATNET_OK;
   }
   const int qt = pack ? kGemvPacked : (int)type;
   for (int n = 0; n < N; n++) {  // one fused GEMV per column

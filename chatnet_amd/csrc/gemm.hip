@@ -78,16 +78,22 @@ __device__ __forceinline__ void write_h(const GemmArgs& a, int n, int j, float v
   a.hb_lo[i] = (uint16_t)lo;
 }
 
-// An output of chatnet_matmul's F16 rows that came out NaN, summed again from
-// the fp32 x: in two planes an infinite weight meets x's low part too (inf * 0
-// or inf - inf), where the plain product is infinite.  Never taken for finite
-// operands.
-__device__ __attribute__((noinline)) float f16_dot_again(const GemmArgs& a, int n, int m) {
-  const _Float16* w = reinterpret_cast<const _Float16*>(a.w[0]) + (size_t)m * a.K;
-  const float* x = a.x32 + (size_t)n * a.K;
-  float s = 0.f;
-  for (int k = 0; k < a.K; k++) s = fmaf((float)w[k], x[k], s);
-  return s;
+// Outputs of chatnet_matmul's F16 rows (rows m..m+3 of column n) that came out
+// NaN, summed again from the fp32 x: in two planes an infinite weight meets x's
+// low part too (inf * 0 or inf - inf), where the plain product is infinite.
+// Never taken for finite operands.  Only the compensated instances call it (a
+// loop in every instance's epilogue cost the others registers).
+__device__ __forceinline__ void f16_dot_again(const GemmArgs& a, int n, int m, f32x4& v) {
+  const float t = (v[0] + v[1]) + (v[2] + v[3]);
+  if (t == t || n >= a.N) return;
+  for (int i = 0; i < 4 && m + i < a.M; i++) {
+    if (v[i] == v[i]) continue;
+    const _Float16* w = reinterpret_cast<const _Float16*>(a.w[0]) + (size_t)(m + i) * a.K;
+    const float* x = a.x32 + (size_t)n * a.K;
+    float s = 0.f;
+    for (int k = 0; k < a.K; k++) s = fmaf((float)w[k], x[k], s);
+    v[i] = s;
+  }
 }
 
 // Final write of 4 consecutive rows m..m+3 of column n.
@@ -108,13 +114,6 @@ __device__ __forceinline__ void write_out4(const GemmArgs& a, int epi, int n, in
       write_h(a, n, m >> 1, silu_mul(v[0], v[1]));
     }
     return;
-  }
-  if (a.x32) {
-    const float t = (v[0] + v[1]) + (v[2] + v[3]);
-    if (!(t == t)) {
-      for (int i = 0; i < 4 && m + i < a.M; i++)
-        if (!(v[i] == v[i])) v[i] = f16_dot_again(a, n, m + i);
-    }
   }
   float* y = a.y + (size_t)n * a.ldy + m;
   if (full) {
@@ -512,7 +511,7 @@ struct TileIO {
   }
 
   // Final tiles: K-split partials [splits][N][M] or the epilogue.
-  template <int TN>
+  template <int TN, bool COMP = false>
   __device__ __forceinline__ void store(const GemmArgs& a, const f32x16 (&acc)[TN], const float (&scl)[TN],
                                         int mt = 0) const {
 #pragma unroll
@@ -522,7 +521,7 @@ struct TileIO {
 #pragma unroll
       for (int v4 = 0; v4 < 4; v4++) {
         const int m = m0 + wm * 32 * C::MTILES + 32 * mt + 8 * v4 + 4 * h;
-        const f32x4 v = f32x4{acc[cc][4 * v4], acc[cc][4 * v4 + 1], acc[cc][4 * v4 + 2], acc[cc][4 * v4 + 3]} * sc;
+        f32x4 v = f32x4{acc[cc][4 * v4], acc[cc][4 * v4 + 1], acc[cc][4 * v4 + 2], acc[cc][4 * v4 + 3]} * sc;
         if (a.splits > 1) {
           if (n < a.N && m < a.M) {
             float* p = a.part + ((size_t)ks * a.N + n) * a.M + m;
@@ -531,6 +530,7 @@ struct TileIO {
               for (int i = 0; i < 4 && m + i < a.M; i++) p[i] = v[i];
           }
         } else {
+          if constexpr (COMP) f16_dot_again(a, n, m, v);
           write_out4(a, a.epi, n, m, v);
         }
       }
@@ -929,12 +929,14 @@ __global__ __launch_bounds__(CN_BLOCK) void gemm_s_kernel(GemmArgs a) {
   }
   float sc[TN];
   io.template load_scales<TN>(a, sc);
-  if constexpr (COMP) io.template store<TN>(a, sum, sc);
+  if constexpr (COMP) io.template store<TN, true>(a, sum, sc);
   else io.template store<TN>(a, acc, sc);
 }
 
 // Sums the K-split partials [splits][N][M] and applies the epilogue; one
 // thread per 4 consecutive rows of one column.
+// COMP: the F16 product of chatnet_matmul (compensated, see gemm_s_kernel).
+template <bool COMP>
 __global__ __launch_bounds__(CN_BLOCK) void gemm_reduce_kernel(GemmArgs a) {
   const int m4 = (a.M + 3) / 4;
   const long long t = (long long)blockIdx.x * CN_BLOCK + threadIdx.x;
@@ -949,9 +951,10 @@ __global__ __launch_bounds__(CN_BLOCK) void gemm_reduce_kernel(GemmArgs a) {
     } else {
       for (int i = 0; i < 4 && m + i < a.M; i++) v[i] = p[i];
     }
-    if (a.x32) add_compensated(s, c, v);
+    if constexpr (COMP) add_compensated(s, c, v);
     else s += v;
   }
+  if constexpr (COMP) f16_dot_again(a, n, m, s);
   write_out4(a, a.epi, n, m, s);
 }
 
@@ -1670,7 +1673,9 @@ hipError_t gemm_launch(const GemmArgs& a_in, int num_cus, hipStream_t st, int* s
     return hipSuccess;
   }
   const long long work = (long long)((a.M + 3) / 4) * a.N;
-  hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((work + CN_BLOCK - 1) / CN_BLOCK)), dim3(CN_BLOCK), 0, st, a);
+  const dim3 rgrid((unsigned)((work + CN_BLOCK - 1) / CN_BLOCK));
+  if (a.x32) hipLaunchKernelGGL((gemm_reduce_kernel<true>), rgrid, dim3(CN_BLOCK), 0, st, a);
+  else hipLaunchKernelGGL((gemm_reduce_kernel<false>), rgrid, dim3(CN_BLOCK), 0, st, a);
   return hipGetLastError();
 }
 

@@ -1,0 +1,11 @@
+// gemv_q4_k.hip — the Q4_K instances of the quantized GEMV (gemv_quant.h) and of
+// the few-column product (gemv_mcol.h).
+#include "gemv_mcol.h"
+
+hipError_t gemv_q4_k_launch(int epi, const GemvArgs& a, int num_cus, hipStream_t st) {
+  return launch_type<QT_Q4_K>(epi, a, num_cus, st);
+}
+
+hipError_t gemv_q4_k_cols_launch(const GemvArgs& a, int ncols, int num_cus, char* pre, hipStream_t st) {
+  return launch_mcol<QT_Q4_K>(a, ncols, num_cus, pre, st);
+}

@@ -66,11 +66,11 @@ struct GemvArgs {
   const int* stop;
 };
 
-// Weight types: Q4_0, Q8_0 (K % 64 == 0), Q4_K, Q5_K, Q6_K (K % 256 == 0), and
-// F32 / F16 (K % 64 == 0, gemv_float.hip); K <= 16384.  gemv_float_launch
-// also takes kGemvPacked: w[] holding packed units (gemm_pack_launch), how the
-// model runs Q4_1, Q5_0, Q5_1, IQ4_NL (K % 64 == 0), Q2_K, Q8_K and the other
-// IQ types (K % 256 == 0).
+// Weight types: Q4_0, Q4_1, Q5_0, Q5_1, Q8_0, IQ4_NL (K % 64 == 0), Q2_K, Q3_K,
+// Q4_K, Q5_K, Q6_K, IQ4_XS (K % 256 == 0), and F32 / F16 (K % 64 == 0,
+// gemv_float.hip); K <= 16384.  gemv_float_launch also takes kGemvPacked: w[]
+// holding packed units (gemm_pack_launch), how the model runs Q8_K and the
+// other IQ types (K % 256 == 0).
 constexpr int kGemvPacked = -1;
 bool gemv_supports(int qtype, int K);
 // True for the types gemv_supports accepts only as packed units.
@@ -87,7 +87,25 @@ hipError_t gemv_cols_launch(const void* w, const float* x, float* y, int M, int 
 int gemv_float_cols_max(int K);
 hipError_t gemv_float_cols_launch(int qtype, const void* w, const float* x, float* y, int M, int K, int N, int num_cus,
                                   hipStream_t st);
-size_t gemv_lds_bytes(int qtype, int K);
+// Block types other than Q4_0 read from their stored blocks against N columns of
+// x on the int8 matrix cores (gemv_mcol.h), up to 16 per launch, x to 23 bits of
+// each 32-element block's largest.
+bool gemv_qcols_supports(int qtype);
+// Workspace for x staged once ahead of the product (0: not worth the launch,
+// every workgroup stages it); gemv_qcols_launch takes it or null.
+size_t gemv_qcols_workspace(int M, int K, int N, int num_cus);
+hipError_t gemv_qcols_launch(int qtype, const void* w, const float* x, float* y, int M, int K, int N, int num_cus,
+                             void* ws, hipStream_t st);
+// The merge epilogue's instance for a launch of `splits` chunks (gemv_common.h).
+int gemv_merge_epi(int splits);
+// One type's instances (gemv_<type>.hip); epi GEMV_EPI_* or gemv_merge_epi's.
+#define CN_GEMV_TYPE(t)                                                                    \
+  hipError_t gemv_##t##_launch(int epi, const GemvArgs& a, int num_cus, hipStream_t st);   \
+  hipError_t gemv_##t##_cols_launch(const GemvArgs& a, int ncols, int num_cus, char* pre, hipStream_t st);
+CN_GEMV_TYPE(q4_1) CN_GEMV_TYPE(q5_0) CN_GEMV_TYPE(q5_1) CN_GEMV_TYPE(q8_0) CN_GEMV_TYPE(q2_k) CN_GEMV_TYPE(q3_k)
+CN_GEMV_TYPE(q4_k) CN_GEMV_TYPE(q5_k) CN_GEMV_TYPE(q6_k) CN_GEMV_TYPE(iq4_nl) CN_GEMV_TYPE(iq4_xs)
+#undef CN_GEMV_TYPE
+hipError_t gemv_q4_0_launch(int epi, const GemvArgs& a, int num_cus, hipStream_t st);
 hipError_t gemv_launch(int qtype, int epi, const GemvArgs& a, int num_cus, hipStream_t st);
 hipError_t gemv_float_launch(int qtype, int epi, const GemvArgs& a, int num_cus, hipStream_t st);
 

@@ -132,8 +132,8 @@ CHATNET_API int chatnet_create(const chatnet_config* cfg, int device, chatnet_mo
  * (as DequantIQ.cs decodes them), each dispatched on its own type.  Q4_1,
  * Q5_0, Q5_1, Q2_K, Q8_K and the IQ types are also re-encoded on the
  * device at upload (u8 codes with an fp32 scale and offset per 16 weights,
- * M*(K/64)*96 bytes beside the stored blocks), the form the GEMV reads them
- * in.  An IQ3_S row's last block reads 28 bytes past the row, as the
+ * M*(K/64)*96 bytes beside the stored blocks), the form spans read them in
+ * and, for Q8_K and the IQ types but IQ4_NL and IQ4_XS, the GEMV.  An IQ3_S row's last block reads 28 bytes past the row, as the
  * reference does (DequantIQ.cs:255-283): the next row's first bytes, or for
  * the last row zeros (the reference reads whatever follows the tensor in the
  * file).  Without output.weight the LM head is token_embd.weight, of whatever
@@ -245,7 +245,8 @@ CHATNET_API int chatnet_get_logits(chatnet_model* m, float* logits_host);
  * zero).
  * Q4_0 with 2 <= N < 8, or N <= 16 with M*K*N <= 8*4096*4096, runs one
  * multi-column GEMV (each column the N = 1 product's exact arithmetic).  Other
- * calls with N >= 8 and a block type run the dequant-to-LDS fp16 MFMA GEMM (x
+ * calls with N > 16 and a block type (Q4_0, Q8_K and the IQ types above: N >= 8)
+ * run the dequant-to-LDS fp16 MFMA GEMM (x
  * rounded to fp16 after scaling each column by a power of two that keeps it
  * inside fp16's range, each weight rounded once to fp16; Q4_0 read as raw
  * blocks, the other types first re-encoded
@@ -255,10 +256,12 @@ CHATNET_API int chatnet_get_logits(chatnet_model* m, float* logits_host);
  * product's exact arithmetic), F16 with more columns than one launch of it
  * holds (8 up to K = 4864, fewer above) an MFMA product of the exact weights
  * with x as two fp16 planes, summed with compensation in fp32 (its error
- * against float64 is the GEMV's, 1e-7).  Any other call (block types at N < 8)
- * runs the fused GEMV once per column, which reads Q4_1,
- * Q5_0, Q5_1, Q2_K, Q8_K and the IQ types from that same re-encoded
- * copy, made in the workspace first.  A GEMM whose grid of 128 x 128 tiles
+ * against float64 is the GEMV's, 1e-7).  Q4_1, Q5_0, Q5_1,
+ * Q8_0, Q2_K .. Q6_K, IQ4_NL and IQ4_XS run up to 16 columns on their stored
+ * blocks with x to 23 bits of each 32 elements' largest (one column, and two or
+ * three of a large matrix: the fused GEMV per column); Q8_K and the other IQ
+ * types below 8 columns run the GEMV once per column on the re-encoded copy,
+ * made in the workspace first.  A GEMM whose grid of 128 x 128 tiles
  * is just over one tile per CU (e.g. 11008 x 4096 at N = 512) runs as a
  * stream-K launch: one whole tile per CU, the other tiles' K chunks shared
  * out evenly, a shared tile summed in K order by its last contributor (the

@@ -5,6 +5,7 @@ values, a capturing stream and the no-allocation variant."""
 import numpy as np
 import pytest
 
+import oracle
 from chatnet_amd import _native, hiprt, ops, synth
 from gpu_util import announce, gpu_matmul, normwise
 
@@ -88,6 +89,109 @@ def test_f16_columns_captured_without_a_workspace_and_noalloc(M, K, N):
     hiprt.synchronize()
     lib = _native.hip_lib()
     _native.check(lib.chatnet_matmul_noalloc(F16, w_d.ptr, x_d.ptr, y_d.ptr, M, K, N, stream.h))
+    stream.synchronize()
+    assert np.array_equal(y_d.to_numpy(np.float32, N * M).reshape(N, M), ref)
+    del graph
+    for b in (w_d, x_d, y_d):
+        b.free()
+
+
+BLOCK_TYPES = {3: "q4_1", 6: "q5_0", 7: "q5_1", 8: "q8_0", 10: "q2_k", 11: "q3_k", 12: "q4_k", 13: "q5_k", 14: "q6_k",
+               20: "iq4_nl", 23: "iq4_xs"}
+FINE_TYPES = (3, 6, 7, 10, 20, 23)  # x to 23 bits of its 16-element group, 19 for the others
+
+
+def digit_bound(qtype, x, w):
+    """Half a step of x's digits in every element: a step is at most 2^-22 of its
+    16-element group's maximum (fine types), or 2^-18 of its group's (of 16 or 32
+    elements); plus 16 roundings of 2^-24 of sum |w x| for the 32-bit sums."""
+    n = 16 if qtype in FINE_TYPES else 32
+    ax = np.abs(x).astype(np.float64)
+    g = np.repeat(ax.reshape(x.shape[0], -1, n).max(2), n, axis=1)
+    step = 2.0 ** (-22 if qtype in FINE_TYPES else -18)
+    return 0.5 * step * (g @ np.abs(w).T) + 16 * 2.0 ** -24 * (ax @ np.abs(w).T)
+
+
+# One column (the GEMV), then one, two and three tiles of digit rows (5, 10 and
+# 16 columns at most), one and two row tiles per wave (from 4097 rows), several
+# row groups per workgroup (over 16384 rows), rows whose x is staged in several
+# rounds, ahead of the launch or in the workgroup, and ragged last row tiles.
+@pytest.mark.parametrize("M,K,N", [
+    (1, 256, 1), (3, 512, 2), (130, 4096, 7), (37, 11008, 1), (37, 11008, 5), (65, 16384, 3), (8200, 768, 4),
+    (4100, 5120, 2), (5, 2304, 1), (17, 256, 6), (70, 1024, 10), (4200, 512, 8), (130, 2304, 16), (33, 11008, 11),
+    (17000, 256, 3),
+])
+@pytest.mark.parametrize("qtype", sorted(BLOCK_TYPES))
+def test_block_types_few_columns_match_float64(qtype, M, K, N):
+    """Every column against the float64 product of the dequantized weights, within
+    digit_bound."""
+    announce(f"few columns {BLOCK_TYPES[qtype]} M={M} K={K} N={N}")
+    t = synth.tensor(qtype, 31, f"few{qtype}-{M}x{K}", M, K)
+    x = synth.normal(32, f"fewx{N}x{K}", N * K, 1.0).reshape(N, K)
+    x[:, K // 2] *= 20.0
+    y = gpu_matmul(qtype, t.data, x, M, K)
+    w = oracle.dequant(qtype, t.data, M * K).reshape(M, K).astype(np.float64)
+    r = x.astype(np.float64) @ w.T
+    bound = digit_bound(qtype, x, w)
+    assert np.all(np.abs(y - r) <= bound), float(np.max(np.abs(y - r) / bound))
+
+
+def test_odd_rows_of_short_k_match_float64():
+    """K = 64 and 192: one pair of blocks, and rows whose records end mid-unit."""
+    for qtype in (3, 6, 7, 8, 20):
+        for (M, K, N) in [(1, 64, 1), (70, 64, 3), (33, 192, 5), (64, 960, 2)]:
+            announce(f"short rows {BLOCK_TYPES[qtype]} M={M} K={K} N={N}")
+            t = synth.tensor(qtype, 33, f"short{qtype}-{M}x{K}", M, K)
+            x = synth.normal(34, f"shortx{N}x{K}", N * K, 1.0).reshape(N, K)
+            y = gpu_matmul(qtype, t.data, x, M, K)
+            w = oracle.dequant(qtype, t.data, M * K).reshape(M, K).astype(np.float64)
+            assert np.all(np.abs(y - x.astype(np.float64) @ w.T) <= digit_bound(qtype, x, w))
+
+
+@pytest.mark.parametrize("qtype", [3, 6, 7, 10, 20, 23])
+@pytest.mark.parametrize("N", [1, 3])
+def test_non_finite_x_and_wide_magnitudes(qtype, N):
+    """A column with an infinity or NaN gives no finite output (the packed-unit
+    product these types ran before met it in fp32); columns of 1e30 and 1e-30
+    keep their accuracy."""
+    M, K = 40, 512
+    t = synth.tensor(qtype, 35, f"nf{qtype}", M, K)
+    w = oracle.dequant(qtype, t.data, M * K).reshape(M, K).astype(np.float64)
+    for bad in (np.inf, -np.inf, np.nan):
+        x = synth.normal(36, "nfx", N * K, 1.0).reshape(N, K)
+        x[N - 1, 77] = bad
+        y = gpu_matmul(qtype, t.data, x, M, K)
+        assert not np.any(np.isfinite(y[N - 1]))
+        assert np.all(np.isfinite(y[: N - 1]))
+    for mag in (1e30, 1e-30):
+        x = (synth.normal(37, "nfy", N * K, 1.0) * mag).reshape(N, K).astype(np.float32)
+        y = gpu_matmul(qtype, t.data, x, M, K)
+        r = x.astype(np.float64) @ w.T
+        assert max(normwise(y[n], r[n]) for n in range(N)) <= 2e-6
+
+
+@pytest.mark.parametrize("qtype", [12, 6])
+def test_few_columns_captured_without_a_workspace_and_noalloc(qtype):
+    """x staged ahead needs the stream's workspace: a capturing stream without one
+    and the no-allocation variant stage it in every workgroup, to the same bits."""
+    M, K, N = 96, 4096, 9
+    announce(f"few columns captured {BLOCK_TYPES[qtype]}")
+    t = synth.tensor(qtype, 38, f"cap{qtype}", M, K)
+    x = synth.normal(39, "capx", N * K, 1.0).reshape(N, K)
+    ref = gpu_matmul(qtype, t.data, x, M, K)
+    w_d = hiprt.DeviceBuffer.from_numpy(t.data, pad=256)
+    x_d, y_d = hiprt.DeviceBuffer.from_numpy(x), hiprt.DeviceBuffer(4 * N * M)
+    stream = hiprt.Stream()
+    graph = hiprt.Graph(stream, lambda: ops.matmul_ptr(qtype, w_d.ptr, x_d.ptr, y_d.ptr, M, K, N, stream.h))
+    for _ in range(2):
+        y_d.fill(0xFF)
+        hiprt.synchronize()
+        graph.launch()
+        stream.synchronize()
+        assert np.array_equal(y_d.to_numpy(np.float32, N * M).reshape(N, M), ref)
+    y_d.fill(0xFF)
+    hiprt.synchronize()
+    _native.check(_native.hip_lib().chatnet_matmul_noalloc(qtype, w_d.ptr, x_d.ptr, y_d.ptr, M, K, N, stream.h))
     stream.synchronize()
     assert np.array_equal(y_d.to_numpy(np.float32, N * M).reshape(N, M), ref)
     del graph
