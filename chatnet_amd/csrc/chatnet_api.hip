@@ -85,9 +85,9 @@ int device_cus(int dev) {
 // LlamaModel.cs:488-562) from packed units made at upload.
 bool is_matrix_type(uint32_t t) { return gemv_supports((int)t, 256); }
 
-// The types that spans and wide products read as packed units made ahead
-// (a model's at upload) and that chatnet_matmul_noalloc takes only while
-// their packed copy fits its scratch.
+// The types that chatnet_matmul_noalloc runs on the GEMM besides Q4_0, and takes
+// only while a packed copy of W would fit its scratch (those not in
+// gemv_needs_pack are read as stored since).
 bool packed_ahead(uint32_t t) {
   return gemv_needs_pack((int)t) || t == CHATNET_GGML_Q4_1 || t == CHATNET_GGML_Q5_0 || t == CHATNET_GGML_Q5_1 ||
          t == CHATNET_GGML_Q2_K || t == CHATNET_GGML_IQ4_NL || t == CHATNET_GGML_IQ4_XS;
@@ -576,13 +576,12 @@ int chatnet_upload_tensor(chatnet_model* m, const char* name, uint32_t type, con
     return fail(CHATNET_ERR_OUT_OF_MEMORY, "hipMalloc of %llu bytes for %s failed", (unsigned long long)nbytes, name);
   const bool neox_rows = c.arch == CHATNET_ARCH_QWEN2 && layer >= 0 &&
                          (slot == &m->layers[layer].wq || slot == &m->layers[layer].wk);
-  // Types that spans (or the embedding gather) read as packed units are
+  // Types the GEMV (or the embedding gather) reads only as packed units are
   // packed below, one pass over the uploaded rows; the stored blocks stay for
-  // the other readers.  The types the GEMV reads only packed keep the file's
-  // row order even where the Qwen2 row order applies (an IQ3_S row reads into
-  // the row after it in the file, DequantIQ.cs:255-283): their packed rows are
-  // put in that order instead.
-  const bool pack_now = (matrix && packed_ahead(type)) || (slot == &m->emb && !embed_raw_type(type));
+  // the other readers.  Such a matrix keeps the file's row order even where the
+  // Qwen2 row order applies (an IQ3_S row reads into the row after it in the
+  // file, DequantIQ.cs:255-283): its packed rows are put in that order instead.
+  const bool pack_now = (matrix && gemv_needs_pack((int)type)) || (slot == &m->emb && !embed_raw_type(type));
   const bool file_rows = gemv_needs_pack((int)type);
   if (neox_rows && !file_rows) {
     const size_t bpr = (size_t)(nbytes / ne1);
@@ -834,9 +833,9 @@ LayerMats layer_mats(Layer& L) { return {{&L.wq, &L.wk, &L.wv, &L.wo, &L.wg, &L.
 // How a span's projections read their weights, per GEMM of the layer (QKV,
 // O, gate/up, down): F16 and F32 matrices as their own rows (GEMM_W_F16 /
 // GEMM_W_F32), block types from their stored blocks when every matrix of that
-// GEMM in every layer is Q4_0 (GEMM_W_Q4_0) or every one is Q4_K
-// (GEMM_W_Q4_K), else as packed units (block types mixed freely, made once
-// per model).  The matrices one GEMM concatenates (q|k|v) or interleaves
+// GEMM in every layer has one type that has such a format
+// (gemm_stored_format), else as packed units (block types mixed freely, made
+// once per model).  The matrices one GEMM concatenates (q|k|v) or interleaves
 // (gate/up) must share a class (float type or block type); a span whose layers
 // cannot (ffn_gate Q4_0 with ffn_up F16, a type neither packable nor float)
 // runs token by token.
@@ -862,7 +861,7 @@ SpanPlan span_plan(chatnet_model* m, int n) {
   };
   const int group_of[7] = {SG_QKV, SG_QKV, SG_QKV, SG_O, SG_GU, SG_GU, SG_D};
   int gcls[4] = {0, 0, 0, 0};  // 0: not seen yet
-  bool all_q4_0[4] = {true, true, true, true}, all_q4_k[4] = {true, true, true, true};
+  int fmt[4] = {-2, -2, -2, -2};  // the stored format every matrix of the GEMM shares, -1: none, -2: not seen yet
   for (Layer& L : m->layers) {
     const LayerMats lm = layer_mats(L);
     for (int i = 0; i < 7; i++) {
@@ -872,14 +871,12 @@ SpanPlan span_plan(chatnet_model* m, int n) {
       int& g = gcls[gi];
       if (g == 0) g = k;
       else if (g != k) return p;
-      if (t->type != CHATNET_GGML_Q4_0 || !gemm_supports(CHATNET_GGML_Q4_0, (int)t->ne0)) all_q4_0[gi] = false;
-      if (t->type != CHATNET_GGML_Q4_K || t->ne0 % 256) all_q4_k[gi] = false;
+      const int f = gemm_stored_format((int)t->type, (int)t->ne0);
+      if (fmt[gi] == -2) fmt[gi] = f;
+      else if (fmt[gi] != f) fmt[gi] = -1;
     }
   }
-  for (int g = 0; g < 4; g++) {
-    if (gcls[g] != GEMM_W_PACKED) p.fmt[g] = gcls[g];
-    else p.fmt[g] = all_q4_0[g] ? GEMM_W_Q4_0 : (all_q4_k[g] ? GEMM_W_Q4_K : GEMM_W_PACKED);
-  }
+  for (int g = 0; g < 4; g++) p.fmt[g] = fmt[g] >= 0 ? fmt[g] : GEMM_W_PACKED;
   p.ok = true;
   return p;
 }
@@ -1211,18 +1208,19 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
   // 61.2).  Two columns (Q3_K, whose unpacking costs the most: three) of a
   // matrix of at least kTwoGemvs weights run the single-column GEMV for each
   // (11008 x 4096: Q4_K at 2 columns 13.1 against 16.6 us, Q3_K at 3 24.7
-  // against 29.0).  More columns run the GEMM: Q4_0 reads its
-  // raw blocks, the other types are packed into the workspace first, one pass
-  // over W (in the no-allocation variant only the packed_ahead types).  The
+  // against 29.0).  More columns run the GEMM on the
+  // stored blocks; Q3_K, Q6_K, Q8_K and the other IQ types are packed into the
+  // workspace first, one pass over W (the no-allocation variant runs the GEMM
+  // for Q4_0 and the packed_ahead types only).  The
   // types the GEMV reads only as packed units are packed for every N.
   constexpr int kColsGemv = 16;
   constexpr long long kTwoGemvs = 32LL << 20;
-  const bool raw = gemm_supports((int)type, K);
+  const int stored = gemm_stored_format((int)type, K);  // the GEMM's format on the stored blocks, -1: packed units
   const bool must_pack = gemv_needs_pack((int)type);
   const bool ahead = packed_ahead(type);
   const bool batched = N >= 8 && !(N <= kColsGemv && gemv_qcols_supports((int)type)) &&
-                       (raw || ahead || (!noalloc && gemm_pack_supports((int)type, K)));
-  const bool pack = must_pack || (batched && !raw);
+                       (type == CHATNET_GGML_Q4_0 || ahead || (!noalloc && gemm_pack_supports((int)type, K)));
+  const bool pack = must_pack || (batched && stored < 0);
   const uint8_t* wp = (const uint8_t*)w_dev;
   std::unique_lock<std::mutex> lk(g_enqueue_mu, std::defer_lock);
   if (batched || pack || (noalloc && ahead)) {
@@ -1234,7 +1232,7 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
     const size_t xh_bytes = cnt_bytes + (batched ? ((size_t)N * K * sizeof(uint16_t) + 255) & ~(size_t)255 : 0);
     const size_t xb_bytes = batched ? xh_bytes + (((size_t)N * sizeof(float) + 255) & ~(size_t)255) : cnt_bytes;
     const size_t part_bytes =
-        batched ? (gemm_workspace_bytes(M, N, K, cus, false, pack, !noalloc) + 255) & ~(size_t)255 : 0;
+        batched ? (gemm_workspace_bytes(M, N, K, cus, false, pack ? GEMM_W_PACKED : stored, !noalloc) + 255) & ~(size_t)255 : 0;
     const size_t pack_bytes = pack || (noalloc && ahead) ? gemm_pack_bytes(M, K) : 0;
     const size_t need = xb_bytes + part_bytes + pack_bytes;
     char* ws = nullptr;
@@ -1260,7 +1258,7 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
       GemmArgs g;
       memset(&g, 0, sizeof(g));
       g.qtype = (int)type;
-      g.packed = pack;
+      g.packed = pack ? GEMM_W_PACKED : stored;
       g.w[0] = g.w[1] = g.w[2] = wp;
       g.seg_rows[0] = M;
       g.seg_mode = GEMM_SEG_SINGLE;

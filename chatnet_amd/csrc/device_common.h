@@ -56,6 +56,22 @@ __device__ __forceinline__ float cn_ubyte(uint32_t v) {
   return (float)((v >> (8 * B)) & 0xFFu);
 }
 
+// Bits 0..3 of t at bit 0 of bytes 0..3.
+__device__ __forceinline__ uint32_t spread4(uint32_t t) { return ((t & 0xFu) * 0x00204081u) & 0x01010101u; }
+
+// IQ4_NL's values (DequantIQ.IQ4NL_Table, DequantIQ.cs:29-33) of the four 4-bit
+// indexes in the bytes of s: two byte permutes of the table's halves, then bit
+// 3 of each index picks one.
+__device__ __forceinline__ uint32_t iq4_values(uint32_t s) {
+  constexpr uint32_t T0 = 0xBFAD9881u, T1 = 0xF6EADDCFu;  // -127 -104 -83 -65 | -49 -35 -22 -10
+  constexpr uint32_t T2 = 0x26190D01u, T3 = 0x71594535u;  // 1 13 25 38 | 53 69 89 113
+  const uint32_t lo = __builtin_amdgcn_perm(T1, T0, s & 0x07070707u);
+  const uint32_t hi = __builtin_amdgcn_perm(T3, T2, s & 0x07070707u);
+  const uint32_t b = (s >> 3) & 0x01010101u;
+  const uint32_t m = (b << 8) - b;  // 0xFF in the bytes whose bit 3 is set
+  return (hi & m) | (lo & ~m);
+}
+
 // Inputs of the exact-weight span GEMM (x of every projection in a span) are
 // two fp16 planes, hi = fp16(x) and lo = fp16(x - hi) (about 22 significant
 // bits while |x| stays in fp16's normal range), with each 32-element block

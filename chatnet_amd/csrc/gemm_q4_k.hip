@@ -1,0 +1,10 @@
+// gemm_q4_k.hip — the matrix-core GEMM (gemm_tile.h) over Q4_K weights.
+#include "gemm_tile.h"
+
+hipError_t gemm_q4_k_plane(const GemmArgs& a, int tn, int mt, int grid, hipStream_t st) {
+  return launch_one_plane<GEMM_W_Q4_K>(a, tn, mt, grid, st);
+}
+
+hipError_t gemm_q4_k_span(const GemmArgs& a, int tn, int stages, int grid, hipStream_t st) {
+  return launch_span<GEMM_W_Q4_K>(a, tn, stages, grid, st);
+}

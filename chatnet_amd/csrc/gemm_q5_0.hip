@@ -1,0 +1,10 @@
+// gemm_q5_0.hip — the matrix-core GEMM (gemm_tile.h) over Q5_0 weights.
+#include "gemm_tile.h"
+
+hipError_t gemm_q5_0_plane(const GemmArgs& a, int tn, int mt, int grid, hipStream_t st) {
+  return launch_one_plane<GEMM_W_Q5_0>(a, tn, mt, grid, st);
+}
+
+hipError_t gemm_q5_0_span(const GemmArgs& a, int tn, int stages, int grid, hipStream_t st) {
+  return launch_span<GEMM_W_Q5_0>(a, tn, stages, grid, st);
+}

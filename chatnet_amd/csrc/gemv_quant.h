@@ -1018,22 +1018,6 @@ __device__ __forceinline__ void dot_unit_k45_dig8(const uint32_t (*w)[QTraits<QT
 template <int QT>
 constexpr bool group_min() { return QT == QT_Q4_1 || QT == QT_Q5_1 || QT == QT_Q2_K || QT == QT_Q4_K || QT == QT_Q5_K; }
 
-// The fifth bits of elements 16hh + 4k .. +3 (low bits of `t`) at bit 0 of each byte.
-__device__ __forceinline__ uint32_t spread4(uint32_t t) { return ((t & 0xFu) * 0x00204081u) & 0x01010101u; }
-
-// IQ4_NL's values (DequantIQ.IQ4NL_Table, DequantIQ.cs:29-33) of the four 4-bit
-// indexes in the bytes of s: two byte permutes of the table's halves, then bit
-// 3 of each index picks one.
-__device__ __forceinline__ uint32_t iq4_values(uint32_t s) {
-  constexpr uint32_t T0 = 0xBFAD9881u, T1 = 0xF6EADDCFu;  // -127 -104 -83 -65 | -49 -35 -22 -10
-  constexpr uint32_t T2 = 0x26190D01u, T3 = 0x71594535u;  // 1 13 25 38 | 53 69 89 113
-  const uint32_t lo = __builtin_amdgcn_perm(T1, T0, s & 0x07070707u);
-  const uint32_t hi = __builtin_amdgcn_perm(T3, T2, s & 0x07070707u);
-  const uint32_t b = (s >> 3) & 0x01010101u;
-  const uint32_t m = (b << 8) - b;  // 0xFF in the bytes whose bit 3 is set
-  return (hi & m) | (lo & ~m);
-}
-
 template <int QT>
 __device__ __forceinline__ void unit_group(const uint32_t* w, int h, int g, uint32_t (&q)[4], float& a, float& b) {
   b = 0.f;

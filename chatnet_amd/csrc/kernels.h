@@ -115,10 +115,14 @@ hipError_t gemv_float_launch(int qtype, int epi, const GemvArgs& a, int num_cus,
 // GEMV_EPI_SWIGLU h[n][vr/2] = silu(acc[vr even]) * acc[vr odd] as fp16 hi + lo
 // planes (hb, hb_lo) in the cn_span_pos order.
 enum { GEMM_SEG_SINGLE = 0, GEMM_SEG_CONCAT = 1, GEMM_SEG_INTERLEAVE = 2 };
-// How W is stored (GemmArgs::packed): raw Q4_0 blocks, gemm_pack_launch units
-// (any packable type), or (the span kernel only) rows of F16 / F32 values or
-// raw Q4_K super-blocks.
-enum { GEMM_W_Q4_0 = 0, GEMM_W_PACKED = 1, GEMM_W_F16 = 2, GEMM_W_F32 = 3, GEMM_W_Q4_K = 4 };
+// How W is stored (GemmArgs::packed): gemm_pack_launch units (any packable
+// type), rows of F16 / F32 values (the span kernel only), or a type's own blocks.
+enum { GEMM_W_Q4_0 = 0, GEMM_W_PACKED = 1, GEMM_W_F16 = 2, GEMM_W_F32 = 3, GEMM_W_Q4_K = 4, GEMM_W_Q8_0 = 5,
+       GEMM_W_Q5_0 = 6, GEMM_W_Q4_1 = 7, GEMM_W_Q5_1 = 8, GEMM_W_IQ4_NL = 9, GEMM_W_Q5_K = 10, GEMM_W_IQ4_XS = 11,
+       GEMM_W_Q2_K = 12, GEMM_W_COUNT = 13 };
+// The format that reads matrices of `qtype` as they are stored, -1 if there is
+// none (Q3_K, Q6_K, Q8_K and the other IQ types, read as packed units).
+int gemm_stored_format(int qtype, int K);
 struct GemmArgs {
   int qtype;
   int packed;             // GEMM_W_*: how w is stored
@@ -166,6 +170,17 @@ size_t gemm_workspace_bytes(int M, int N, int K, int num_cus, bool precise, int 
 // the epilogue ran): the caller folds them into its next kernel
 // (add_rmsnorm_span_launch for a residual add).
 hipError_t gemm_launch(const GemmArgs& a, int num_cus, hipStream_t st, int* splits_left = nullptr);
+// One format's instances (gemm_<format>.hip): column tiles per wave, then row
+// tiles per wave (one-plane kernel) or ring stages (span kernel).
+#define CN_GEMM_SPAN(f) hipError_t gemm_##f##_span(const GemmArgs& a, int tn, int stages, int grid, hipStream_t st);
+#define CN_GEMM_FMT(f) \
+  hipError_t gemm_##f##_plane(const GemmArgs& a, int tn, int mt, int grid, hipStream_t st); \
+  CN_GEMM_SPAN(f)
+CN_GEMM_FMT(q4_0) CN_GEMM_FMT(packed) CN_GEMM_FMT(q4_k) CN_GEMM_FMT(q8_0) CN_GEMM_FMT(q5_0) CN_GEMM_FMT(q4_1)
+CN_GEMM_FMT(q5_1) CN_GEMM_FMT(iq4_nl) CN_GEMM_FMT(q5_k) CN_GEMM_FMT(iq4_xs) CN_GEMM_FMT(q2_k) CN_GEMM_SPAN(f16)
+CN_GEMM_SPAN(f32)
+#undef CN_GEMM_FMT
+#undef CN_GEMM_SPAN
 // x [N][K] fp32 -> the one-plane GEMM's input: xh[n] = fp16(x[n] * 2^e_n) in
 // the cn_span_pos order, 2^e_n bringing max|x[n]| into [2^14, 2^15), and
 // xinv[n] = 2^-e_n.  K % 32 == 0, K <= 16384.

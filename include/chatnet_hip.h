@@ -129,11 +129,10 @@ CHATNET_API int chatnet_create(const chatnet_config* cfg, int device, chatnet_mo
  * of every type LlamaModel.MatVecMulByType dispatches (LlamaModel.cs:470-567):
  * F32, F16, Q4_0, Q4_1, Q5_0, Q5_1, Q8_0, Q2_K, Q3_K, Q4_K, Q5_K, Q6_K, Q8_K
  * and IQ2_XXS, IQ2_XS, IQ3_XXS, IQ1_S, IQ4_NL, IQ3_S, IQ2_S, IQ4_XS, IQ1_M
- * (as DequantIQ.cs decodes them), each dispatched on its own type.  Q4_1,
- * Q5_0, Q5_1, Q2_K, Q8_K and the IQ types are also re-encoded on the
+ * (as DequantIQ.cs decodes them), each dispatched on its own type.  Q8_K
+ * and the IQ types other than IQ4_NL and IQ4_XS are also re-encoded on the
  * device at upload (u8 codes with an fp32 scale and offset per 16 weights,
- * M*(K/64)*96 bytes beside the stored blocks), the form spans read them in
- * and, for Q8_K and the IQ types but IQ4_NL and IQ4_XS, the GEMV.  An IQ3_S row's last block reads 28 bytes past the row, as the
+ * M*(K/64)*96 bytes beside the stored blocks), the form they are read in.  An IQ3_S row's last block reads 28 bytes past the row, as the
  * reference does (DequantIQ.cs:255-283): the next row's first bytes, or for
  * the last row zeros (the reference reads whatever follows the tensor in the
  * file).  Without output.weight the LM head is token_embd.weight, of whatever
@@ -161,9 +160,10 @@ CHATNET_API int chatnet_upload_tensor(chatnet_model* m, const char* name, uint32
  * gate|up, down) reads its matrices in one format: F16 rows as stored (two
  * products per step, exact weights), F32 rows split into fp16 hi + lo as
  * read (three products, ~22 bits), block types from their stored blocks when
- * every matrix of that GEMM is Q4_0 (each weight exact as two fp16 planes) or
- * every one is Q4_K (~22 bits), otherwise re-encoded once into packed units
- * kept for the model's lifetime (~22 bits).  Shorter spans, and models whose
+ * every matrix of that GEMM is of one type (Q4_0: each weight exact as two
+ * fp16 planes; Q4_1, Q5_0, Q5_1, Q8_0, Q2_K, Q4_K, Q5_K, IQ4_NL, IQ4_XS: ~22
+ * bits), otherwise re-encoded once into packed units kept for the model's
+ * lifetime (~22 bits).  Shorter spans, and models whose
  * layers give one GEMM matrices of both a float and a block type (ffn_gate
  * Q4_0 with ffn_up F16), run token by token. */
 CHATNET_API int chatnet_forward(chatnet_model* m, const int32_t* tokens, int n, int position,
@@ -248,8 +248,8 @@ CHATNET_API int chatnet_get_logits(chatnet_model* m, float* logits_host);
  * calls with N > 16 and a block type (Q4_0, Q8_K and the IQ types above: N >= 8)
  * run the dequant-to-LDS fp16 MFMA GEMM (x
  * rounded to fp16 after scaling each column by a power of two that keeps it
- * inside fp16's range, each weight rounded once to fp16; Q4_0 read as raw
- * blocks, the other types first re-encoded
+ * inside fp16's range, each weight rounded once to fp16; the blocks read as
+ * stored, Q3_K, Q6_K, Q8_K and the other IQ types first re-encoded
  * into the workspace as u8 codes with an fp32 scale and offset per 16 weights,
  * M*(K/64)*96 bytes, giving the same dequantized values).  F32 and F16 rows
  * with several columns run a multi-column GEMV (each column the N = 1

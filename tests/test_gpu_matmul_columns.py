@@ -197,3 +197,20 @@ def test_few_columns_captured_without_a_workspace_and_noalloc(qtype):
     del graph
     for b in (w_d, x_d, y_d):
         b.free()
+
+
+# Types whose GEMM reads the stored blocks: 32-, 64- and 128-column tiles, one
+# chunk and odd chunk counts, K split and whole, single and ragged rows.
+@pytest.mark.parametrize("M,K,N", [(1, 256, 17), (130, 768, 40), (67, 2304, 129), (300, 4096, 65), (2050, 512, 300)])
+@pytest.mark.parametrize("qtype", [3, 6, 7, 8, 10, 12, 13, 20, 23])
+def test_stored_block_gemm_edges(qtype, M, K, N):
+    """Both operands meet in fp16, each rounded once: |error| <= 2 * 2^-11 (1 +
+    2^-11) of sum |w x|, and the 32-bit sums' part far below."""
+    announce(f"stored gemm {BLOCK_TYPES[qtype]} M={M} K={K} N={N}")
+    t = synth.tensor(qtype, 41, f"sg{qtype}-{M}x{K}", M, K)
+    x = synth.normal(42, f"sgx{N}x{K}", N * K, 1.0).reshape(N, K)
+    y = gpu_matmul(qtype, t.data, x, M, K)
+    w = oracle.dequant(qtype, t.data, M * K).reshape(M, K).astype(np.float64)
+    r = x.astype(np.float64) @ w.T
+    scale = np.abs(x).astype(np.float64) @ np.abs(w).T
+    assert np.all(np.abs(y - r) <= 2.0 ** -10 * 1.01 * scale), float(np.max(np.abs(y - r) / scale))
