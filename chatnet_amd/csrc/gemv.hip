@@ -94,16 +94,36 @@ bool gemv_qcols_supports(int qtype) {
   return qtype == 3 || qtype == 6 || qtype == 7 || qtype == 8 || (qtype >= 10 && qtype <= 14) || qtype == 20 || qtype == 23;
 }
 
-// Staging x costs a workgroup about 15 VALU instructions an element, so from
-// 22000 elements per CU on (columns x K, times the workgroups a CU runs) it is
-// done once ahead, a launch of 3 us: Q4_K 11008 x 4096 at 4 columns 20.8 us with
-// every workgroup staging and 17.9 ahead, at 2 columns 16.6 and 17.8; Q8_0 4096
-// x 4096 at 4 columns 8.8 and 11.7, at 7 columns 13.1 and 11.9.
-size_t gemv_qcols_workspace(int M, int K, int N, int num_cus) {
-  const int n = N < kColsMax ? N : kColsMax;
+// Few row groups and long rows (at most half a workgroup of 16 rows per CU, at
+// least 24 steps of 128 weights): K shared out over up to 16 workgroups per row
+// group, each wave keeping a step, and a launch that adds the shares: Q4_K 164 x
+// 11008 at 6 columns 21.2 -> 10.9 us, Q8_0 90 x 10432 at 2 11.3 -> 7.9.  At up to
+// two workgroups per CU it lost (4096 x 4096 at 5 columns 9.0 -> 11.1 us, 3000 x
+// 8192 at 8 16.1 -> 27.8; 1500 x 14336 won 1 to 3 us of 13 to 29).
+// Otherwise staging x costs a workgroup about 15 VALU instructions an element,
+// so from 22000 elements per CU on (columns x K, times the workgroups a CU runs)
+// it is done once ahead, a launch of 3 us: Q4_K 11008 x 4096 at 4 columns 20.8
+// us with every workgroup staging and 17.9 ahead, at 2 columns 16.6 and 17.8;
+// Q8_0 4096 x 4096 at 4 columns 8.8 and 11.7, at 7 columns 13.1 and 11.9.
+static int mcol_shares(int M, int K, int num_cus) {
+  const int groups = (M + 15) / 16, nsteps = (K + 127) / 128;
+  if (nsteps < 24 || 2 * groups > num_cus) return 1;
+  int s = num_cus / groups;
+  if (s > nsteps / 8) s = nsteps / 8;
+  return s > 16 ? 16 : s;
+}
+
+static bool mcol_ahead(int M, int K, int n, int num_cus) {
   const long long rows = M <= 16 * num_cus ? 16 : 32;
   const double wgs = (double)((M + rows - 1) / rows) / num_cus;
-  if ((double)n * K * (wgs < 1 ? 1 : wgs > 2 ? 2 : wgs) < 22000.0) return 0;
+  return (double)n * K * (wgs < 1 ? 1 : wgs > 2 ? 2 : wgs) >= 22000.0;
+}
+
+size_t gemv_qcols_workspace(int M, int K, int N, int num_cus) {
+  const int n = N < kColsMax ? N : kColsMax;
+  const int shares = mcol_shares(M, K, num_cus);
+  if (shares > 1) return (size_t)shares * n * M * sizeof(float);
+  if (!mcol_ahead(M, K, n, num_cus)) return 0;
   const size_t tiles = (3 * n + 15) / 16;
   return (size_t)((K + 127) / 128) * 4 * tiles * 704;  // the largest block (gemv_mcol.h)
 }
@@ -113,6 +133,12 @@ hipError_t gemv_qcols_launch(int qtype, const void* w, const float* x, float* y,
   if (!gemv_qcols_supports(qtype) || !gemv_supports(qtype, K) || M <= 0 || N < 1 || !w || !x || !y)
     return hipErrorInvalidValue;
   const int g = kColsMax;
+  McolPlan plan{nullptr, 1, nullptr};
+  if (ws) {
+    plan.shares = mcol_shares(M, K, num_cus);
+    if (plan.shares > 1) plan.part = static_cast<float*>(ws);
+    else plan.pre = static_cast<char*>(ws);
+  }
   for (int c0 = 0; c0 < N;) {
     const int left = N - c0, groups = (left + g - 1) / g;
     const int nc = (left + groups - 1) / groups;  // even groups: 17 columns run as 9 + 8
@@ -127,17 +153,17 @@ hipError_t gemv_qcols_launch(int qtype, const void* w, const float* x, float* y,
     hipError_t e;
     if (nc == 1) e = gemv_launch(qtype, GEMV_EPI_STORE, a, num_cus, st);
     else switch (qtype) {
-      case 3: e = gemv_q4_1_cols_launch(a, nc, num_cus, static_cast<char*>(ws), st); break;
-      case 6: e = gemv_q5_0_cols_launch(a, nc, num_cus, static_cast<char*>(ws), st); break;
-      case 7: e = gemv_q5_1_cols_launch(a, nc, num_cus, static_cast<char*>(ws), st); break;
-      case 8: e = gemv_q8_0_cols_launch(a, nc, num_cus, static_cast<char*>(ws), st); break;
-      case 10: e = gemv_q2_k_cols_launch(a, nc, num_cus, static_cast<char*>(ws), st); break;
-      case 11: e = gemv_q3_k_cols_launch(a, nc, num_cus, static_cast<char*>(ws), st); break;
-      case 12: e = gemv_q4_k_cols_launch(a, nc, num_cus, static_cast<char*>(ws), st); break;
-      case 13: e = gemv_q5_k_cols_launch(a, nc, num_cus, static_cast<char*>(ws), st); break;
-      case 14: e = gemv_q6_k_cols_launch(a, nc, num_cus, static_cast<char*>(ws), st); break;
-      case 20: e = gemv_iq4_nl_cols_launch(a, nc, num_cus, static_cast<char*>(ws), st); break;
-      default: e = gemv_iq4_xs_cols_launch(a, nc, num_cus, static_cast<char*>(ws), st); break;
+      case 3: e = gemv_q4_1_cols_launch(a, nc, num_cus, plan, st); break;
+      case 6: e = gemv_q5_0_cols_launch(a, nc, num_cus, plan, st); break;
+      case 7: e = gemv_q5_1_cols_launch(a, nc, num_cus, plan, st); break;
+      case 8: e = gemv_q8_0_cols_launch(a, nc, num_cus, plan, st); break;
+      case 10: e = gemv_q2_k_cols_launch(a, nc, num_cus, plan, st); break;
+      case 11: e = gemv_q3_k_cols_launch(a, nc, num_cus, plan, st); break;
+      case 12: e = gemv_q4_k_cols_launch(a, nc, num_cus, plan, st); break;
+      case 13: e = gemv_q5_k_cols_launch(a, nc, num_cus, plan, st); break;
+      case 14: e = gemv_q6_k_cols_launch(a, nc, num_cus, plan, st); break;
+      case 20: e = gemv_iq4_nl_cols_launch(a, nc, num_cus, plan, st); break;
+      default: e = gemv_iq4_xs_cols_launch(a, nc, num_cus, plan, st); break;
     }
     if (e != hipSuccess) return e;
     c0 += nc;

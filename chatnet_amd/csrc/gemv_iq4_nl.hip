@@ -6,6 +6,6 @@ hipError_t gemv_iq4_nl_launch(int epi, const GemvArgs& a, int num_cus, hipStream
   return launch_type<QT_IQ4_NL>(epi, a, num_cus, st);
 }
 
-hipError_t gemv_iq4_nl_cols_launch(const GemvArgs& a, int ncols, int num_cus, char* pre, hipStream_t st) {
-  return launch_mcol<QT_IQ4_NL>(a, ncols, num_cus, pre, st);
+hipError_t gemv_iq4_nl_cols_launch(const GemvArgs& a, int ncols, int num_cus, const McolPlan& p, hipStream_t st) {
+  return launch_mcol<QT_IQ4_NL>(a, ncols, num_cus, p, st);
 }

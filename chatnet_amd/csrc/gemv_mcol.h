@@ -350,19 +350,23 @@ __global__ __launch_bounds__(CN_BLOCK) void mcol_prep_kernel(const float* __rest
 // weight rows per wave.  The eight waves of a workgroup are rg row groups x 8 /
 // rg interleaved shares of K.  kc elements of x at a time are staged in LDS, or
 // with PRE copied from what mcol_prep_kernel staged (pre).
+// With several workgroups along K (blockIdx.y, spb steps each) the sums go to
+// part [blockIdx.y][column][row].
 template <int QT, int CT, int RT, bool PRE>
-__global__ __launch_bounds__(512) void gemv_mcol_kernel(GemvArgs a, int ncols, int kc, int rg, const char* pre) {
+__global__ __launch_bounds__(512) void gemv_mcol_kernel(GemvArgs a, int ncols, int kc, int rg, int spb, const char* pre,
+                                                       float* part) {
   using T = QTraits<QT>;
   constexpr int NW = 8, NR = mc_raw<QT>(), BB = mc_block_bytes<QT>();
   constexpr bool HALF = mc_half_scales<QT>(), MIN = group_min<QT>();
   extern __shared__ __attribute__((aligned(16))) char mlds[];
-  const int K = a.K, M = a.n_vrows;
+  const int M = a.n_vrows;
+  const int kb = blockIdx.y * spb * 128, K = min(a.K, kb + spb * 128);  // this workgroup's share
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int p = lane >> 4, li = lane & 15;
   const int nks = NW / rg, ks = wave % nks;
   const int row0 = (blockIdx.x * rg + wave / nks) * (16 * RT);
-  const size_t bpr = (size_t)(K / T::BLOCK) * T::BLOCK_BYTES;
-  const int nsteps = (K + 127) >> 7;
+  const size_t bpr = (size_t)(a.K / T::BLOCK) * T::BLOCK_BYTES;
+  const int nsteps = (K + 127) >> 7;  // end of the share
 
   const cn_gbyte* rp[RT];
 #pragma unroll
@@ -370,9 +374,9 @@ __global__ __launch_bounds__(512) void gemv_mcol_kernel(GemvArgs a, int ncols, i
   uint32_t raw[RT][NR];
   auto load = [&](int s) {
 #pragma unroll
-    for (int t = 0; t < RT; t++) mc_load<QT>(rp[t], min(s, nsteps - 1), p, K, raw[t]);
+    for (int t = 0; t < RT; t++) mc_load<QT>(rp[t], min(s, nsteps - 1), p, a.K, raw[t]);
   };
-  load(ks);  // travels while x is staged
+  load((kb >> 7) + ks);  // travels while x is staged
 
   float acc[RT][CT][4];
 #pragma unroll
@@ -382,9 +386,9 @@ __global__ __launch_bounds__(512) void gemv_mcol_kernel(GemvArgs a, int ncols, i
 #pragma unroll
       for (int i = 0; i < 4; i++) acc[t][c][i] = 0.f;
 
-  for (int k0 = 0; k0 < K; k0 += kc) {
+  for (int k0 = kb; k0 < K; k0 += kc) {
     const int kn = (min(kc, K - k0) + 127) & ~127;  // staged with zeros past K
-    if (k0) __syncthreads();
+    if (k0 > kb) __syncthreads();
     if constexpr (PRE) {  // a copy of the staged blocks
       const char* src = pre + (size_t)(k0 >> 5) * CT * BB;
       const int pieces = (kn >> 5) * CT * (BB / 16);
@@ -398,7 +402,7 @@ __global__ __launch_bounds__(512) void gemv_mcol_kernel(GemvArgs a, int ncols, i
       for (int t = threadIdx.x; t < ncols * halves; t += 512) {
         const int c = t / halves, hb = t - c * halves, k = k0 + 16 * hb;
         float v[16];
-        mc_load16(a.x + (size_t)c * K + k, k < K, v);
+        mc_load16(a.x + (size_t)c * a.K + k, k < K, v);
         mc_stage<QT, CT>(v, c, hb, mlds);
       }
     }
@@ -467,19 +471,31 @@ __global__ __launch_bounds__(512) void gemv_mcol_kernel(GemvArgs a, int ncols, i
       }
       v += part;
     }
-    if (row < M) a.out[0][(size_t)c * M + row] = v;
+    float* to = part ? part + (size_t)blockIdx.y * ncols * M : a.out[0];
+    if (row < M) to[(size_t)c * M + row] = v;
   }
 }
 
+// y[i] = sum over the K shares, in order.
+__global__ __launch_bounds__(CN_BLOCK) void mcol_reduce_kernel(const float* __restrict__ part, float* __restrict__ y,
+                                                              int n, int shares) {
+  const int i = blockIdx.x * CN_BLOCK + threadIdx.x;
+  if (i >= n) return;
+  float v = 0.f;
+  for (int s = 0; s < shares; s++) v += part[(size_t)s * n + i];
+  y[i] = v;
+}
+
 template <int QT, int CT, int RT, bool PRE>
-hipError_t launch_mcol_one(const GemvArgs& a, int ncols, int num_cus, const char* pre, hipStream_t st) {
+hipError_t launch_mcol_one(const GemvArgs& a, int ncols, int num_cus, const char* pre, int shares, float* part,
+                           hipStream_t st) {
   // staged x: at most 78 KB where two workgroups share a CU, else 156 KB; when
   // it takes several rounds, a multiple of the waves' turns
   constexpr int per_step = 4 * CT * mc_block_bytes<QT>();
   const int groups = (a.n_vrows + 16 * RT - 1) / (16 * RT);
   int rg = 1;
   while (rg < 8 && (groups + rg - 1) / rg > 2 * num_cus) rg *= 2;
-  const int nsteps = (a.K + 127) / 128, turn = 8 / rg;
+  const int spb = ((a.K + 127) / 128 + shares - 1) / shares, nsteps = spb, turn = 8 / rg;
   int fit = (78 * 1024) / per_step;  // steps of 128
   if ((groups + rg - 1) / rg <= num_cus) fit = (156 * 1024) / per_step;
   const int steps = nsteps <= fit ? nsteps : fit / turn * turn;
@@ -492,38 +508,43 @@ hipError_t launch_mcol_one(const GemvArgs& a, int ncols, int num_cus, const char
     const hipError_t e = allow_full_lds(reinterpret_cast<const void*>(kern), lds_done);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(kern, dim3((groups + rg - 1) / rg), dim3(512), smem, st, a, ncols, steps * 128, rg, pre);
+  hipLaunchKernelGGL(kern, dim3((groups + rg - 1) / rg, shares), dim3(512), smem, st, a, ncols, steps * 128, rg, spb, pre,
+                     shares > 1 ? part : nullptr);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || shares == 1) return e;
+  const int n = ncols * a.n_vrows;
+  hipLaunchKernelGGL(mcol_reduce_kernel, dim3((n + CN_BLOCK - 1) / CN_BLOCK), dim3(CN_BLOCK), 0, st, part, a.out[0], n,
+                     shares);
   return hipGetLastError();
 }
 
 // One row tile per wave while that leaves at most a workgroup per CU, else two
 // (each x fragment read then feeds two products).
 template <int QT, int CT>
-hipError_t launch_mcol_ct(const GemvArgs& a, int ncols, int num_cus, char* pre, hipStream_t st) {
+hipError_t launch_mcol_ct(const GemvArgs& a, int ncols, int num_cus, const McolPlan& p, hipStream_t st) {
   const bool one = CT == 3 || a.n_vrows <= 16 * num_cus;
-  if (pre) {
+  if (p.pre) {
     const int halves = (a.K + 127) / 128 * 8;
     hipLaunchKernelGGL((mcol_prep_kernel<QT, CT>), dim3((halves + CN_BLOCK - 1) / CN_BLOCK, ncols), dim3(CN_BLOCK), 0, st,
-                       a.x, a.K, halves, pre);
+                       a.x, a.K, halves, p.pre);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if constexpr (CT < 3) {
-      if (!one) return launch_mcol_one<QT, CT, 2, true>(a, ncols, num_cus, pre, st);
+      if (!one) return launch_mcol_one<QT, CT, 2, true>(a, ncols, num_cus, p.pre, 1, nullptr, st);
     }
-    return launch_mcol_one<QT, CT, 1, true>(a, ncols, num_cus, pre, st);
+    return launch_mcol_one<QT, CT, 1, true>(a, ncols, num_cus, p.pre, 1, nullptr, st);
   }
   if constexpr (CT < 3) {
-    if (!one) return launch_mcol_one<QT, CT, 2, false>(a, ncols, num_cus, pre, st);
+    if (!one) return launch_mcol_one<QT, CT, 2, false>(a, ncols, num_cus, nullptr, 1, nullptr, st);
   }
-  return launch_mcol_one<QT, CT, 1, false>(a, ncols, num_cus, pre, st);
+  return launch_mcol_one<QT, CT, 1, false>(a, ncols, num_cus, nullptr, p.shares, p.part, st);
 }
 
-// pre: workspace for the staged x, or null to stage it in every workgroup.
 template <int QT>
-hipError_t launch_mcol(const GemvArgs& a, int ncols, int num_cus, char* pre, hipStream_t st) {
-  if (ncols <= 5) return launch_mcol_ct<QT, 1>(a, ncols, num_cus, pre, st);
-  if (ncols <= 10) return launch_mcol_ct<QT, 2>(a, ncols, num_cus, pre, st);
-  return launch_mcol_ct<QT, 3>(a, ncols, num_cus, pre, st);
+hipError_t launch_mcol(const GemvArgs& a, int ncols, int num_cus, const McolPlan& p, hipStream_t st) {
+  if (ncols <= 5) return launch_mcol_ct<QT, 1>(a, ncols, num_cus, p, st);
+  if (ncols <= 10) return launch_mcol_ct<QT, 2>(a, ncols, num_cus, p, st);
+  return launch_mcol_ct<QT, 3>(a, ncols, num_cus, p, st);
 }
 
 }  // namespace

@@ -6,6 +6,6 @@ hipError_t gemv_q6_k_launch(int epi, const GemvArgs& a, int num_cus, hipStream_t
   return launch_type<QT_Q6_K>(epi, a, num_cus, st);
 }
 
-hipError_t gemv_q6_k_cols_launch(const GemvArgs& a, int ncols, int num_cus, char* pre, hipStream_t st) {
-  return launch_mcol<QT_Q6_K>(a, ncols, num_cus, pre, st);
+hipError_t gemv_q6_k_cols_launch(const GemvArgs& a, int ncols, int num_cus, const McolPlan& p, hipStream_t st) {
+  return launch_mcol<QT_Q6_K>(a, ncols, num_cus, p, st);
 }

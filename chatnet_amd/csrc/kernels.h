@@ -91,8 +91,15 @@ hipError_t gemv_float_cols_launch(int qtype, const void* w, const float* x, floa
 // x on the int8 matrix cores (gemv_mcol.h), up to 16 per launch, x to 23 bits of
 // each 32-element block's largest.
 bool gemv_qcols_supports(int qtype);
-// Workspace for x staged once ahead of the product (0: not worth the launch,
-// every workgroup stages it); gemv_qcols_launch takes it or null.
+// How a few-column product uses the workspace, if it has one: x staged once ahead
+// of the product (pre), or K shared out over `shares` workgroups per row group
+// whose sums meet in part.
+struct McolPlan {
+  char* pre;
+  int shares;
+  float* part;
+};
+// The workspace gemv_qcols_launch wants (0: none); it takes it or null.
 size_t gemv_qcols_workspace(int M, int K, int N, int num_cus);
 hipError_t gemv_qcols_launch(int qtype, const void* w, const float* x, float* y, int M, int K, int N, int num_cus,
                              void* ws, hipStream_t st);
@@ -101,7 +108,7 @@ int gemv_merge_epi(int splits);
 // One type's instances (gemv_<type>.hip); epi GEMV_EPI_* or gemv_merge_epi's.
 #define CN_GEMV_TYPE(t)                                                                    \
   hipError_t gemv_##t##_launch(int epi, const GemvArgs& a, int num_cus, hipStream_t st);   \
-  hipError_t gemv_##t##_cols_launch(const GemvArgs& a, int ncols, int num_cus, char* pre, hipStream_t st);
+  hipError_t gemv_##t##_cols_launch(const GemvArgs& a, int ncols, int num_cus, const McolPlan& p, hipStream_t st);
 CN_GEMV_TYPE(q4_1) CN_GEMV_TYPE(q5_0) CN_GEMV_TYPE(q5_1) CN_GEMV_TYPE(q8_0) CN_GEMV_TYPE(q2_k) CN_GEMV_TYPE(q3_k)
 CN_GEMV_TYPE(q4_k) CN_GEMV_TYPE(q5_k) CN_GEMV_TYPE(q6_k) CN_GEMV_TYPE(iq4_nl) CN_GEMV_TYPE(iq4_xs)
 #undef CN_GEMV_TYPE

@@ -170,15 +170,21 @@ def test_non_finite_x_and_wide_magnitudes(qtype, N):
         assert max(normwise(y[n], r[n]) for n in range(N)) <= 2e-6
 
 
+@pytest.mark.parametrize("M,same_order", [(2100, True), (96, False)])
 @pytest.mark.parametrize("qtype", [12, 6])
-def test_few_columns_captured_without_a_workspace_and_noalloc(qtype):
-    """x staged ahead needs the stream's workspace: a capturing stream without one
-    and the no-allocation variant stage it in every workgroup, to the same bits."""
-    M, K, N = 96, 4096, 9
+def test_few_columns_captured_without_a_workspace_and_noalloc(qtype, M, same_order):
+    """x staged ahead, and K shared over workgroups (few rows), need the stream's
+    workspace: a capturing stream without one and the no-allocation variant stage
+    x in every workgroup, to the same bits, and sum K in one workgroup."""
+    K, N = 4096, 9
     announce(f"few columns captured {BLOCK_TYPES[qtype]}")
     t = synth.tensor(qtype, 38, f"cap{qtype}", M, K)
     x = synth.normal(39, "capx", N * K, 1.0).reshape(N, K)
     ref = gpu_matmul(qtype, t.data, x, M, K)
+    bound = np.zeros(ref.shape)
+    if not same_order:  # 32-bit sums in another order
+        w = oracle.dequant(qtype, t.data, M * K).reshape(M, K).astype(np.float64)
+        bound = 16 * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T)
     w_d = hiprt.DeviceBuffer.from_numpy(t.data, pad=256)
     x_d, y_d = hiprt.DeviceBuffer.from_numpy(x), hiprt.DeviceBuffer(4 * N * M)
     stream = hiprt.Stream()
@@ -188,12 +194,12 @@ def test_few_columns_captured_without_a_workspace_and_noalloc(qtype):
         hiprt.synchronize()
         graph.launch()
         stream.synchronize()
-        assert np.array_equal(y_d.to_numpy(np.float32, N * M).reshape(N, M), ref)
+        assert np.all(np.abs(y_d.to_numpy(np.float32, N * M).reshape(N, M) - ref) <= bound)
     y_d.fill(0xFF)
     hiprt.synchronize()
     _native.check(_native.hip_lib().chatnet_matmul_noalloc(qtype, w_d.ptr, x_d.ptr, y_d.ptr, M, K, N, stream.h))
     stream.synchronize()
-    assert np.array_equal(y_d.to_numpy(np.float32, N * M).reshape(N, M), ref)
+    assert np.all(np.abs(y_d.to_numpy(np.float32, N * M).reshape(N, M) - ref) <= bound)
     del graph
     for b in (w_d, x_d, y_d):
         b.free()
