@@ -118,7 +118,7 @@ def digit_bound(qtype, x, w):
 # rounds, ahead of the launch or in the workgroup, and ragged last row tiles.
 @pytest.mark.parametrize("M,K,N", [
     (1, 256, 1), (3, 512, 2), (130, 4096, 7), (37, 11008, 1), (37, 11008, 5), (65, 16384, 3), (8200, 768, 4),
-    (4100, 5120, 2), (5, 2304, 1), (17, 256, 6), (70, 1024, 10), (4200, 512, 8), (130, 2304, 16), (33, 11008, 11),
+    (4100, 5120, 2), (5, 2304, 1), (17, 256, 6), (70, 1024, 10), (4200, 512, 8), (130, 2304, 16), (33, 7936, 11),
     (17000, 256, 3),
 ])
 @pytest.mark.parametrize("qtype", sorted(BLOCK_TYPES))
