@@ -523,10 +523,15 @@ __global__ __launch_bounds__(CN_BLOCK) void gemm_pack_kernel(int qtype, const ui
 // Column tile by batch size and kernel.  One-plane kernel: see pick_gemm
 // (at least 8 chunks of 64 per split).  Span kernel: 32 or 64 columns; a tile grid of more than two workgroups per CU
 // takes the 2-stage ring (44 KB for raw Q4_0 at 64 columns, three workgroups
-// per CU; 56 KB for packed units, two), a smaller one the 3-stage ring (two
-// per CU) and a K split into the largest count that keeps the grid within one
-// round of resident workgroups with at least 8 chunks per split (a grid just
-// over a round would run a second round on a few CUs).
+// per CU; 56 KB for packed units and Q8_0, two), a smaller one the 3-stage ring
+// (two per CU), unless three stages leave one workgroup per CU (packed units,
+// Q8_0, F16: 7B-shaped Q4_K_M 2 layers, 333 tokens 1428 -> 1363 us; F16 200
+// tokens 887 -> 818), and a K split into the largest count that keeps the grid
+// within one round of resident workgroups with at least 8 chunks per split (a
+// grid just over a round would run a second round on a few CUs).  Rows of less
+// than 32 chunks whose grid leaves CUs idle go down to 2 chunks per split
+// (Qwen2-0.5B-shaped Q8_0, 6 layers: 6 tokens at 700 592 -> 488 us, 100 tokens
+// 624 -> 500; at K = 2048 and more 2 to 4 % slower).
 struct GemmShape {
   int tn, splits, stages, mt = 1;
   int sk_wgs = 0, sk_dp = 0;  // one-plane kernel: stream-K workgroups (0: none), of them whole-tile ones
@@ -561,10 +566,12 @@ GemmShape pick_gemm(int M, int N, int K, int num_cus, bool precise, int wf, bool
   if (precise) {
     s.tn = N <= 32 ? 1 : 2;
     const long long tiles = (long long)((M + 127) / 128) * ((N + 32 * s.tn - 1) / (32 * s.tn));
-    s.stages = tiles > 2LL * num_cus ? 2 : 3;
+    s.stages = tiles > 2LL * num_cus || (s.tn == 2 && span_ring_bytes(2, 3, wf) > 80 * 1024) ? 2 : 3;
     const int per_cu = std::max(1, std::min(3, 160 * 1024 / span_ring_bytes(s.tn, s.stages, wf)));
     const long long slots = (long long)per_cu * num_cus;
-    while (s.splits < 16 && tiles * (s.splits + 1) <= slots && nchunks / (s.splits + 1) >= 8) s.splits++;
+    while (s.splits < 16 && tiles * (s.splits + 1) <= slots &&
+           (nchunks / (s.splits + 1) >= 8 || (nchunks < 32 && tiles * (s.splits + 1) <= num_cus && nchunks / (s.splits + 1) >= 2)))
+      s.splits++;
   } else {
     // 32, 64 or 128 columns per workgroup.  Tiles of 64 and 128 columns run
     // the 2-stage ring (44 KB of LDS for raw Q4_0 at 128 columns: three
