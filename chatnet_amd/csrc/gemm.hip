@@ -353,23 +353,6 @@ __global__ __launch_bounds__(CN_BLOCK) void gemm_pack_kernel(int qtype, const ui
         of[j >> 4] = -(dmin * (float)(sb >> 4));
       }
     }
-  } else if (qtype == 11) {  // Q3_K: elements 64(c%4) .. +63 of the super-block
-    const uint8_t* blk = row + (size_t)(c >> 2) * 110;
-    const float d = h2f_at(blk + 108);
-    const uint8_t* s = blk + 96;
-#pragma unroll
-    for (int j = 0; j < 64; j++) {
-      const int e = 64 * (c & 3) + j;
-      const uint32_t q2 = (blk[32 + e / 4] >> (2 * (e % 4))) & 3u, hb = (blk[e / 8] >> (e % 8)) & 1u;
-      put(j, q2 | (hb << 2));
-      if ((j & 15) == 0) {
-        const int i = e >> 4;  // the sub-block's 6-bit scale, stored + 32
-        const int lo = i < 8 ? (s[i] & 15) : (s[i - 8] >> 4);
-        const int v = (lo | (((s[8 + (i & 3)] >> (2 * (i >> 2))) & 3) << 4)) - 32;
-        sc[j >> 4] = d * (float)v;
-        of[j >> 4] = -4.0f * sc[j >> 4];
-      }
-    }
   } else if (qtype == 15) {  // Q8_K: elements 64(c%4) .. +63 of the super-block
     const uint8_t* blk = row + (size_t)(c >> 2) * 292;
     float d;
@@ -495,29 +478,61 @@ __global__ __launch_bounds__(CN_BLOCK) void gemm_pack_kernel(int qtype, const ui
       sc[g] = step;
       of[g] = -128.0f * step;
     }
-  } else {  // Q6_K: elements 64(c%4) .. +63 of the super-block
-    const uint8_t* blk = row + (size_t)(c >> 2) * 210;
-    const float d = h2f_at(blk + 208);
-    const int8_t* scl = reinterpret_cast<const int8_t*>(blk + 192);
-#pragma unroll
-    for (int j = 0; j < 64; j++) {
-      const int e = 64 * (c & 3) + j, hh = e >> 7, e2 = e & 127, qq = e2 >> 5, l = e2 & 31;
-      const uint8_t qlb = blk[64 * hh + l + 32 * (qq & 1)];
-      const uint32_t nib = qq >= 2 ? (uint32_t)(qlb >> 4) : (qlb & 15u);
-      const uint32_t hb = (blk[128 + 32 * hh + l] >> (2 * qq)) & 3u;
-      put(j, nib | (hb << 4));
-      if ((j & 15) == 0) {
-        const float s = d * (float)scl[8 * hh + l / 16 + 2 * qq];
-        sc[j >> 4] = s;
-        of[j >> 4] = -32.0f * s;
-      }
-    }
   }
   uint4* o = reinterpret_cast<uint4*>(dst + ((size_t)r * nchunks + c) * kGemmPackUnit);
 #pragma unroll
   for (int i = 0; i < 4; i++) o[i] = make_uint4(code[4 * i], code[4 * i + 1], code[4 * i + 2], code[4 * i + 3]);
   o[4] = make_uint4(__float_as_uint(sc[0]), __float_as_uint(sc[1]), __float_as_uint(sc[2]), __float_as_uint(sc[3]));
   o[5] = make_uint4(__float_as_uint(of[0]), __float_as_uint(of[1]), __float_as_uint(of[2]), __float_as_uint(of[3]));
+}
+
+// Q6_K and Q3_K, whose 210- and 110-byte super-blocks start on 2-byte boundaries:
+// one thread per 16 weights instead of 64, dword reads instead of bytes (a group
+// of either type takes whole dwords of its quants), four threads writing a unit.
+// Bound by memory (the stored blocks read, 1.5 bytes a weight written) and the
+// scattered reads: 4096 x 4096 Q6_K 16 -> 11.0 us, Q3_K 31 -> 11.7.
+typedef uint32_t pk_u32a2 __attribute__((aligned(2)));
+template <bool Q6>
+__global__ __launch_bounds__(CN_BLOCK) void gemm_pack16_kernel(const uint8_t* __restrict__ w, size_t row_bytes, int M,
+                                                              int nchunks, uint8_t* __restrict__ dst) {
+  const long long t = (long long)blockIdx.x * CN_BLOCK + threadIdx.x;
+  const long long unit = t >> 2;
+  if (unit >= (long long)M * nchunks) return;
+  const int g = (int)(t & 3);
+  const int r = (int)(unit / nchunks), c = (int)(unit % nchunks);
+  const int G = 4 * (c & 3) + g;  // group of the super-block
+  uint32_t code[4];
+  float sc, of;
+  if constexpr (Q6) {
+    const uint8_t* blk = w + (size_t)r * row_bytes + (size_t)(c >> 2) * 210;
+    const int h = G >> 3, qq = (G >> 1) & 3, lb = G & 1;
+    const uint8_t* ql = blk + 64 * h + 32 * (qq & 1) + 16 * lb;
+    const uint8_t* qh = blk + 128 + 32 * h + 16 * lb;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint32_t l = *reinterpret_cast<const pk_u32a2*>(ql + 4 * k), u = *reinterpret_cast<const pk_u32a2*>(qh + 4 * k);
+      code[k] = ((l >> (4 * (qq >> 1))) & 0x0F0F0F0Fu) | (((u >> (2 * qq)) & 0x03030303u) << 4);
+    }
+    sc = h2f_at(blk + 208) * (float)(int8_t)blk[192 + G];
+    of = -32.0f * sc;
+  } else {
+    const uint8_t* blk = w + (size_t)r * row_bytes + (size_t)(c >> 2) * 110;
+    const uint32_t q = *reinterpret_cast<const pk_u32a2*>(blk + 32 + 4 * G);
+    const uint32_t hm = *reinterpret_cast<const uint16_t*>(blk + 2 * G);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {  // element 4k + i: bits 2i of byte k, mask bit 4k + i
+      const uint32_t b = (q >> (8 * k)) & 0xFFu;
+      code[k] = ((b | (b << 6) | (b << 12) | (b << 18)) & 0x03030303u) | (spread4(hm >> (4 * k)) << 2);
+    }
+    const uint8_t* s = blk + 96;
+    const int lo = G < 8 ? (s[G] & 15) : (s[G - 8] >> 4);
+    sc = h2f_at(blk + 108) * (float)((lo | (((s[8 + (G & 3)] >> (2 * (G >> 2))) & 3) << 4)) - 32);
+    of = -4.0f * sc;
+  }
+  uint8_t* o = dst + (size_t)unit * kGemmPackUnit;
+  *reinterpret_cast<uint4*>(o + 16 * g) = make_uint4(code[0], code[1], code[2], code[3]);
+  *reinterpret_cast<float*>(o + 64 + 4 * g) = sc;
+  *reinterpret_cast<float*>(o + 80 + 4 * g) = of;
 }
 
 // Column tile by batch size and kernel.  One-plane kernel: see pick_gemm
@@ -698,6 +713,15 @@ hipError_t gemm_pack_launch(int qtype, const void* w, int M, int K, void* dst, h
   const long long n = (long long)M * (K / 64);
   const long long blocks = (n + CN_BLOCK - 1) / CN_BLOCK;
   if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
+  if (qtype == 11 || qtype == 14) {
+    if (4 * blocks > 0x7FFFFFFF) return hipErrorInvalidValue;  // 2^39 weights and more
+    const dim3 grid((unsigned)((4 * n + CN_BLOCK - 1) / CN_BLOCK));
+    const uint8_t* wb = static_cast<const uint8_t*>(w);
+    uint8_t* to = static_cast<uint8_t*>(dst);
+    if (qtype == 14) hipLaunchKernelGGL((gemm_pack16_kernel<true>), grid, dim3(CN_BLOCK), 0, st, wb, row_bytes, M, K / 64, to);
+    else hipLaunchKernelGGL((gemm_pack16_kernel<false>), grid, dim3(CN_BLOCK), 0, st, wb, row_bytes, M, K / 64, to);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL(gemm_pack_kernel, dim3((unsigned)blocks), dim3(CN_BLOCK), 0, st, qtype,
                      static_cast<const uint8_t*>(w), row_bytes, (size_t)M * row_bytes, M, K / 64,
                      static_cast<uint8_t*>(dst));
