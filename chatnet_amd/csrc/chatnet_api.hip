@@ -938,18 +938,22 @@ int ensure_span_buffers(chatnet_model* m) {
   return CHATNET_OK;
 }
 
+// At least `need` bytes at sp_part, which the stream's kernels use in turn.
+int span_part(chatnet_model* m, size_t need) {
+  if (need <= m->sp_part_bytes) return CHATNET_OK;
+  HIP_TRY(hipStreamSynchronize(m->stream));
+  if (m->sp_part) (void)hipFree(m->sp_part);
+  m->sp_part = nullptr;
+  m->sp_part_bytes = 0;
+  if (hipMalloc(&m->sp_part, need) != hipSuccess)
+    return fail(CHATNET_ERR_OUT_OF_MEMORY, "hipMalloc of %zu bytes failed", need);
+  m->sp_part_bytes = need;
+  return CHATNET_OK;
+}
+
 int span_gemm(chatnet_model* m, GemmArgs& g, int* splits_left = nullptr) {
   g.precise = 1;
-  const size_t need = gemm_workspace_bytes(g.M, g.N, g.K, m->num_cus, true, g.packed);
-  if (need > m->sp_part_bytes) {
-    HIP_TRY(hipStreamSynchronize(m->stream));
-    if (m->sp_part) (void)hipFree(m->sp_part);
-    m->sp_part = nullptr;
-    m->sp_part_bytes = 0;
-    if (hipMalloc(&m->sp_part, need) != hipSuccess)
-      return fail(CHATNET_ERR_OUT_OF_MEMORY, "hipMalloc of %zu bytes failed", need);
-    m->sp_part_bytes = need;
-  }
+  if (int rc = span_part(m, gemm_workspace_bytes(g.M, g.N, g.K, m->num_cus, true, g.packed))) return rc;
   g.part = m->sp_part;
   HIP_TRY(gemm_launch(g, m->num_cus, m->stream, splits_left));
   return CHATNET_OK;
@@ -1046,6 +1050,10 @@ int run_span(chatnet_model* m, const int32_t* tokens, int n, int position, const
       at.kv_dim = kvd;
       at.kv_f16 = r.kv_f16;
       at.scale = 1.0f / sqrtf((float)c.head_dim);  // LlamaModel.cs:248
+      // the QKV GEMM's partials at sp_part are read by now (RoPE, in stream order)
+      at.splits = attn_prefill_splits(cn, p0, c.n_heads, at.kv_mul, m->num_cus);
+      if ((rc = span_part(m, attn_prefill_workspace(cn, c.n_heads, c.head_dim, at.splits)))) return rc;
+      at.part = m->sp_part;
       HIP_TRY(attn_prefill_launch(at, st));
 
       GemmArgs o;

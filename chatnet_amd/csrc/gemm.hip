@@ -490,7 +490,7 @@ __global__ __launch_bounds__(CN_BLOCK) void gemm_pack_kernel(int qtype, const ui
 // one thread per 16 weights instead of 64, dword reads instead of bytes (a group
 // of either type takes whole dwords of its quants), four threads writing a unit.
 // Bound by memory (the stored blocks read, 1.5 bytes a weight written) and the
-// scattered reads: 4096 x 4096 Q6_K 16 -> 11.0 us, Q3_K 31 -> 11.7.
+// scattered reads: 4096 x 4096 Q6_K 16.1 -> 11.0 us, Q3_K 30.7 -> 11.7.
 typedef uint32_t pk_u32a2 __attribute__((aligned(2)));
 template <bool Q6>
 __global__ __launch_bounds__(CN_BLOCK) void gemm_pack16_kernel(const uint8_t* __restrict__ w, size_t row_bytes, int M,

@@ -233,8 +233,12 @@ struct PrefillAttnArgs {
   int ldo;
   int n, p0, n_heads, kv_mul, head_dim, kv_dim, kv_f16;
   float scale;
+  int splits;        // key shares per row block (attn_prefill_splits); 0 or 1: none
+  float* part;       // attn_prefill_workspace bytes when splits > 1
 };
 bool attn_prefill_supports(int head_dim, int kv_mul);
+int attn_prefill_splits(int n, int p0, int n_heads, int kv_mul, int num_cus);
+size_t attn_prefill_workspace(int n, int n_heads, int head_dim, int splits);
 hipError_t attn_prefill_launch(const PrefillAttnArgs& a, hipStream_t st);
 
 // Embedding row gather (LlamaModel.LoadEmbedding, LlamaModel.cs:365-394) of

@@ -153,6 +153,9 @@ __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
 // Each group's next chunk is loaded into registers while it computes the
 // current one.  The output is written for the O-projection span GEMM: fp16
 // hi + lo planes (out, out_lo) in the cn_span_pos order.
+// A span too short to fill the chip shares its keys out over gridDim.z
+// workgroups per row block (attn_prefill_splits): each leaves its unnormalised
+// fp32 output and softmax state, and attn_prefill_merge_kernel adds them.
 constexpr int kSpanThreads = 512;
 
 template <int HD>
@@ -187,7 +190,10 @@ __global__ __launch_bounds__(kSpanThreads) void attn_prefill_kernel(PrefillAttnA
   const bool real = r < QB * a.kv_mul && t < a.n;
   const int qpos = real ? a.p0 + t : -1;  // -1: padding row, every key masked
   const int t_last = min(a.n, t0 + QB) - 1;
-  const int kend = a.p0 + t_last + 1;        // keys [0, kend)
+  // this workgroup's keys: rounds [r0, r1) of two chunks, below the last token
+  const int rounds = (a.p0 + t_last + 2 * KB) / (2 * KB);
+  const int r0 = (int)blockIdx.z * rounds / (int)gridDim.z, r1 = ((int)blockIdx.z + 1) * rounds / (int)gridDim.z;
+  const int kend = min(a.p0 + t_last + 1, r1 * 2 * KB);
 
   // q of row r: k-step s, lane group g holds dims 32s + 8g .. +7
   float4 qr[NS][2];
@@ -272,8 +278,7 @@ __global__ __launch_bounds__(kSpanThreads) void attn_prefill_kernel(PrefillAttnA
 
   // group grp walks chunks grp, grp + 2, ...; both groups run the same number
   // of rounds, a group past the last chunk only keeps the barriers
-  const int rounds = (kend + 2 * KB - 1) / (2 * KB);
-  int c0 = grp * KB;
+  int c0 = (2 * r0 + grp) * KB;
   if (c0 < kend) load_chunk(c0);
 
   // q * scale * log2(e) as bf16 hi/lo B operands
@@ -288,7 +293,7 @@ __global__ __launch_bounds__(kSpanThreads) void attn_prefill_kernel(PrefillAttnA
     ql[s] = as_bf16x8(make_uint4(l0.x, l0.y, l1.x, l1.y));
   }
 
-  for (int it = 0; it < rounds; it++, c0 += 2 * KB) {
+  for (int it = r0; it < r1; it++, c0 += 2 * KB) {
     __syncthreads();  // the previous chunk's LDS readers are done
     if (c0 < kend) store_chunk();
     __syncthreads();
@@ -384,10 +389,28 @@ __global__ __launch_bounds__(kSpanThreads) void attn_prefill_kernel(PrefillAttnA
   }
   __syncthreads();
   if (grp == 1 || !real) return;
-  // group 0 scored key 0 of every real row, so m is finite; a row group 1 never
-  // scored has m1 = -inf and weight 0
   const float m1 = xm[r], l1 = xm[64 + r];
   const float m = fmaxf(m_run, m1);
+  if (gridDim.z > 1) {
+    // a row with no key in this share keeps m = -inf and sums of 0
+    const float mu = m == -INFINITY ? 0.f : m;
+    const float a0 = __builtin_amdgcn_exp2f(m_run - mu), a1 = __builtin_amdgcn_exp2f(m1 - mu);
+    const size_t slot = ((size_t)blockIdx.z * a.n + t) * a.n_heads + hh;
+#pragma unroll
+    for (int i = 0; i < NT; i++) {
+      const float4 o1 = *reinterpret_cast<const float4*>(&xs[4 * ((4 * i + g) * 64 + r)]);
+      *reinterpret_cast<float4*>(a.part + slot * HD + 16 * i + 4 * g) =
+          make_float4(o[i][0] * a0 + o1.x * a1, o[i][1] * a0 + o1.y * a1, o[i][2] * a0 + o1.z * a1,
+                      o[i][3] * a0 + o1.w * a1);
+    }
+    if (g == 0) {
+      float2* ml = reinterpret_cast<float2*>(a.part + (size_t)gridDim.z * a.n * a.n_heads * HD);
+      ml[slot] = make_float2(m, l * a0 + l1 * a1);
+    }
+    return;
+  }
+  // group 0 scored key 0 of every real row, so m is finite; a row group 1 never
+  // scored has m1 = -inf and weight 0
   const float a0 = __builtin_amdgcn_exp2f(m_run - m), a1 = __builtin_amdgcn_exp2f(m1 - m);
   const float inv = 1.0f / (l * a0 + l1 * a1);
   const float s0 = a0 * inv, s1 = a1 * inv;
@@ -406,6 +429,48 @@ __global__ __launch_bounds__(kSpanThreads) void attn_prefill_kernel(PrefillAttnA
   }
 }
 
+// Adds the shares of one (token, head) row: a thread per four dims, every share's
+// load in flight at once.  Some share scored key 0, so m is finite.
+template <int SPL>
+__global__ __launch_bounds__(CN_BLOCK) void attn_prefill_merge_kernel(PrefillAttnArgs a) {
+  const int q4 = a.head_dim / 4;
+  const int i = blockIdx.x * CN_BLOCK + threadIdx.x;
+  if (i >= a.n * a.n_heads * q4) return;
+  const int slot = i / q4, d = i % q4, rows = a.n * a.n_heads;
+  const float2* ml = reinterpret_cast<const float2*>(a.part + (size_t)a.splits * rows * a.head_dim);
+  float2 st[SPL];
+  float4 v[SPL];
+#pragma unroll
+  for (int s = 0; s < SPL; s++) {
+    const int k = min(s, a.splits - 1);
+    st[s] = ml[(size_t)k * rows + slot];
+    v[s] = *reinterpret_cast<const float4*>(a.part + ((size_t)k * rows + slot) * a.head_dim + 4 * d);
+  }
+  float m = st[0].x;
+#pragma unroll
+  for (int s = 1; s < SPL; s++) m = fmaxf(m, st[s].x);
+  float l = 0.f;
+  float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int s = 0; s < SPL; s++) {
+    if (s >= a.splits) break;
+    const float w = __builtin_amdgcn_exp2f(st[s].x - m);
+    l += st[s].y * w;
+    o.x += v[s].x * w;
+    o.y += v[s].y * w;
+    o.z += v[s].z * w;
+    o.w += v[s].w * w;
+  }
+  const float inv = 1.0f / l;
+  const int t = slot / a.n_heads, e = (slot % a.n_heads) * a.head_dim + 4 * d;
+  uint2 hi, lo;
+  cn_split_f16x2(o.x * inv, o.y * inv, hi.x, lo.x);
+  cn_split_f16x2(o.z * inv, o.w * inv, hi.y, lo.y);
+  const size_t at = (size_t)t * a.ldo + cn_span_pos(e);
+  *reinterpret_cast<uint2*>(a.out + at) = hi;
+  *reinterpret_cast<uint2*>(a.out_lo + at) = lo;
+}
+
 template <int HD>
 size_t prefill_lds_bytes() {
   // the end-of-kernel exchange (64 rows of HD floats, then m and l) fits in
@@ -417,11 +482,18 @@ size_t prefill_lds_bytes() {
 template <int HD, bool F16>
 hipError_t attn_prefill_t(const PrefillAttnArgs& a, hipStream_t st) {
   const int QB = 64 / a.kv_mul;
-  const dim3 grid(a.n_heads / a.kv_mul, (a.n + QB - 1) / QB);
+  const dim3 grid(a.n_heads / a.kv_mul, (a.n + QB - 1) / QB, a.splits > 1 ? a.splits : 1);
   static std::atomic<uint64_t> lds_done{0};  // > 64 KB of dynamic LDS must be allowed (once per device)
   const hipError_t e = allow_full_lds(reinterpret_cast<const void*>(&attn_prefill_kernel<HD, F16>), lds_done);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((attn_prefill_kernel<HD, F16>), grid, dim3(kSpanThreads), prefill_lds_bytes<HD>(), st, a);
+  if (a.splits > 1) {
+    const dim3 mg((a.n * a.n_heads * (HD / 4) + CN_BLOCK - 1) / CN_BLOCK);
+    if (a.splits <= 2) hipLaunchKernelGGL(attn_prefill_merge_kernel<2>, mg, dim3(CN_BLOCK), 0, st, a);
+    else if (a.splits <= 4) hipLaunchKernelGGL(attn_prefill_merge_kernel<4>, mg, dim3(CN_BLOCK), 0, st, a);
+    else if (a.splits <= 8) hipLaunchKernelGGL(attn_prefill_merge_kernel<8>, mg, dim3(CN_BLOCK), 0, st, a);
+    else hipLaunchKernelGGL(attn_prefill_merge_kernel<16>, mg, dim3(CN_BLOCK), 0, st, a);
+  }
   return hipGetLastError();
 }
 
@@ -431,8 +503,32 @@ bool attn_prefill_supports(int head_dim, int kv_mul) {
   return (head_dim == 64 || head_dim == 128) && kv_mul >= 1 && kv_mul <= 64;
 }
 
+// Key shares per row block: as many as fill the chip once (a workgroup takes most
+// of a CU's LDS), where that saves at least kSplitSaves rounds of 128 keys, each a
+// chain of loads, stores and products of 2.5 (head_dim 64) to 5 us (128); the merge
+// is a launch more.  Per layer: 14/2 heads of 64, 6 tokens at 700, -8 us, at 330
+// -1 us; 32 heads of 128, 100 tokens at 1000, -23 us, 10 at 330 -6 us; saving a
+// single round (10 tokens at 200) changed nothing.
+constexpr int kSplitMax = 16, kSplitSaves = 2;
+
+int attn_prefill_splits(int n, int p0, int n_heads, int kv_mul, int num_cus) {
+  const int qb = 64 / kv_mul;
+  const long long wgs = (long long)(n_heads / kv_mul) * ((n + qb - 1) / qb);
+  const int rounds = (p0 + n + 127) / 128;
+  int s = (int)(num_cus / wgs);
+  if (s > rounds) s = rounds;
+  if (s > kSplitMax) s = kSplitMax;
+  return s > 1 && rounds - (rounds + s - 1) / s >= kSplitSaves ? s : 1;
+}
+
+size_t attn_prefill_workspace(int n, int n_heads, int head_dim, int splits) {
+  return splits > 1 ? sizeof(float) * splits * n * n_heads * (head_dim + 2) : 0;
+}
+
 hipError_t attn_prefill_launch(const PrefillAttnArgs& a, hipStream_t st) {
-  if (!attn_prefill_supports(a.head_dim, a.kv_mul) || a.n <= 0 || !a.out || !a.out_lo) return hipErrorInvalidValue;
+  if (!attn_prefill_supports(a.head_dim, a.kv_mul) || a.n <= 0 || !a.out || !a.out_lo || a.splits > kSplitMax ||
+      (a.splits > 1 && !a.part))
+    return hipErrorInvalidValue;
   if (a.head_dim == 64) return a.kv_f16 ? attn_prefill_t<64, true>(a, st) : attn_prefill_t<64, false>(a, st);
   return a.kv_f16 ? attn_prefill_t<128, true>(a, st) : attn_prefill_t<128, false>(a, st);
 }

@@ -223,3 +223,12 @@ def test_stored_block_gemm_edges(qtype, M, K, N):
     r = x.astype(np.float64) @ w.T
     scale = np.abs(x).astype(np.float64) @ np.abs(w).T
     assert np.all(np.abs(y - r) <= 2.0 ** -10 * 1.01 * scale), float(np.max(np.abs(y - r) / scale))
+
+
+# Q6_K and Q3_K re-encoded by a thread per 16 weights: one super-block, odd counts
+# of them (rows starting on 2-byte boundaries), and a last workgroup partly filled.
+@pytest.mark.parametrize("M,K,N", [(1, 256, 17), (3, 768, 17), (65, 2304, 40), (300, 4096, 129)])
+@pytest.mark.parametrize("qtype", [11, 14])
+def test_repacked_gemm_edges(qtype, M, K, N):
+    """The bound of the stored blocks' test: one fp16 rounding of each operand."""
+    test_stored_block_gemm_edges(qtype, M, K, N)

@@ -6,9 +6,9 @@ import os
 import numpy as np
 import pytest
 
-from chatnet_amd import QWEN2_0_5B, HipLlamaModel, synth
+from chatnet_amd import QWEN2_0_5B, HipLlamaModel, _native, synth
 from gpu_util import announce
-from test_gpu_model import SPAN_SMALL, span_case
+from test_gpu_model import LOGIT_TOL, SPAN_SMALL, span_case
 
 pytestmark = pytest.mark.gpu
 
@@ -61,3 +61,21 @@ def test_short_span_after_a_long_one_uses_the_packs():
     h = per_token(SPAN_SMALL, ck, toks[12:], 12, toks[:12])
     assert not np.array_equal(g, h)
     assert float(np.max(np.abs(g - h))) <= 1e-3
+
+
+# Keys shared out over workgroups: both head sizes and cache types, groups of 1, 2
+# and 7 heads, two shares to sixteen, a share past a token's own keys.
+@pytest.mark.parametrize("heads,kv,hd,f16", [(14, 2, 64, False), (4, 4, 64, True), (4, 2, 128, False), (2, 1, 128, True)])
+@pytest.mark.parametrize("pos,n", [(377, 8), (250, 10), (630, 100), (2030, 12)])
+def test_spans_deep_in_the_context_share_their_keys(heads, kv, hd, f16, pos, n):
+    announce(f"shared keys: {heads}/{kv} heads of {hd}, f16 cache {f16}, {n} tokens at {pos}")
+    cfg = SPAN_SMALL.replace(n_layers=2, dim=heads * hd, hidden_dim=512, n_heads=heads, n_kv_heads=kv, head_dim=hd,
+                             vocab_size=512, context_length=2048, kv_dtype=_native.KV_F16 if f16 else _native.KV_F32)
+    ck = synth.llama_checkpoint(cfg, seed=65, mix="q4_0")
+    toks = synth.tokens(65, "prompt", pos + n, cfg.vocab_size)
+    with HipLlamaModel(cfg, ck) as m:
+        m.forward(toks[:pos], 0)
+        g = m.forward(toks[pos:], pos).copy()
+    h = per_token(cfg, ck, toks[pos:], pos, toks[:pos])
+    # each schedule's bound against the oracle, twice that for an fp16 cache
+    assert float(np.max(np.abs(g - h))) <= 2 * LOGIT_TOL * (2 if f16 else 1)
