@@ -261,9 +261,10 @@ int bucket_cap(const chatnet_model* m, int seq) {
   return cap < m->cfg.context_length ? cap : m->cfg.context_length;
 }
 
-// Decode-attention launch for sequence lengths up to cap: chunks of at least
-// one round of the workgroup's wave steps, as many as attn_max_splits allows;
-// chunk * splits >= cap, and every chunk starts below cap.  Where two chunks
+// Decode-attention launch for sequence lengths up to cap: a split's share of the
+// positions (chunk) is at least one round of the workgroup's wave steps, as many
+// splits as attn_max_splits allows; chunk * splits >= cap, and every chunk starts
+// below cap (the launch deals them out in blocks of a round).  Where two chunks
 // would do, one chunk of two rounds is used instead: its second round costs
 // less than the merge launch a second chunk needs.
 struct AttnPlan {
@@ -271,7 +272,7 @@ struct AttnPlan {
 };
 AttnPlan attn_plan(const chatnet_model* m, int cap) {
   const int smax = m->attn_splits_max;
-  const int round = attn_decode_round(m->cfg.head_dim, m->cfg.n_heads / m->cfg.n_kv_heads);
+  const int round = attn_decode_round(m->cfg.head_dim, m->cfg.n_heads / m->cfg.n_kv_heads, 256);
   int chunk = (cap + smax - 1) / smax;
   if (chunk < round) chunk = round;
   const int splits = (cap + chunk - 1) / chunk;
@@ -732,11 +733,14 @@ int launch_token(chatnet_model* m, bool lm_head, int cap, bool decode = false) {
     at.scale = 1.0f / sqrtf((float)c.head_dim);  // LlamaModel.cs:248
     const AttnPlan plan = attn_plan(m, cap);
     at.splits = plan.splits;
-    at.chunk = plan.chunk;
     at.part_o = m->attn_part_o;
     at.part_ml = m->attn_part_ml;
     at.stop = a.stop;
     at.hsplit = attn_decode_hsplit(c.n_kv_heads, at.kv_mul, plan.splits, m->num_cus);
+    const int kvm = at.kv_mul / at.hsplit;
+    at.threads = attn_decode_threads(c.n_kv_heads, c.head_dim, kvm, at.hsplit, plan.splits, plan.chunk, at.kv_f16);
+    const int round = attn_decode_round(c.head_dim, kvm, at.threads);
+    at.chunk = plan.chunk < round ? plan.chunk : round;
     HIP_TRY(attn_decode_launch(at, st));
 
     GemvArgs o = base_args(m, decode);
@@ -751,7 +755,7 @@ int launch_token(chatnet_model* m, bool lm_head, int cap, bool decode = false) {
       o.part_o = m->attn_part_o;
       o.part_ml = m->attn_part_ml;
       o.msplits = plan.splits;
-      o.mchunk = plan.chunk;
+      o.mchunk = at.chunk;
     }
     HIP_TRY(gemv_launch(gemv_qt(L.wo), fold ? GEMV_EPI_ADD_MERGE : GEMV_EPI_ADD, o, m->num_cus, st));
 

@@ -106,25 +106,29 @@ __device__ __forceinline__ void attn_put(const AttnArgs& a, int h, int split, in
 // LlamaModel.cs:241-346): for query head h with kvh = h / kv_mul (:265),
 //   s[p] = (q_h . K[p][kvh]) * scale  for p <= pos,  w = softmax(s) (TensorMath.cs:177-241),
 //   out_h = sum_p w[p] V[p][kvh].
-// Grid = n_kv_heads x a.splits; workgroup (kvh, c) takes the positions
-// [c*chunk, (c+1)*chunk) below seq = pos+1.  Its four waves split the kv_mul
-// query heads WH ways (WH = 4, 2 or 1 as kv_mul allows, HPW heads per wave
-// and pass) and the positions WP = 4/WH ways.  A wave is 4 rows of 16 lanes:
+// Grid = n_kv_heads x a.splits; workgroup (kvh, c) takes every a.splits-th block
+// of chunk positions below seq = pos+1, from block c on: whatever seq is within
+// the launch's bucket, the splits' shares differ by at most a block.  (One
+// contiguous share each left some idle in the lower half of a bucket: 32 heads of
+// 128, fp16 cache, at 1100 of 2048 13.6 -> 9.9 us, 14/2 heads of 64 16.2 -> 11.4,
+// at 700 of 1024 10.4 -> 8.6.)  Its four or eight waves split the kv_mul query
+// heads WH ways (WH = 4, 2 or 1 as kv_mul allows, HPW heads per wave and pass)
+// and the positions WP ways.  A wave is 4 rows of 16 lanes:
 // row r holds one position, lane i of the row the head elements
 // [i*EPL, (i+1)*EPL) (EPL = HD/16).  A wave step covers SP = 4*PG consecutive
 // positions for the wave's heads: 16-lane dot products reduced with DPP inside
 // the row, one max over the step's positions per head, one rescale of the
 // running (max, sum, o) per head (online softmax; sums and o stay per row
 // until the end, then add across rows).  The first step's K/V loads depend
-// only on the chunk, so they are in flight before the position arrives.  With
+// only on the split, so they are in flight before the position arrives.  With
 // WP = 1 each wave holds its heads' complete result for the chunk; otherwise
 // the WP waves of a head fold through LDS.  A launch of one chunk writes the
 // output itself; more chunks (at most kFoldMaxSplits) leave partials that the
 // O projection combines as it stages its x (GEMV_EPI_ADD_MERGE).
-template <int HD, bool F16, int HPW, int PG>
-__global__ __launch_bounds__(CN_BLOCK) void attn_decode_kernel(AttnArgs a) {
+template <int HD, bool F16, int HPW, int PG, int BS>
+__global__ __launch_bounds__(BS) void attn_decode_kernel(AttnArgs a) {
   constexpr int EPL = HD / 16;   // head elements per lane
-  constexpr int NW = CN_BLOCK / CN_WAVE;
+  constexpr int NW = BS / CN_WAVE;
   constexpr int SP = 4 * PG;     // positions per wave step
   // workgroup (kv head, head group, split): a.hsplit workgroups share a kv
   // head, each taking kvm = kv_mul / hsplit of its query heads
@@ -138,8 +142,9 @@ __global__ __launch_bounds__(CN_BLOCK) void attn_decode_kernel(AttnArgs a) {
   const int WP = NW / WH;
   const int hw = wave % WH, pw = wave / WH;
   const int h0 = kvh * a.kv_mul + hs * kvm;
-  const int p0 = split * a.chunk;
-  const int pcap = min(p0 + a.chunk, a.ctx);  // this split's positions, all inside the cache (p0 < ctx)
+  const int p0 = split * a.chunk, stride = a.splits * a.chunk;
+  // a split that is one short block ends with it
+  const int pcap = a.chunk < WP * SP ? min(p0 + a.chunk, a.ctx) : a.ctx;  // p0 < ctx
   const size_t koff = (size_t)kvh * HD + col * EPL;
   __shared__ float so[NW * HPW * HD];
   __shared__ float sml[NW * HPW * 2];
@@ -163,12 +168,12 @@ __global__ __launch_bounds__(CN_BLOCK) void attn_decode_kernel(AttnArgs a) {
 #pragma unroll
       for (int e = 0; e < EPL; e++) o[j][e] = 0.f;
     }
-    // K/V rows of a wave step starting at position pb: rows past the chunk
-    // re-read its last position (masked below), so every load is issued
-    auto load_step = [&](int pb, float (&kr)[PG][EPL], float (&vr)[PG][EPL]) {
+    // K/V rows of a wave step starting at position pb: rows past end re-read
+    // the last position below it (masked below), so every load is issued
+    auto load_step = [&](int pb, int end, float (&kr)[PG][EPL], float (&vr)[PG][EPL]) {
 #pragma unroll
       for (int g = 0; g < PG; g++) {
-        const int p = min(pb + 4 * g + row, pcap - 1);
+        const int p = min(pb + 4 * g + row, end - 1);
         kv_load_n<F16, EPL>(a.kc, (size_t)p * a.kv_dim + koff, kr[g]);
         kv_load_n<F16, EPL>(a.vc, (size_t)p * a.kv_dim + koff, vr[g]);
       }
@@ -176,7 +181,7 @@ __global__ __launch_bounds__(CN_BLOCK) void attn_decode_kernel(AttnArgs a) {
     // first step: positions below pcap regardless of seq
     int pb = p0 + pw * SP;
     float kr[PG][EPL], vr[PG][EPL];
-    load_step(pb, kr, vr);
+    load_step(pb, pcap, kr, vr);
     if (first_pass) {
       if (__builtin_amdgcn_readfirstlane(stop_v)) return;  // uniform: before any barrier
       first_pass = false;
@@ -186,7 +191,7 @@ __global__ __launch_bounds__(CN_BLOCK) void attn_decode_kernel(AttnArgs a) {
     while (pb < p1) {  // uniform across the wave
       // the next step's loads go out before this step is computed
       float kn[PG][EPL], vn[PG][EPL];
-      load_step(pb + WP * SP, kn, vn);
+      load_step(pb + stride, p1, kn, vn);
       float sc[PG][HPW];
 #pragma unroll
       for (int g = 0; g < PG; g++) {
@@ -230,7 +235,7 @@ __global__ __launch_bounds__(CN_BLOCK) void attn_decode_kernel(AttnArgs a) {
         }
         m[j] = mn;
       }
-      pb += WP * SP;
+      pb += stride;
 #pragma unroll
       for (int g = 0; g < PG; g++)
 #pragma unroll
@@ -277,19 +282,19 @@ __global__ __launch_bounds__(CN_BLOCK) void attn_decode_kernel(AttnArgs a) {
       }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < WH * HPW * HD; i += CN_BLOCK) {
+    for (int i = threadIdx.x; i < WH * HPW * HD; i += BS) {
       const int d = i % HD, jj = (i / HD) % HPW, hh = i / (HD * HPW);  // head jg + hh*HPW + jj
       if (jg + hh * HPW + jj >= kvm) continue;
       float M = -INFINITY;
       for (int w = 0; w < WP; w++) {
         const int sl = (w * WH + hh) * HPW + jj;
-        if (sml[2 * sl + 1] > 0.f) M = fmaxf(M, sml[2 * sl]);
+        if (sml[2 * sl + 1] != 0.f) M = fmaxf(M, sml[2 * sl]);
       }
       float L = 0.f, acc = 0.f;
       for (int w = 0; w < WP; w++) {
         const int sl = (w * WH + hh) * HPW + jj;
         const float lw = sml[2 * sl + 1];
-        if (lw > 0.f) {
+        if (lw != 0.f) {  // NaN sums included
           const float f = expf(sml[2 * sl] - M);
           L += lw * f;
           acc += so[sl * HD + d] * f;
@@ -419,9 +424,12 @@ constexpr int attn_pg(int hd, int hpw) {
 
 template <int HD, bool F16, int HPW>
 void attn_launch_k(const AttnArgs& a, hipStream_t st) {
-  const int n_kv = a.n_heads / a.kv_mul;
-  hipLaunchKernelGGL((attn_decode_kernel<HD, F16, HPW, attn_pg(HD, HPW)>), dim3(n_kv * a.hsplit * a.splits),
-                     dim3(CN_BLOCK), 0, st, a);
+  const dim3 grid(a.n_heads / a.kv_mul * a.hsplit * a.splits);
+  constexpr int PG = attn_pg(HD, HPW);
+  if (HPW <= 2 && a.threads == 512)
+    hipLaunchKernelGGL((attn_decode_kernel<HD, F16, HPW, PG, HPW <= 2 ? 512 : CN_BLOCK>), grid, dim3(512), 0, st, a);
+  else
+    hipLaunchKernelGGL((attn_decode_kernel<HD, F16, HPW, PG, CN_BLOCK>), grid, dim3(CN_BLOCK), 0, st, a);
 }
 
 template <int HD, bool F16>
@@ -450,16 +458,31 @@ int attn_decode_hsplit(int n_kv_heads, int kv_mul, int splits, int num_cus) {
   return hs;
 }
 
-int attn_decode_round(int head_dim, int kv_mul) {
+// Threads of a workgroup.  A chunk of many rounds is a chain of memory latencies
+// where the grid keeps little in flight, and eight waves halve it; else the fold of
+// eight waves costs 0.5 to 1 us more.  At 256 and 512 threads, us: 32 heads of 128,
+// fp16 cache (2 MB in flight) 13.9 and 11.0 at position 1900 (16 rounds), 9.6 and
+// 8.8 at 1000 (8); fp32 cache (4 MB) 16.0 and 17.0 at 1900; 2 kv heads of 64, fp32
+// 13.6 and 12.1 at 1500 (8 rounds), 8.6 and 8.8 at 700 (4).
+int attn_decode_threads(int n_kv_heads, int head_dim, int kvm, int hsplit, int splits, int chunk, bool f16) {
+  const int round = attn_decode_round(head_dim, kvm, CN_BLOCK);
+  const long long flight = 2ll * n_kv_heads * hsplit * splits * round * head_dim * (f16 ? 2 : 4);
+  return attn_hpw(kvm) <= 2 && chunk >= 8 * round && flight <= (2 << 20) ? 512 : CN_BLOCK;
+}
+
+int attn_decode_round(int head_dim, int kv_mul, int threads) {
+  const int nw = threads / CN_WAVE;
   const int wh = kv_mul >= 4 ? 4 : (kv_mul >= 2 ? 2 : 1);
   int hpw = attn_hpw(kv_mul);
   if (head_dim > 128 && hpw > 2) hpw = 2;
-  return (4 / wh) * 4 * attn_pg(head_dim, hpw);
+  return (nw / wh) * 4 * attn_pg(head_dim, hpw);
 }
 
 hipError_t attn_decode_launch(const AttnArgs& a, hipStream_t st) {
   if (a.splits < 1 || a.splits > kFoldMaxSplits || a.chunk < 1 || a.head_dim % 16 != 0 || a.hsplit < 1 ||
-      a.kv_mul % a.hsplit != 0)
+      a.kv_mul % a.hsplit != 0 || (a.threads != CN_BLOCK && a.threads != 512) ||
+      (a.threads == 512 && attn_hpw(a.kv_mul / a.hsplit) > 2) ||
+      a.chunk > attn_decode_round(a.head_dim, a.kv_mul / a.hsplit, a.threads))
     return hipErrorInvalidValue;
   if (a.head_dim == 64) return a.kv_f16 ? attn_launch_t<64, true>(a, st) : attn_launch_t<64, false>(a, st);
   if (a.head_dim == 128) return a.kv_f16 ? attn_launch_t<128, true>(a, st) : attn_launch_t<128, false>(a, st);

@@ -1,13 +1,15 @@
-// gemm.hip — quantized-weight GEMM on the matrix cores of gfx950 (N >= 8).
+// gemm.hip — quantized-weight GEMM on the matrix cores of gfx950: x conversion,
+// packing, K-split reduce, tile choice and the dispatch over weight formats (the
+// kernels are gemm_tile.h, instantiated in gemm_*.hip).
 //
 // y[n][m] = sum_k W[m][k] * x[n][k] for a batch of N inputs: the batched form
 // of TensorMath.MatVecMulQ4_0 (src/ChatNet.Core/Tensors/TensorMath.cs:548-578)
-// that chatnet_matmul with N >= 8 and a multi-token LlamaModel.Forward span
+// that chatnet_matmul with many columns and a multi-token LlamaModel.Forward span
 // (LlamaModel.cs:93-238) need.
 //
-// W is read either as raw Q4_0 blocks or as packed units (gemm_pack_kernel:
-// the other block types re-encoded as u8 codes with an fp32 scale and offset
-// per 16 weights); x arrives from the producer kernel in the cn_span_pos
+// W is read as stored (gemm_stored_format) or as packed units (gemm_pack_kernel:
+// Q3_K, Q6_K, Q8_K and seven IQ types re-encoded as u8 codes with an fp32 scale
+// and offset per 16 weights); x arrives from the producer kernel in the cn_span_pos
 // order, either as one fp16 plane scaled per column by a power of two
 // (to_f16_scaled_kernel, chatnet_matmul) or, for the exact-weight variant the
 // spans run, as fp16 hi + lo planes (conversion, RMSNorm, attention or the

@@ -1,5 +1,5 @@
 // gemv_float.hip — GEMV for F32 and F16 weight matrices, and for packed units
-// (the block types without a digit-path kernel), on gfx950.
+// (Q8_K and the IQ types without a digit-path kernel), on gfx950.
 //
 // Replaces the two float branches of LlamaModel.MatVecMulByType
 // (src/ChatNet.Core/Models/Llama/LlamaModel.cs:470-567):

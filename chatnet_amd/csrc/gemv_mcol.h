@@ -13,7 +13,9 @@
 // What bounds it: the four conversions, multiplies and adds per block and tile
 // (12 to 16 VALU instructions for 16 rows x 32 weights x 5 columns); dot4 on
 // packed digits took 21 per 16 weights and column, one launch per column the
-// weight stream N times.  Measured (N columns, us): see launch_mcol.
+// weight stream N times.  Against the MFMA GEMM and the column by column GEMV:
+// Q4_K 11008 x 4096 at 5 columns 31 -> 18 us, at 16 68 -> 26, Q8_0 4864 x 896 at 5
+// 18.9 -> 5.2.
 #pragma once
 #include "gemv_quant.h"
 

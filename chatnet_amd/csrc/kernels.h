@@ -56,7 +56,7 @@ struct GemvArgs {
   int kv_f16;
   const float* bias;  // QKV: optional per-row bias added before RoPE, indexed by virtual row
   // ADD_MERGE: attention partials [heads][msplits][head_dim] and (max, sum)
-  // pairs, chunks of mchunk positions of which those below *pos + 1 count
+  // pairs, of the splits whose first block of mchunk positions starts below *pos + 1
   const float* part_o;
   const float* part_ml;
   int msplits, mchunk;
@@ -260,15 +260,18 @@ struct AttnArgs {
   float scale;
   float* part_o;      // split partials: [n_heads][splits][head_dim]
   float* part_ml;     // [n_heads][splits][2] (max, sum)
-  int splits;         // position chunks of the launch (<= kFoldMaxSplits), one workgroup per kv head each
-  int chunk;          // positions per chunk: chunk c covers [c*chunk, (c+1)*chunk) below pos+1
+  int splits;         // position splits of the launch (<= kFoldMaxSplits), one workgroup per kv head each
+  int chunk;          // positions per block, at most a round: split c covers blocks c, c + splits, ... below
+                      // pos+1; blocks shorter than a round are one per split (chunk * splits > pos)
   int hsplit;         // workgroups per kv head, each taking kv_mul / hsplit query heads
+  int threads;        // attn_decode_threads
   const int* stop;    // decode loops: return at once while *stop is set (nullptr: never)
 };
 hipError_t attn_decode_launch(const AttnArgs& a, hipStream_t st);
 // Positions one decode-attention workgroup covers per round of wave steps
-// (kv_mul: the query heads the workgroup takes).
-int attn_decode_round(int head_dim, int kv_mul);
+// (kv_mul: the query heads the workgroup takes), and its threads.
+int attn_decode_round(int head_dim, int kv_mul, int threads);
+int attn_decode_threads(int n_kv_heads, int head_dim, int kvm, int hsplit, int splits, int chunk, bool f16);
 // Workgroups per kv head for a launch of `splits` position chunks.
 int attn_decode_hsplit(int n_kv_heads, int kv_mul, int splits, int num_cus);
 

@@ -64,7 +64,8 @@ def test_short_span_after_a_long_one_uses_the_packs():
 
 
 # Keys shared out over workgroups: both head sizes and cache types, groups of 1, 2
-# and 7 heads, two shares to sixteen, a share past a token's own keys.
+# and 7 heads, two shares to sixteen, a share past a token's own keys.  The token by
+# token side deals its blocks out to 4- and 8-wave workgroups (8 for all but 4/4).
 @pytest.mark.parametrize("heads,kv,hd,f16", [(14, 2, 64, False), (4, 4, 64, True), (4, 2, 128, False), (2, 1, 128, True)])
 @pytest.mark.parametrize("pos,n", [(377, 8), (250, 10), (630, 100), (2030, 12)])
 def test_spans_deep_in_the_context_share_their_keys(heads, kv, hd, f16, pos, n):
