@@ -282,9 +282,10 @@ CHATNET_API int chatnet_matmul(uint32_t ggml_type, const void* w_dev, const floa
 /* chatnet_matmul without any allocation, for callers that cannot allocate
  * device memory: code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc.  No counterpart in the reference.  Same arguments,
- * kernels and results as chatnet_matmul for Q4_0 and for the types read
- * only as packed units (Q4_1, Q5_0, Q5_1, Q2_K, Q8_K and the IQ types,
- * whose packed copy of W, M*(K/64)*96 bytes, goes into the scratch), except
+ * kernels and results as chatnet_matmul for Q4_0, Q4_1, Q5_0, Q5_1, Q2_K,
+ * Q8_K and the IQ types (Q8_K's and the re-encoded IQ types' copy of W,
+ * M*(K/64)*96 bytes, goes into the scratch; the size limit below counts such a
+ * copy for each of these types but Q4_0), except
  * that it runs no stream-K launch: where chatnet_matmul shares tiles it runs
  * the plain tile grid, the same product summed in another order.  Q8_0,
  * Q3_K, Q4_K, Q5_K and Q6_K run the fused GEMV once per column on their stored
