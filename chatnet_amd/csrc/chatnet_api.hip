@@ -824,16 +824,11 @@ int ensure_out_tokens(chatnet_model* m, int cap) {
   return CHATNET_OK;
 }
 
-// Spans of at least this many tokens run as one batch on the MFMA GEMM.  Below
-// kSpanAny tokens only models of the types whose GEMV takes x to 19 bits, in
-// no less precision batched (the logits' error against float64 halves, 8e-6 to
-// 4e-6; the other types' token by token schedule is more precise), and only
-// while no matrix has to be packed for it.  Measured, token by token and
-// batched: Qwen2-0.5B-shaped Q8_0, 6 layers, 6 tokens at position 700 1237 and
-// 488 us; TinyLlama-shaped Q4_0, 4 layers, 2 tokens 253 and 288; 7B-shaped
-// Q4_0, 2 layers, 2 tokens 217 and 264, 3 tokens 288 and 264.
-constexpr int kSpanMin = 3;
-constexpr int kSpanAny = 8;
+// Spans of at least this many tokens run as one batch on the MFMA GEMM.  Shorter
+// ones run token by token: there the activations, q, k, v and the attention
+// weights are fp32 (or digits scaled to their own group), which keeps what the
+// batch's fp16 and bf16 planes would round and any magnitude fp32 holds.
+constexpr int kSpanMin = 8;
 constexpr int kSpanCap = 512;
 
 // The seven projection matrices of a layer.
@@ -889,17 +884,6 @@ SpanPlan span_plan(chatnet_model* m, int n) {
     }
   }
   for (int g = 0; g < 4; g++) p.fmt[g] = fmt[g] >= 0 ? fmt[g] : GEMM_W_PACKED;
-  if (n < kSpanAny) {
-    for (Layer& L : m->layers) {
-      const LayerMats lm = layer_mats(L);
-      for (int i = 0; i < 7; i++) {
-        const uint32_t ty = lm.t[i]->type;
-        const bool digits19 = ty == CHATNET_GGML_Q4_0 || ty == CHATNET_GGML_Q8_0 || ty == CHATNET_GGML_Q3_K ||
-                              ty == CHATNET_GGML_Q4_K || ty == CHATNET_GGML_Q5_K || ty == CHATNET_GGML_Q6_K;
-        if (!digits19 || (p.fmt[group_of[i]] == GEMM_W_PACKED && !lm.t[i]->pk)) return p;
-      }
-    }
-  }
   p.ok = true;
   return p;
 }

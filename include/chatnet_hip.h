@@ -153,8 +153,7 @@ CHATNET_API int chatnet_upload_tensor(chatnet_model* m, const char* name, uint32
  * (IModel.cs:18, LlamaModel.cs:93-238).  Processes tokens[0..n) at positions
  * position..position+n-1, writing their K/V into the cache; logits of the last
  * token stay on the device and are copied to `logits_host` (vocab_size
- * floats) when it is non-NULL.  Spans of 8 or more tokens (3 or more when every
- * matrix is Q4_0, Q8_0 or Q3_K .. Q6_K and none has yet to be packed) run as batches of
+ * floats) when it is non-NULL.  Spans of 8 or more tokens run as batches of
  * up to 512 tokens when head_dim is 64 or 128 and n_heads / n_kv_heads is at
  * most 64: MFMA GEMMs on fp16 operands (activations as fp16 hi + lo planes)
  * and causal attention over the cache.  Each GEMM of a layer (q|k|v, o,
