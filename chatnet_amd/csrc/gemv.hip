@@ -21,7 +21,9 @@
 // nibbles on v_dot8_i32_i4) or base-256 digits (Q8_0, Q5_K, Q6_K, long Q4_K
 // rows: weight bytes on v_dot4_i32_i8).  Each group's dot is exact in int32;
 // the per-group scales, offsets (q-8, q-32, dmin*m) and 2^-e are applied in
-// fp32 once per group.  Partial row sums are reduced across the LPR lanes with
+// fp32 once per group.  Q4_1, Q5_0, Q5_1, Q2_K, IQ4_NL and IQ4_XS keep x in fp32
+// (products code * x on fmaf, the group's scale and offset after 16 of them).
+// Partial row sums are reduced across the LPR lanes with
 // cross-lane shuffles.
 //
 // Epilogues (fused into the lane that finishes a row pair):

@@ -18,9 +18,7 @@ constexpr int QT_Q4_0 = 2, QT_Q4_1 = 3, QT_Q5_0 = 6, QT_Q5_1 = 7, QT_Q8_0 = 8, Q
 constexpr int QT_Q6_KQ = 114;
 
 template <int QT> struct QTraits;
-// Types whose products used fp32 x (packed units) before they were read from
-// their stored blocks: x keeps 23 to 24 bits of its 16-element group's maximum
-// (digitize16<.., FINE>), and a non-finite x gives NaN as it did there.
+// Types multiplied with x in fp32 (stage_fp32, dot_unit_fp32).
 template <int QT>
 constexpr bool fine_type() {
   return QT == QT_Q4_1 || QT == QT_Q5_0 || QT == QT_Q5_1 || QT == QT_IQ4_NL || QT == QT_Q2_K || QT == QT_IQ4_XS;
@@ -370,27 +368,14 @@ __device__ __forceinline__ void stage_load16(const float* __restrict__ x, const 
 // TR (Q3_K): record dword w, byte b holds element 4b + w of the group instead
 // of element 4w + b, the order in which Q3_K's 2-bit fields come out of a qs
 // dword (shift by 2w, mask 0x03030303).
-// FINE: X takes the digits' whole range (|X| <= 0x7F7F7F: 23 - e, or 22 - e when
-// the maximum's fraction is above 0.996) instead of 2^18; returns false when an
-// element is not finite.
-template <bool TR, bool FINE>
-__device__ __forceinline__ bool digitize16(const float (&v)[16], uint32_t* rec, bool on) {
+template <bool TR>
+__device__ __forceinline__ void digitize16(const float (&v)[16], uint32_t* rec, bool on) {
   float m = 0.f;
-  bool finite = true;
-  if constexpr (FINE) {
-    uint32_t mb = 0;  // magnitudes as bits: infinities and NaN compare above every number
 #pragma unroll
-    for (int i = 0; i < 16; i++) mb = max(mb, __float_as_uint(v[i]) & 0x7FFFFFFFu);
-    finite = mb < 0x7F800000u;
-    m = __uint_as_float(mb);
-  } else {
-#pragma unroll
-    for (int i = 0; i < 16; i++) m = fmaxf(m, fabsf(v[i]));
-  }
+  for (int i = 0; i < 16; i++) m = fmaxf(m, fabsf(v[i]));
   int e = 0;
-  const float f = frexpf(m, &e);
-  const int bits = FINE ? (f > 0.996f ? 22 : 23) : 18;
-  const int sc = m > 0.f ? bits - e : 0;
+  (void)frexpf(m, &e);
+  const int sc = m > 0.f ? 18 - e : 0;
   // U = X + 0x808080: its bytes 0..2 are D_d + 128
   uint32_t U[16];
   int sum = 0;
@@ -421,13 +406,11 @@ __device__ __forceinline__ bool digitize16(const float (&v)[16], uint32_t* rec, 
     rec[12] = (uint32_t)sum;
     rec[13] = (uint32_t)sc;
   }
-  return finite;
 }
 
 // Writes the base-256 digit records of x * norm_w (x alone without NORM) and,
-// as stage_digitize, leaves each wave's share of sum x^2 in red[wave] (NaN with
-// FINE when the wave met a non-finite element).
-template <int MAXT, bool NORM, int BS, bool TR = false, bool FINE = false>
+// as stage_digitize, leaves each wave's share of sum x^2 in red[wave].
+template <int MAXT, bool NORM, int BS, bool TR = false>
 __device__ __forceinline__ void stage_digitize16(const XStage16<MAXT, NORM>& st, int K, uint32_t* xd, float* red) {
   const int ngroups = K >> 4;
   float ss = 0.f;
@@ -445,8 +428,53 @@ __device__ __forceinline__ void stage_digitize16(const XStage16<MAXT, NORM>& st,
 #pragma unroll
       for (int i = 0; i < 16; i++) v[i] = v[i] * st.g[j][i];
     }
-    const bool finite = digitize16<TR, FINE>(v, xd + (t >> 3) * XD6_UNIT_DW + 16 * (t & 7), on);
-    if (FINE && on && !finite) ss = NAN;
+    digitize16<TR>(v, xd + (t >> 3) * XD6_UNIT_DW + 16 * (t & 7), on);
+  }
+  ss = cn_wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+}
+
+// ---------------------------------------------------------------------------
+// x of the fine types in fp32.  LDS record of a lane unit (64 or 128 elements):
+// its elements, then the sum of every 16 (the types with an offset).  The
+// records' strides put the 16-byte reads of 16 neighbouring lanes on different
+// banks.
+// ---------------------------------------------------------------------------
+template <int QT>
+constexpr int xf_unit_dw() { return QTraits<QT>::UNIT == 64 ? 68 : 140; }
+
+// The 16 elements v of group t into the records.
+template <int QT>
+__device__ __forceinline__ void store_group_fp32(const float (&v)[16], int t, float* xr) {
+  constexpr int G = QTraits<QT>::UNIT / 16;  // groups per unit
+  float* rec = xr + (t / G) * xf_unit_dw<QT>();
+  const int g = t % G;
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    *reinterpret_cast<float4*>(rec + 16 * g + 4 * k) = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+  float s[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) s[i] = v[i] + v[i + 8];
+  rec[16 * G + g] = ((s[0] + s[4]) + (s[1] + s[5])) + ((s[2] + s[6]) + (s[3] + s[7]));
+}
+
+// Writes the records of x * norm_w (x alone without NORM) and, as
+// stage_digitize, leaves each wave's share of sum x^2 in red[wave].
+template <int QT, int MAXT, bool NORM, int BS>
+__device__ __forceinline__ void stage_fp32(const XStage16<MAXT, NORM>& st, int K, float* xr, float* red) {
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < MAXT; j++) {
+    const int t = threadIdx.x + BS * j;
+    const bool on = t < (K >> 4);  // threads past the last group hold a re-read group
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      v[i] = st.x[j][i];
+      ss += on ? v[i] * v[i] : 0.f;
+      if constexpr (NORM) v[i] *= st.g[j][i];
+    }
+    if (on) store_group_fp32<QT>(v, t, xr);
   }
   ss = cn_wave_sum(ss);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
@@ -1008,9 +1036,8 @@ __device__ __forceinline__ void dot_unit_k45_dig8(const uint32_t (*w)[QTraits<QT
 
 // ---------------------------------------------------------------------------
 // One 16-element group of a unit of the fine types:
-//   sum_k w_k x_k = 2^-e (a T + b SX),  T = sum q X, SX = sum X
-// with the group's 16 codes as signed bytes q[0..3] in the digit records'
-// element order and
+//   sum_k w_k x_k = a sum_k q_k x_k + b sum_k x_k
+// with the group's 16 codes as signed bytes q[0..3] in element order and
 //   Q5_0 a = d (codes q5 - 16);  Q4_1, Q5_1 a = d, b = m;  IQ4_NL a = d and
 //   IQ4_XS a = d sc (codes from the table);  Q2_K a = d sc, b = -dmin m.
 // ---------------------------------------------------------------------------
@@ -1067,35 +1094,44 @@ __device__ __forceinline__ void unit_group(const uint32_t* w, int h, int g, uint
   }
 }
 
+template <int B>
+__device__ __forceinline__ float cn_sbyte(uint32_t v) {
+  return (float)(int8_t)(v >> (8 * B));
+}
+
+// sum_k q_k x_k of a group in fp32.
+__device__ __forceinline__ float group_dot(const uint32_t (&q)[4], const float4 (&x)[4]) {
+  float s = 0.f;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    s = fmaf(cn_sbyte<0>(q[k]), x[k].x, s);
+    s = fmaf(cn_sbyte<1>(q[k]), x[k].y, s);
+    s = fmaf(cn_sbyte<2>(q[k]), x[k].z, s);
+    s = fmaf(cn_sbyte<3>(q[k]), x[k].w, s);
+  }
+  return s;
+}
+
 // A unit of RPW rows (half h of its super-block, where the type has halves)
-// against its digit record.  The digit sums meet as T2 2^16 + (T1 2^8 + T0), the
-// bracket exact below 2^24 for codes to 31 and rounded once for IQ4's.
+// against its record.  32 conversions and fmas a group, 16 digit dots and their
+// joining before, both hidden behind the weight stream: Q5_0 4096 x 11008 10.7
+// (x to 23 bits of its group) -> 10.9 us, 11008 x 4096 9.6 -> 9.5, IQ4_XS 4096 x
+// 4096 4.9 -> 5.1; error against float64 1.7e-7 -> 1.1e-7.
 template <int QT, int RPW>
-__device__ __forceinline__ void dot_unit_groups(const uint32_t (*w)[QTraits<QT>::NDW], const uint32_t* xd, int h,
-                                                float* acc) {
+__device__ __forceinline__ void dot_unit_fp32(const uint32_t (*w)[QTraits<QT>::NDW], const float* rec, int h, float* acc) {
+  constexpr int G = QTraits<QT>::UNIT / 16;
 #pragma unroll
-  for (int g = 0; g < QTraits<QT>::UNIT / 16; g++) {
-    const uint32_t* rec = xd + 16 * g;
-    uint32_t D[3][4];
+  for (int g = 0; g < G; g++) {
+    float4 x[4];
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
-      const uint4 t = *reinterpret_cast<const uint4*>(rec + 4 * d);
-      D[d][0] = t.x; D[d][1] = t.y; D[d][2] = t.z; D[d][3] = t.w;
-    }
-    const uint2 se = *reinterpret_cast<const uint2*>(rec + 12);  // sum X, e
+    for (int k = 0; k < 4; k++) x[k] = *reinterpret_cast<const float4*>(rec + 16 * g + 4 * k);
 #pragma unroll
     for (int i = 0; i < RPW; i++) {
       uint32_t q[4];
       float a, b;
       unit_group<QT>(w[i], h, g, q, a, b);
-      int t[3] = {0, 0, 0};
-#pragma unroll
-      for (int d = 0; d < 3; d++)
-#pragma unroll
-        for (int k = 0; k < 4; k++) t[d] = __builtin_amdgcn_sdot4((int)q[k], (int)D[d][k], t[d], false);
-      float v = fmaf((float)t[2], 65536.0f, (float)(t[1] * 256 + t[0])) * a;
-      if constexpr (group_min<QT>()) v = fmaf(b, (float)(int)se.x, v);
-      acc[i] += ldexpf(v, -(int)se.y);
+      if constexpr (group_min<QT>()) acc[i] = fmaf(b, rec[16 * G + g], acc[i]);
+      acc[i] = fmaf(a, group_dot(q, x), acc[i]);
     }
   }
 }
@@ -1160,7 +1196,7 @@ __global__ __launch_bounds__(BS) void gemv_kernel(GemvArgs a) {
   constexpr int NS = merge_slots(EPI);
   const int stop_v = cn_load_late(stop_flag(a));
   const int pos_v = (EPI == GEMV_EPI_QKV || MERGE) ? cn_load_late(a.pos) : 0;
-  constexpr bool kDig8 =
+  constexpr bool kGroups =  // staged by 16-element groups: fp32 records or base-256 digits
       fine_type<QT>() || QT == QT_Q8_0 || QT == QT_Q3_K || QT == QT_Q6_K || QT == QT_Q6_KQ || QT == QT_Q5_K || (QT == QT_Q4_K && LPR > 32);
   MergeSrc ms{};
   if constexpr (MERGE) {
@@ -1168,8 +1204,8 @@ __global__ __launch_bounds__(BS) void gemv_kernel(GemvArgs a) {
     ms.ml = a.part_ml;
     ms.hd = a.head_dim;
     ms.splits = a.msplits;
-    // the base-256 staging merges while it loads: it needs the position now
-    if constexpr (kDig8)
+    // staging by groups merges while it loads: it needs the position now
+    if constexpr (kGroups)
       ms.s_eff = min(a.msplits, (__builtin_amdgcn_readfirstlane(pos_v) + a.mchunk) / a.mchunk);
   }
 
@@ -1182,7 +1218,7 @@ __global__ __launch_bounds__(BS) void gemv_kernel(GemvArgs a) {
     constexpr bool NORM = EPI == GEMV_EPI_QKV || EPI == GEMV_EPI_SWIGLU || EPI == GEMV_EPI_LOGITS;
     uint32_t* xd = reinterpret_cast<uint32_t*>(smem);
     float* xred;
-    if constexpr (kDig8) {
+    if constexpr (kGroups) {
       // groups per thread: K <= UNIT * LPR * NU, so K/16 <= (UNIT/16) * LPR * NU groups over BS threads
       constexpr int MAXT = ((UNIT / 16) * LPR * NU + BS - 1) / BS;
       XStage16<MAXT, NORM> st;
@@ -1195,8 +1231,9 @@ __global__ __launch_bounds__(BS) void gemv_kernel(GemvArgs a) {
         issue_loads<QT, RPW, LPR, NU, EPI>(a, it, sub, li, nunits, bpr, w);
         load_residual<EPI, RPW, NR>(a, it * RW + sub * RPW, li, 0, res);
       }
-      xred = reinterpret_cast<float*>(smem) + (size_t)((K + 127) >> 7) * XD6_UNIT_DW;
-      stage_digitize16<MAXT, NORM, BS, QT == QT_Q3_K, fine_type<QT>()>(st, K, xd, xred);
+      xred = smem + (fine_type<QT>() ? nunits * xf_unit_dw<QT>() : ((K + 127) >> 7) * XD6_UNIT_DW);
+      if constexpr (fine_type<QT>()) stage_fp32<QT, MAXT, NORM, BS>(st, K, smem, xred);
+      else stage_digitize16<MAXT, NORM, BS, QT == QT_Q3_K>(st, K, xd, xred);
       if constexpr (kLate) {
         issue_loads<QT, RPW, LPR, NU, EPI>(a, it, sub, li, nunits, bpr, w);
         load_residual<EPI, RPW, NR>(a, it * RW + sub * RPW, li, 0, res);
@@ -1223,8 +1260,7 @@ __global__ __launch_bounds__(BS) void gemv_kernel(GemvArgs a) {
     float ss = 0.f;
 #pragma unroll
     for (int v = 0; v < NWV; v++) ss += xred[v];
-    float rms = NORM ? 1.0f / sqrtf(ss / (float)K + a.eps) : 1.0f;
-    if (fine_type<QT>() && !(ss == ss)) rms = ss;  // a non-finite x
+    const float rms = NORM ? 1.0f / sqrtf(ss / (float)K + a.eps) : 1.0f;
     if (__builtin_amdgcn_readfirstlane(stop_v)) return;
     const int pos = __builtin_amdgcn_readfirstlane(pos_v);
     while (it < n_iters) {
@@ -1242,15 +1278,12 @@ __global__ __launch_bounds__(BS) void gemv_kernel(GemvArgs a) {
 #pragma unroll
             for (int k = 0; k < T::NDW; k++) wu[i][k] = w[i][n][k];
           if constexpr (QT == QT_Q4_0) dot_unit_q4_0_dig<RPW>(wu, xd + u * XD_UNIT_DW, acc);
-          else if constexpr (fine_type<QT>()) {
-            const uint32_t* rec = UNIT == 64 ? xd + (u >> 1) * XD6_UNIT_DW + 64 * (u & 1) : xd + u * XD6_UNIT_DW;
-            dot_unit_groups<QT, RPW>(wu, rec, u & 1, acc);
-          }
+          else if constexpr (fine_type<QT>()) dot_unit_fp32<QT, RPW>(wu, smem + u * xf_unit_dw<QT>(), u & 1, acc);
           else if constexpr (QT == QT_Q8_0) dot_unit_q8_0_dig8<RPW>(wu, xd + (u >> 1) * XD6_UNIT_DW + 64 * (u & 1), acc);
           else if constexpr (QT == QT_Q6_K) dot_unit_q6_k_dig<RPW>(wu, xd + u * XD6_UNIT_DW, acc);
           else if constexpr (QT == QT_Q6_KQ) dot_unit_q6_kq_dig<RPW>(wu, xd + (u >> 1) * XD6_UNIT_DW, u & 1, acc);
           else if constexpr (QT == QT_Q3_K) dot_unit_q3_k_dig<RPW>(wu, xd + u * XD6_UNIT_DW, u & 1, acc);
-          else if constexpr (kDig8) dot_unit_k45_dig8<QT, RPW>(wu, xd + u * XD6_UNIT_DW, u & 1, acc);
+          else if constexpr (kGroups) dot_unit_k45_dig8<QT, RPW>(wu, xd + u * XD6_UNIT_DW, u & 1, acc);
           else dot_unit_q4_k_dig<RPW>(wu, xd + 2 * u * XD_UNIT_DW, u & 1, acc);
         }
       }
@@ -1279,7 +1312,8 @@ size_t gemv_smem_bytes(int K) {
   using T = QTraits<QT>;
   const int nunits = K / T::UNIT;
   // digit records (base 16: Q4_0, Q4_K up to 32 half super-blocks per row;
-  // base 256 per 128 elements otherwise) + one float per wave
+  // base 256 per 128 elements otherwise) or fp32 records + one float per wave
+  if constexpr (fine_type<QT>()) return ((size_t)nunits * xf_unit_dw<QT>() + 16) * sizeof(float);
   if (QT == QT_Q4_0 || (QT == QT_Q4_K && nunits <= 32)) return ((size_t)(K >> 6) * XD_UNIT_DW + 16) * sizeof(uint32_t);
   return ((size_t)((K + 127) >> 7) * XD6_UNIT_DW + 16) * sizeof(uint32_t);
 }

@@ -101,7 +101,7 @@ def test_f16_columns_captured_without_a_workspace_and_noalloc(M, K, N):
 
 BLOCK_TYPES = {3: "q4_1", 6: "q5_0", 7: "q5_1", 8: "q8_0", 10: "q2_k", 11: "q3_k", 12: "q4_k", 13: "q5_k", 14: "q6_k",
                20: "iq4_nl", 23: "iq4_xs"}
-FINE_TYPES = (3, 6, 7, 10, 20, 23)  # x to 23 bits of its 16-element group, 19 for the others
+FINE_TYPES = (3, 6, 7, 10, 20, 23)  # one column: x in fp32, 19 bits of its group for the others
 
 
 def digit_bound(qtype, x, w):
@@ -171,6 +171,53 @@ def test_non_finite_x_and_wide_magnitudes(qtype, N):
         y = gpu_matmul(qtype, t.data, x, M, K)
         r = x.astype(np.float64) @ w.T
         assert max(normwise(y[n], r[n]) for n in range(N)) <= 2e-6
+
+
+def smallest_weights_at(qtype, t, M, K, k):
+    """The tensor's bytes with the weight of column k (5, 15 or 10 in its block: a
+    low nibble, or Q2_K's lowest field) of every row at its type's smallest
+    magnitude: 0, or the table's 1 (IQ4)."""
+    n, size = (256, {10: 84, 23: 136}[qtype]) if qtype in (10, 23) else (32, {3: 20, 6: 22, 7: 24, 20: 18}[qtype])
+    b = t.data.reshape(M, K // n, size).copy()
+    j, blk = k % n, b[:, k // n]
+    if qtype == 3:
+        b[:, :, 2:4] = 0
+        blk[:, 4 + j] &= 0xF0
+    elif qtype == 6:
+        blk[:, 6 + j] &= 0xF0
+        blk[:, 2 + j // 8] |= 1 << (j % 8)
+    elif qtype == 7:
+        b[:, :, 2:4] = 0
+        blk[:, 8 + j] &= 0xF0
+        blk[:, 4 + j // 8] &= 0xFF ^ (1 << (j % 8))
+    elif qtype == 20:
+        blk[:, 2 + j] = (blk[:, 2 + j] & 0xF0) | 8
+    elif qtype == 10:
+        b[:, :, 82:84] = 0
+        blk[:, 16 + j] &= 0xFC
+    else:
+        blk[:, 8 + j] = (blk[:, 8 + j] & 0xF0) | 8
+    return b.reshape(-1)
+
+
+# K = 512 and 3 or 4 units per lane's worth of K; the outlier in a group's first
+# and last quarter.
+@pytest.mark.parametrize("M,K,k", [(40, 512, 5), (33, 768, 256 + 15), (9, 11008, 10 + 512), (6, 16384, 5)])
+@pytest.mark.parametrize("N", [1])
+@pytest.mark.parametrize("qtype", FINE_TYPES)
+def test_fp32_types_keep_the_neighbours_of_a_large_element(qtype, M, K, k, N):
+    """x is fp32 for these types: an element of 1e5 under a zero (or the smallest)
+    weight leaves its neighbours' bits alone.  Bound: 32 roundings of 2^-24 of
+    sum |w x| (a group's 16 products, the groups of a lane, the lanes)."""
+    announce(f"large element {BLOCK_TYPES[qtype]} M={M} K={K} N={N}")
+    data = smallest_weights_at(qtype, synth.tensor(qtype, 51, f"out{qtype}-{M}x{K}", M, K), M, K, k)
+    x = synth.normal(52, f"outx{N}x{K}", N * K, 1.0).reshape(N, K)
+    x[:, k] = 1e5
+    w = oracle.dequant(qtype, data, M * K).reshape(M, K).astype(np.float64)
+    y = gpu_matmul(qtype, data, x, M, K)
+    bound = 32 * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T)
+    err = np.abs(y - x.astype(np.float64) @ w.T)
+    assert np.all(err <= bound), float(np.max(err / bound))
 
 
 @pytest.mark.parametrize("M,same_order", [(2100, True), (96, False)])
