@@ -22,7 +22,7 @@ HIP_SOURCES = ["gemv_q4_0.hip", "gemm.hip", "gemv_q8_0.hip", "gemv_q6_k.hip", "g
                "gemm_q4_0.hip", "gemm_packed.hip", "gemm_q8_0.hip", "gemm_q4_k.hip", "gemm_q5_k.hip", "gemm_q2_k.hip",
                "gemm_q5_0.hip", "gemm_q4_1.hip", "gemm_q5_1.hip", "gemm_iq4_nl.hip", "gemm_iq4_xs.hip", "gemm_f16.hip",
                "gemm_f32.hip", "chatnet_api.hip", "gemv.hip", "gemv_float.hip", "prefill.hip", "decode_ops.hip", "sample.hip"]
-HIP_HEADERS = ["device_common.h", "gemv_common.h", "gemm_tile.h", "gemv_mcol.h", "gemv_quant.h", "kernels.h"]
+HIP_HEADERS = ["device_common.h", "gemv_common.h", "gemm_tile.h", "gemv_mcol.h", "gemv_quant.h", "gemv_xcols.h", "kernels.h"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

@@ -1295,7 +1295,7 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
   }
   if (N >= 2 && !pack && gemv_qcols_supports((int)type) && !(N <= (type == CHATNET_GGML_Q3_K ? 3 : 2) && (long long)M * K >= kTwoGemvs)) {
     // x staged once in the stream's workspace where there is one and it pays
-    const size_t need = noalloc ? 0 : gemv_qcols_workspace(M, K, N, cus);
+    const size_t need = noalloc ? 0 : gemv_qcols_workspace((int)type, M, K, N, cus);
     char* ws = nullptr;
     if (need) {
       lk.lock();

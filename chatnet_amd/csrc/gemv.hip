@@ -31,6 +31,7 @@
 //   ADD     y[r] += dot                          (O / down + residual, TensorMath.Add :712-733)
 //   QKV     RoPE on q/k pairs + K/V cache write  (TensorMath.ApplyRoPE :408-458, LlamaModel.cs:146-153)
 //   SWIGLU  h[r] = silu(gate[r]) * up[r]         (TensorMath.SiluElementwiseMul :253-286)
+#include <algorithm>
 #include <cstring>
 
 #include "kernels.h"
@@ -121,7 +122,24 @@ static bool mcol_ahead(int M, int K, int n, int num_cus) {
   return (double)n * K * (wgs < 1 ? 1 : wgs > 2 ? 2 : wgs) >= 22000.0;
 }
 
-size_t gemv_qcols_workspace(int M, int K, int N, int num_cus) {
+// Types whose x stays in fp32 up to kFp32Cols columns, as the single column's does
+// (a power of two shared by 32 elements costs a large element's neighbours their
+// low bits).  More columns ran the GEMM on x rounded to fp16, which the digits of
+// the matrix-core product are finer than.
+static bool fp32_cols(int qtype, int N) {
+  constexpr int kFp32Cols = 7;
+  return N <= kFp32Cols && (qtype == 3 || qtype == 6 || qtype == 7 || qtype == 10 || qtype == 20 || qtype == 23);
+}
+
+// Columns of one fp32 launch: the records (gemv_quant.h, 68 floats per 64 elements
+// or 140 per 128) of as many as 150 KB of LDS hold, two at K = 16384, 7 at 4096.
+static int fp32_cols_max(int qtype, int K) {
+  const size_t col = (qtype == 10 || qtype == 23 ? (size_t)K / 128 * 140 : (size_t)K / 64 * 68) * sizeof(float);
+  return (int)std::min<size_t>(8, 150 * 1024 / col);
+}
+
+size_t gemv_qcols_workspace(int qtype, int M, int K, int N, int num_cus) {
+  if (fp32_cols(qtype, N)) return 0;
   const int n = N < kColsMax ? N : kColsMax;
   const int shares = mcol_shares(M, K, num_cus);
   if (shares > 1) return (size_t)shares * n * M * sizeof(float);
@@ -134,9 +152,9 @@ hipError_t gemv_qcols_launch(int qtype, const void* w, const float* x, float* y,
                              void* ws, hipStream_t st) {
   if (!gemv_qcols_supports(qtype) || !gemv_supports(qtype, K) || M <= 0 || N < 1 || !w || !x || !y)
     return hipErrorInvalidValue;
-  const int g = kColsMax;
-  McolPlan plan{nullptr, 1, nullptr};
-  if (ws) {
+  McolPlan plan{fp32_cols(qtype, N), nullptr, 1, nullptr};
+  const int g = plan.fp32 ? fp32_cols_max(qtype, K) : kColsMax;
+  if (ws && !plan.fp32) {
     plan.shares = mcol_shares(M, K, num_cus);
     if (plan.shares > 1) plan.part = static_cast<float*>(ws);
     else plan.pre = static_cast<char*>(ws);

@@ -1,11 +1,12 @@
 // gemv_iq4_nl.hip — the IQ4_NL instances of the quantized GEMV (gemv_quant.h) and of
-// the few-column product (gemv_mcol.h).
+// the few-column products (gemv_xcols.h, gemv_mcol.h).
 #include "gemv_mcol.h"
+#include "gemv_xcols.h"
 
 hipError_t gemv_iq4_nl_launch(int epi, const GemvArgs& a, int num_cus, hipStream_t st) {
   return launch_type<QT_IQ4_NL>(epi, a, num_cus, st);
 }
 
 hipError_t gemv_iq4_nl_cols_launch(const GemvArgs& a, int ncols, int num_cus, const McolPlan& p, hipStream_t st) {
-  return launch_mcol<QT_IQ4_NL>(a, ncols, num_cus, p, st);
+  return p.fp32 ? launch_xcols<QT_IQ4_NL>(a, ncols, num_cus, st) : launch_mcol<QT_IQ4_NL>(a, ncols, num_cus, p, st);
 }

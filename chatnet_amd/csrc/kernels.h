@@ -88,19 +88,21 @@ int gemv_float_cols_max(int K);
 hipError_t gemv_float_cols_launch(int qtype, const void* w, const float* x, float* y, int M, int K, int N, int num_cus,
                                   hipStream_t st);
 // Block types other than Q4_0 read from their stored blocks against N columns of
-// x on the int8 matrix cores (gemv_mcol.h), up to 16 per launch, x to 23 bits of
-// each 32-element block's largest.
+// x: Q4_1, Q5_0, Q5_1, Q2_K, IQ4_NL and IQ4_XS up to 7 columns in fp32
+// (gemv_xcols.h), else on the int8 matrix cores (gemv_mcol.h), up to 16 per launch,
+// x to 23 bits of each 32-element block's largest.
 bool gemv_qcols_supports(int qtype);
-// How a few-column product uses the workspace, if it has one: x staged once ahead
-// of the product (pre), or K shared out over `shares` workgroups per row group
-// whose sums meet in part.
+// The kernel of a few-column product, and how the matrix-core one uses the
+// workspace, if it has one: x staged once ahead of the product (pre), or K shared
+// out over `shares` workgroups per row group whose sums meet in part.
 struct McolPlan {
+  bool fp32;
   char* pre;
   int shares;
   float* part;
 };
 // The workspace gemv_qcols_launch wants (0: none); it takes it or null.
-size_t gemv_qcols_workspace(int M, int K, int N, int num_cus);
+size_t gemv_qcols_workspace(int qtype, int M, int K, int N, int num_cus);
 hipError_t gemv_qcols_launch(int qtype, const void* w, const float* x, float* y, int M, int K, int N, int num_cus,
                              void* ws, hipStream_t st);
 // The merge epilogue's instance for a launch of `splits` chunks (gemv_common.h).

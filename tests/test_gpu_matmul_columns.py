@@ -101,18 +101,21 @@ def test_f16_columns_captured_without_a_workspace_and_noalloc(M, K, N):
 
 BLOCK_TYPES = {3: "q4_1", 6: "q5_0", 7: "q5_1", 8: "q8_0", 10: "q2_k", 11: "q3_k", 12: "q4_k", 13: "q5_k", 14: "q6_k",
                20: "iq4_nl", 23: "iq4_xs"}
-FINE_TYPES = (3, 6, 7, 10, 20, 23)  # one column: x in fp32, 19 bits of its group for the others
+FINE_TYPES = (3, 6, 7, 10, 20, 23)  # up to 7 columns: x in fp32
 
 
 def digit_bound(qtype, x, w):
-    """Half a step of x's digits in every element: a step is at most 2^-22 of its
-    16-element group's maximum (fine types), or 2^-18 of its group's (of 16 or 32
-    elements); plus 16 roundings of 2^-24 of sum |w x| for the 32-bit sums."""
-    n = 16 if qtype in FINE_TYPES else 32
+    """32 roundings of 2^-24 of sum |w x| for the 32-bit sums and, where x is held
+    in digits, half a step of them in every element: a step is at most 2^-22 of
+    its group's maximum (fine types from 8 columns on), or 2^-18 of its group's
+    (of 16 or 32 elements)."""
     ax = np.abs(x).astype(np.float64)
-    g = np.repeat(ax.reshape(x.shape[0], -1, n).max(2), n, axis=1)
+    bound = 32 * 2.0 ** -24 * (ax @ np.abs(w).T)
+    if qtype in FINE_TYPES and x.shape[0] < 8:
+        return bound
+    g = np.repeat(ax.reshape(x.shape[0], -1, 32).max(2), 32, axis=1)
     step = 2.0 ** (-22 if qtype in FINE_TYPES else -18)
-    return 0.5 * step * (g @ np.abs(w).T) + 16 * 2.0 ** -24 * (ax @ np.abs(w).T)
+    return bound + 0.5 * step * (g @ np.abs(w).T)
 
 
 # One column (the GEMV), then one, two and three tiles of digit rows (5, 10 and
@@ -200,22 +203,25 @@ def smallest_weights_at(qtype, t, M, K, k):
     return b.reshape(-1)
 
 
-# K = 512 and 3 or 4 units per lane's worth of K; the outlier in a group's first
-# and last quarter.
-@pytest.mark.parametrize("M,K,k", [(40, 512, 5), (33, 768, 256 + 15), (9, 11008, 10 + 512), (6, 16384, 5)])
-@pytest.mark.parametrize("N", [1])
+# One column and several: 16, 32 and 64 lanes a row, one to four units a lane, rows
+# past the grid's first turn, groups of columns (3 and 2 at 11008 and 16384); the
+# outlier in a group's first and last quarter.
+@pytest.mark.parametrize("M,K,k,N", [
+    (40, 512, 5, 1), (9, 11008, 10 + 512, 1), (6, 16384, 5, 1), (33, 768, 256 + 15, 2), (40, 512, 5, 7), (9, 11008, 10, 4),
+    (6, 16384, 5, 3), (9000, 2304, 256 + 15, 7), (70, 4096, 5, 5), (33, 8192, 5, 2),
+])
 @pytest.mark.parametrize("qtype", FINE_TYPES)
 def test_fp32_types_keep_the_neighbours_of_a_large_element(qtype, M, K, k, N):
     """x is fp32 for these types: an element of 1e5 under a zero (or the smallest)
-    weight leaves its neighbours' bits alone.  Bound: 32 roundings of 2^-24 of
-    sum |w x| (a group's 16 products, the groups of a lane, the lanes)."""
+    weight leaves its neighbours' bits alone.  digit_bound's 32 roundings: a group's
+    16 products, the groups of a lane, the lanes."""
     announce(f"large element {BLOCK_TYPES[qtype]} M={M} K={K} N={N}")
     data = smallest_weights_at(qtype, synth.tensor(qtype, 51, f"out{qtype}-{M}x{K}", M, K), M, K, k)
     x = synth.normal(52, f"outx{N}x{K}", N * K, 1.0).reshape(N, K)
     x[:, k] = 1e5
     w = oracle.dequant(qtype, data, M * K).reshape(M, K).astype(np.float64)
     y = gpu_matmul(qtype, data, x, M, K)
-    bound = 32 * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T)
+    bound = digit_bound(qtype, x, w)
     err = np.abs(y - x.astype(np.float64) @ w.T)
     assert np.all(err <= bound), float(np.max(err / bound))
 
