@@ -144,8 +144,8 @@ size_t gemv_qcols_workspace(int qtype, int M, int K, int N, int num_cus) {
   const int shares = mcol_shares(M, K, num_cus);
   if (shares > 1) return (size_t)shares * n * M * sizeof(float);
   if (!mcol_ahead(M, K, n, num_cus)) return 0;
-  const size_t tiles = (3 * n + 15) / 16;
-  return (size_t)((K + 127) / 128) * 4 * tiles * 704;  // the largest block (gemv_mcol.h)
+  const size_t tiles = (n + 3) / 4;
+  return (size_t)((K + 127) / 128) * 4 * tiles * 560;  // the largest block (gemv_mcol.h)
 }
 
 hipError_t gemv_qcols_launch(int qtype, const void* w, const float* x, float* y, int M, int K, int N, int num_cus,

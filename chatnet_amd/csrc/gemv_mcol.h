@@ -2,20 +2,26 @@
 // the int8 matrix cores, instantiated per weight type by the gemv_*.hip files.
 //
 // x is held as base-256 digits: per 32-element block and column a power of two
-// brings the largest |x| to 23 bits, X = D2 2^16 + D1 2^8 + D0 with signed bytes
-// D.  Three digits of N columns are 3N rows of an int8 operand, so one
+// brings the largest |x| to 31 bits, X = D3 2^24 + D2 2^16 + D1 2^8 + D0 with signed
+// bytes D.  Four digits of N columns are 4N rows of an int8 operand, so one
 // v_mfma_i32_16x16x32_i8 multiplies a 32-element block of 16 weight rows (their
-// codes as signed bytes) with five columns exactly, and the block's scale and the
-// column's 2^-e are applied to its four int32 results per lane in fp32.  The
-// weight rows are the operand whose index the lane keeps in the result (lane %
-// 16), so a row's scale is where its codes were unpacked.
+// codes as signed bytes) with four columns exactly.  The four int32 results of a
+// lane are one column's digits of one weight row (the weight rows are the operand
+// whose index the lane keeps, lane % 16): joined as (D3 2^8 + D2) + (D1 2^8 + D0)
+// 2^-16 in fp32, they are scaled by the row's block scale, where its
+// codes were unpacked, and the column's 2^-e.  31 bits of a block's largest are 12
+// more than the single-column GEMV keeps of 16 elements' (three digits, 23 bits,
+// fell short of it where the halves of a block differ by more than 16 times).
 //
-// What bounds it: the four conversions, multiplies and adds per block and tile
-// (12 to 16 VALU instructions for 16 rows x 32 weights x 5 columns); dot4 on
-// packed digits took 21 per 16 weights and column, one launch per column the
-// weight stream N times.  Against the MFMA GEMM and the column by column GEMV:
-// Q4_K 11008 x 4096 at 5 columns 31 -> 18 us, at 16 68 -> 26, Q8_0 4864 x 896 at 5
-// 18.9 -> 5.2.
+// What bounds it: joining, scaling and adding the digits (7 VALU instructions for 16
+// rows x 32 weights x 4 columns); dot4 on packed digits took 21 per 16 weights and
+// column, one launch per column the weight stream N times (18.9 us at 5 columns of
+// Q8_0 4864 x 896, here 5.3; the MFMA GEMM behind its packing pass 67.7 at 16 of Q4_K
+// 11008 x 4096, here 24.5).  Three digits, whose
+// results met a column at a time in fp32, took 12 for 5 columns: Q4_K 4096 x 4096 at
+// 4 columns 9.5 -> 7.0 us, at 5 10.4 -> 8.7, at 16 14.6 -> 14.8, Q8_0 4864 x 896 at
+// 5 6.6 -> 5.3, Q6_K 11008 x 4096 at 5 26.8 -> 30.8; error against float64 2.0e-7 ->
+// 1.0e-7 (Q8_0).
 #pragma once
 #include "gemv_quant.h"
 
@@ -256,11 +262,13 @@ __device__ __forceinline__ void mc_expand(uint32_t* r, int s, int p, int nblk, u
   }
 }
 
-// LDS bytes of one staged 32-element block and tile of 16 digit rows: the digits
-// in operand order, 2^(8 digit - e) per row, and for the types with an offset
-// sum X 2^-e (in the lowest digit's row, else 0), per half where the scales are.
+constexpr int kMcTile = 4;  // columns of a tile of 16 digit rows
+
+// LDS bytes of one staged 32-element block and tile: the digits in operand order,
+// 2^(16 - e) per column, and for the types with an offset the sum of its x, per half
+// where the scales are.
 template <int QT>
-constexpr int mc_block_bytes() { return 512 + 64 + (group_min<QT>() ? (mc_half_scales<QT>() ? 128 : 64) : 0); }
+constexpr int mc_block_bytes() { return 512 + 16 + (group_min<QT>() ? (mc_half_scales<QT>() ? 32 : 16) : 0); }
 
 // Sixteen elements (half hb & 1 of block hb / 2) of column c into the staged
 // blocks at `base`.  The block's two halves are on adjacent lanes.  A
@@ -276,44 +284,41 @@ __device__ __forceinline__ void mc_stage(const float (&v)[16], int c, int hb, ch
   const bool finite = mb < 0x7F800000u;
   int e = 0;
   const float f = frexpf(__uint_as_float(mb), &e);
-  const int sc = mb == 0 || !finite ? 0 : (f > 0.996f ? 22 : 23) - e;  // |X| <= 0x7F7F7F, the digits' range
+  const int sc = mb == 0 || !finite ? 0 : (f > 0.996f ? 30 : 31) - e;  // |X| <= 0x7F7F7F7F, the digits' range
   uint32_t U[16];
-  int sum = 0;
 #pragma unroll
-  for (int j = 0; j < 16; j++) {
-    const int X = (int)rintf(ldexpf(v[j], sc));
-    if constexpr (MIN) sum += X;
-    U[j] = (uint32_t)(X + 0x808080);  // bytes 0..2 are D + 128
-  }
-  const int m0 = 3 * c;
-  char* blk = base + (size_t)(hb >> 1) * CT * BB;
+  for (int j = 0; j < 16; j++)
+    U[j] = (uint32_t)(int)rintf(finite ? ldexpf(v[j], sc) : 0.f) + 0x80808080u;  // its bytes are D + 128
+  const int cc = c % kMcTile;
+  char* blk = base + ((size_t)(hb >> 1) * CT + c / kMcTile) * BB;
 #pragma unroll
   for (int g = 0; g < 4; g++) {  // lane group g's four elements of this half
     const uint32_t u0 = U[TR ? g : 4 * g], u1 = U[TR ? 4 + g : 4 * g + 1];
     const uint32_t u2 = U[TR ? 8 + g : 4 * g + 2], u3 = U[TR ? 12 + g : 4 * g + 3];
     const uint32_t a01 = __builtin_amdgcn_perm(u1, u0, 0x05010400u);  // u0.b0 u1.b0 u0.b1 u1.b1
     const uint32_t a23 = __builtin_amdgcn_perm(u3, u2, 0x05010400u);
-    const uint32_t c01 = __builtin_amdgcn_perm(u1, u0, 0x00000602u);  // u0.b2 u1.b2
-    const uint32_t c23 = __builtin_amdgcn_perm(u3, u2, 0x00000602u);
-    const uint32_t D[3] = {__builtin_amdgcn_perm(a23, a01, 0x05040100u) ^ 0x80808080u,
+    const uint32_t c01 = __builtin_amdgcn_perm(u1, u0, 0x07030602u);  // u0.b2 u1.b2 u0.b3 u1.b3
+    const uint32_t c23 = __builtin_amdgcn_perm(u3, u2, 0x07030602u);
+    const uint32_t D[4] = {__builtin_amdgcn_perm(a23, a01, 0x05040100u) ^ 0x80808080u,
                            __builtin_amdgcn_perm(a23, a01, 0x07060302u) ^ 0x80808080u,
-                           __builtin_amdgcn_perm(c23, c01, 0x05040100u) ^ 0x80808080u};
+                           __builtin_amdgcn_perm(c23, c01, 0x05040100u) ^ 0x80808080u,
+                           __builtin_amdgcn_perm(c23, c01, 0x07060302u) ^ 0x80808080u};
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
-      const int m = m0 + d;
-      *reinterpret_cast<uint32_t*>(blk + (m >> 4) * BB + 8 * (16 * g + (m & 15)) + 4 * (hb & 1)) = D[d];
-    }
+    for (int d = 0; d < 4; d++)  // digit row 4 cc + d
+      *reinterpret_cast<uint32_t*>(blk + 8 * (16 * g + 4 * cc + d) + 4 * (hb & 1)) = D[d];
   }
-  const int other = MIN && !HALF ? __shfl_xor(sum, 1, CN_WAVE) : 0;
+  float* sp = reinterpret_cast<float*>(blk + 512) + cc;
+  if ((hb & 1) == 0) sp[0] = finite ? ldexpf(1.0f, 16 - sc) : NAN;
+  if constexpr (MIN) {
+    float s[8];
 #pragma unroll
-  for (int d = 0; d < 3; d++) {
-    const int m = m0 + d;
-    float* sp = reinterpret_cast<float*>(blk + (m >> 4) * BB + 512) + (m & 15);
-    if ((hb & 1) == 0) sp[0] = finite ? ldexpf(1.0f, 8 * d - sc) : NAN;
-    if constexpr (MIN) {
-      const float sx = d == 0 ? ldexpf((float)(sum + other), -sc) : 0.f;
-      if constexpr (HALF) sp[16 + 16 * (hb & 1)] = sx;
-      else if ((hb & 1) == 0) sp[16] = sx;
+    for (int j = 0; j < 8; j++) s[j] = v[j] + v[j + 8];
+    const float sum = ((s[0] + s[4]) + (s[1] + s[5])) + ((s[2] + s[6]) + (s[3] + s[7]));
+    if constexpr (HALF) {
+      sp[4 + 4 * (hb & 1)] = sum;
+    } else {
+      const float other = __shfl_xor(sum, 1, CN_WAVE);
+      if ((hb & 1) == 0) sp[4] = sum + other;
     }
   }
 }
@@ -348,8 +353,7 @@ __global__ __launch_bounds__(CN_BLOCK) void mcol_prep_kernel(const float* __rest
   mc_stage<QT, CT>(v, c, hb, dst);
 }
 
-// CT: tiles of 16 digit rows (5 columns each, 16 columns in 3), RT: tiles of 16
-// weight rows per wave.  The eight waves of a workgroup are rg row groups x 8 /
+// CT: tiles of 16 digit rows (4 columns each), RT: tiles of 16 weight rows per wave.  The eight waves of a workgroup are rg row groups x 8 /
 // rg interleaved shares of K.  kc elements of x at a time are staged in LDS, or
 // with PRE copied from what mcol_prep_kernel staged (pre).
 // With several workgroups along K (blockIdx.y, spb steps each) the sums go to
@@ -380,13 +384,11 @@ __global__ __launch_bounds__(512) void gemv_mcol_kernel(GemvArgs a, int ncols, i
   };
   load((kb >> 7) + ks);  // travels while x is staged
 
-  float acc[RT][CT][4];
+  float acc[RT][CT];  // weight row li of the tile, column p of the tile
 #pragma unroll
   for (int t = 0; t < RT; t++)
 #pragma unroll
-    for (int c = 0; c < CT; c++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) acc[t][c][i] = 0.f;
+    for (int c = 0; c < CT; c++) acc[t][c] = 0.f;
 
   for (int k0 = kb; k0 < K; k0 += kc) {
     const int kn = (min(kc, K - k0) + 127) & ~127;  // staged with zeros past K
@@ -425,54 +427,40 @@ __global__ __launch_bounds__(512) void gemv_mcol_kernel(GemvArgs a, int ncols, i
         for (int c = 0; c < CT; c++) {
           const char* blk = mlds + ((size_t)(4 * s + b - (k0 >> 5)) * CT + c) * BB;
           const long xf = *reinterpret_cast<const long*>(blk + 8 * lane);
-          const float4 pe = *reinterpret_cast<const float4*>(blk + 512 + 16 * p);
-          const float pev[4] = {pe.x, pe.y, pe.z, pe.w};
+          const float pe = *reinterpret_cast<const float*>(blk + 512 + 4 * p);
 #pragma unroll
           for (int hv = 0; hv < (HALF ? 2 : 1); hv++) {
-            float sxv[4] = {};
-            if constexpr (MIN) {
-              const float4 sx = *reinterpret_cast<const float4*>(blk + 576 + 64 * hv + 16 * p);
-              sxv[0] = sx.x; sxv[1] = sx.y; sxv[2] = sx.z; sxv[3] = sx.w;
-            }
+            float sx = 0.f;
+            if constexpr (MIN) sx = *reinterpret_cast<const float*>(blk + 528 + 16 * hv + 4 * p);
 #pragma unroll
             for (int t = 0; t < RT; t++) {
               const uint32_t w0 = HALF && hv == 1 ? 0u : q[t][b][0], w1 = HALF && hv == 0 ? 0u : q[t][b][1];
               const long wf = (long)(((uint64_t)w1 << 32) | w0);
               const mc_i32x4 r = __builtin_amdgcn_mfma_i32_16x16x32_i8(xf, wf, mc_i32x4{0, 0, 0, 0}, 0, 0, 0);
-#pragma unroll
-              for (int i = 0; i < 4; i++) {
-                acc[t][c][i] = fmaf((float)r[i] * sa[t][b][hv], pev[i], acc[t][c][i]);
-                if constexpr (MIN) acc[t][c][i] = fmaf(sb[t][b][hv], sxv[i], acc[t][c][i]);
-              }
+              // |r| <= 2^19: each pair joined in int32
+              const float v = fmaf((float)(r[1] * 256 + r[0]), 0x1p-16f, (float)(r[3] * 256 + r[2]));
+              if constexpr (MIN) acc[t][c] = fmaf(sb[t][b][hv], sx, acc[t][c]);
+              acc[t][c] = fmaf(v * sa[t][b][hv], pe, acc[t][c]);
             }
           }
         }
       }
     }
   }
-  // the waves' shares of K and the three digits meet in LDS, summed in wave order
+  // the waves' shares of K meet in LDS, summed in wave order
   __syncthreads();
   float* red = reinterpret_cast<float*>(mlds);
 #pragma unroll
   for (int t = 0; t < RT; t++)
 #pragma unroll
-    for (int c = 0; c < CT; c++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) red[((wave * RT + t) * CT + c) * 256 + (4 * p + i) * 16 + li] = acc[t][c][i];
+    for (int c = 0; c < CT; c++) red[((wave * RT + t) * CT + c) * 64 + lane] = acc[t][c];
   __syncthreads();
   for (int o = threadIdx.x; o < rg * RT * 16 * ncols; o += 512) {
     const int n = o & 15, t = (o >> 4) % RT, c = (o / (16 * RT)) % ncols, g = o / (16 * RT * ncols);
     const int row = (blockIdx.x * rg + g) * (16 * RT) + 16 * t + n;
     float v = 0.f;
-    for (int k = 0; k < nks; k++) {
-      float part = 0.f;
-#pragma unroll
-      for (int d = 0; d < 3; d++) {
-        const int m = 3 * c + d;
-        part += red[(((g * nks + k) * RT + t) * CT + (m >> 4)) * 256 + (m & 15) * 16 + n];
-      }
-      v += part;
-    }
+    for (int k = 0; k < nks; k++)
+      v += red[(((g * nks + k) * RT + t) * CT + c / kMcTile) * 64 + 16 * (c % kMcTile) + n];
     float* to = part ? part + (size_t)blockIdx.y * ncols * M : a.out[0];
     if (row < M) to[(size_t)c * M + row] = v;
   }
@@ -502,7 +490,7 @@ hipError_t launch_mcol_one(const GemvArgs& a, int ncols, int num_cus, const char
   if ((groups + rg - 1) / rg <= num_cus) fit = (156 * 1024) / per_step;
   const int steps = nsteps <= fit ? nsteps : fit / turn * turn;
   const size_t stage = (size_t)steps * per_step;
-  const size_t red = (size_t)8 * RT * CT * 256 * sizeof(float);
+  const size_t red = (size_t)8 * RT * CT * 64 * sizeof(float);
   const size_t smem = stage > red ? stage : red;
   const auto kern = &gemv_mcol_kernel<QT, CT, RT, PRE>;
   if (smem > 64 * 1024) {
@@ -524,19 +512,19 @@ hipError_t launch_mcol_one(const GemvArgs& a, int ncols, int num_cus, const char
 // (each x fragment read then feeds two products).
 template <int QT, int CT>
 hipError_t launch_mcol_ct(const GemvArgs& a, int ncols, int num_cus, const McolPlan& p, hipStream_t st) {
-  const bool one = CT == 3 || a.n_vrows <= 16 * num_cus;
+  const bool one = CT > 2 || a.n_vrows <= 16 * num_cus;
   if (p.pre) {
     const int halves = (a.K + 127) / 128 * 8;
     hipLaunchKernelGGL((mcol_prep_kernel<QT, CT>), dim3((halves + CN_BLOCK - 1) / CN_BLOCK, ncols), dim3(CN_BLOCK), 0, st,
                        a.x, a.K, halves, p.pre);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if constexpr (CT < 3) {
+    if constexpr (CT <= 2) {
       if (!one) return launch_mcol_one<QT, CT, 2, true>(a, ncols, num_cus, p.pre, 1, nullptr, st);
     }
     return launch_mcol_one<QT, CT, 1, true>(a, ncols, num_cus, p.pre, 1, nullptr, st);
   }
-  if constexpr (CT < 3) {
+  if constexpr (CT <= 2) {
     if (!one) return launch_mcol_one<QT, CT, 2, false>(a, ncols, num_cus, nullptr, 1, nullptr, st);
   }
   return launch_mcol_one<QT, CT, 1, false>(a, ncols, num_cus, nullptr, p.shares, p.part, st);
@@ -544,9 +532,10 @@ hipError_t launch_mcol_ct(const GemvArgs& a, int ncols, int num_cus, const McolP
 
 template <int QT>
 hipError_t launch_mcol(const GemvArgs& a, int ncols, int num_cus, const McolPlan& p, hipStream_t st) {
-  if (ncols <= 5) return launch_mcol_ct<QT, 1>(a, ncols, num_cus, p, st);
-  if (ncols <= 10) return launch_mcol_ct<QT, 2>(a, ncols, num_cus, p, st);
-  return launch_mcol_ct<QT, 3>(a, ncols, num_cus, p, st);
+  if (ncols <= 4) return launch_mcol_ct<QT, 1>(a, ncols, num_cus, p, st);
+  if (ncols <= 8) return launch_mcol_ct<QT, 2>(a, ncols, num_cus, p, st);
+  if (ncols <= 12) return launch_mcol_ct<QT, 3>(a, ncols, num_cus, p, st);
+  return launch_mcol_ct<QT, 4>(a, ncols, num_cus, p, st);
 }
 
 }  // namespace

@@ -90,7 +90,7 @@ hipError_t gemv_float_cols_launch(int qtype, const void* w, const float* x, floa
 // Block types other than Q4_0 read from their stored blocks against N columns of
 // x: Q4_1, Q5_0, Q5_1, Q2_K, IQ4_NL and IQ4_XS up to 7 columns in fp32
 // (gemv_xcols.h), else on the int8 matrix cores (gemv_mcol.h), up to 16 per launch,
-// x to 23 bits of each 32-element block's largest.
+// x to 31 bits of each 32-element block's largest.
 bool gemv_qcols_supports(int qtype);
 // The kernel of a few-column product, and how the matrix-core one uses the
 // workspace, if it has one: x staged once ahead of the product (pre), or K shared
