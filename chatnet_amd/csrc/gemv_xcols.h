@@ -128,10 +128,15 @@ hipError_t launch_xcols_nc(const GemvArgs& a, int ncols, int num_cus, hipStream_
   if (nunits <= 16) return launch_xcols_k<QT, NC, 16, 1>(a, ncols, num_cus, st);
   if (nunits <= 32) return launch_xcols_k<QT, NC, 32, 1>(a, ncols, num_cus, st);
   if (nunits <= 64) return launch_xcols_k<QT, NC, 64, 1>(a, ncols, num_cus, st);
-  if constexpr (QTraits<QT>::UNIT == 128) {
+  if constexpr (QTraits<QT>::UNIT == 64) {
+    if (nunits <= 128) return launch_xcols_k<QT, NC, 64, 2>(a, ncols, num_cus, st);
+  }
+  // K > 8192: LDS holds four columns at most
+  if constexpr (NC > 4) {
+    return hipErrorInvalidValue;
+  } else if constexpr (QTraits<QT>::UNIT == 128) {
     return launch_xcols_k<QT, NC, 64, 2>(a, ncols, num_cus, st);
   } else {
-    if (nunits <= 128) return launch_xcols_k<QT, NC, 64, 2>(a, ncols, num_cus, st);
     if (nunits <= 192) return launch_xcols_k<QT, NC, 64, 3>(a, ncols, num_cus, st);
     return launch_xcols_k<QT, NC, 64, 4>(a, ncols, num_cus, st);
   }
