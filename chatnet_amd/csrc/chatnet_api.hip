@@ -1217,10 +1217,10 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
   if ((type == CHATNET_GGML_F32 || type == CHATNET_GGML_F16) && N >= 2)
     return matmul_float((int)type, w_dev, x_dev, y_dev, M, K, N, dev, cus, st, noalloc);
   // The other block types up to kColsGemv columns: all columns at once on the
-  // stored blocks (gemv_qcols_launch), more precise and faster than the MFMA
-  // GEMM behind its packing pass (Q4_K 4096 x 4096 at 16 columns 14.7 against
-  // 38.4 us, 11008 x 4096 26.3 against 68.0, Q3_K 2048 x 11008 45.4 against
-  // 61.2).  Two columns (Q3_K, whose unpacking costs the most: three) of a
+  // stored blocks (gemv_qcols_launch), more precise (1e-7 against 3e-4) and
+  // mostly faster than the MFMA GEMM on them: at 16 columns Q4_K 4096 x 4096 14.8
+  // us, 11008 x 4096 24.5 against 22.0, 4096 x 11008 28.8 against 23.1, Q6_K 36.4
+  // against 42.8; at 11 Q4_K 4096 x 11008 22.5 against 23.1.  Two columns (Q3_K, whose unpacking costs the most: three) of a
   // matrix of at least kTwoGemvs weights run the single-column GEMV for each
   // (11008 x 4096: Q4_K at 2 columns 13.1 against 16.6 us, Q3_K at 3 24.7
   // against 29.0).  More columns run the GEMM on the
@@ -1233,8 +1233,7 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
   const int stored = gemm_stored_format((int)type, K);  // the GEMM's format on the stored blocks, -1: packed units
   const bool must_pack = gemv_needs_pack((int)type);
   const bool ahead = packed_ahead(type);
-  const bool long_rows = N > 10 && K > 8192 && stored >= 0;  // 4096 x 11008 at 16 columns: Q4_K 27.7 against 23.3 us
-  const bool batched = N >= 8 && !(N <= kColsGemv && gemv_qcols_supports((int)type) && !long_rows) &&
+  const bool batched = N >= 8 && !(N <= kColsGemv && gemv_qcols_supports((int)type)) &&
                        (type == CHATNET_GGML_Q4_0 || ahead || (!noalloc && gemm_pack_supports((int)type, K)));
   const bool pack = must_pack || (batched && stored < 0);
   const uint8_t* wp = (const uint8_t*)w_dev;

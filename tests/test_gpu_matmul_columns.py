@@ -145,6 +145,22 @@ def test_block_types_few_columns_match_float64(qtype, M, K, N):
         assert np.linalg.norm(y - r) <= 6e-7 * np.linalg.norm(r), float(np.linalg.norm(y - r) / np.linalg.norm(r))
 
 
+@pytest.mark.parametrize("qtype", sorted(BLOCK_TYPES))
+def test_up_to_sixteen_columns_of_any_length_keep_their_precision(qtype):
+    """10 and 11 columns, K = 8192 and beyond, K shared over workgroups and not:
+    digit_bound and 6e-7 in the 2-norm up to 16 columns (fp16 operands, from 17 on,
+    give 3e-4)."""
+    for (M, K, N) in [(33, 8192, 16), (33, 8448, 10), (33, 8448, 11), (2100, 8448, 16), (37, 11008, 11), (20, 16384, 16)]:
+        announce(f"long rows {BLOCK_TYPES[qtype]} M={M} K={K} N={N}")
+        t = synth.tensor(qtype, 55, f"long{qtype}-{M}x{K}", M, K)
+        x = synth.normal(56, f"longx{N}x{K}", N * K, 1.0).reshape(N, K)
+        y = gpu_matmul(qtype, t.data, x, M, K)
+        w = oracle.dequant(qtype, t.data, M * K).reshape(M, K).astype(np.float64)
+        r = x.astype(np.float64) @ w.T
+        assert np.all(np.abs(y - r) <= digit_bound(qtype, x, w))
+        assert np.linalg.norm(y - r) <= 6e-7 * np.linalg.norm(r)
+
+
 def test_odd_rows_of_short_k_match_float64():
     """K = 64 and 192: one pair of blocks, and rows whose records end mid-unit."""
     for qtype in (3, 6, 7, 8, 20):
