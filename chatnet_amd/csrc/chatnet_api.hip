@@ -1220,14 +1220,17 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
   // stored blocks (gemv_qcols_launch), more precise (1e-7 against 3e-4) and
   // mostly faster than the MFMA GEMM on them: at 16 columns Q4_K 4096 x 4096 14.8
   // us, 11008 x 4096 24.5 against 22.0, 4096 x 11008 28.8 against 23.1, Q6_K 36.4
-  // against 42.8; at 11 Q4_K 4096 x 11008 22.5 against 23.1.  Two columns (Q3_K, whose unpacking costs the most: three) of a
-  // matrix of at least kTwoGemvs weights run the single-column GEMV for each
-  // (11008 x 4096: Q4_K at 2 columns 13.1 against 16.6 us, Q3_K at 3 24.7
-  // against 29.0).  More columns run the GEMM on the
-  // stored blocks; Q3_K, Q6_K, Q8_K and the other IQ types are packed into the
-  // workspace first, one pass over W (the no-allocation variant runs the GEMM
-  // for Q4_0 and the packed_ahead types only).  The
-  // types the GEMV reads only as packed units are packed for every N.
+  // against 42.8; at 11 Q4_K 4096 x 11008 22.5 against 23.1.  Two columns of
+  // Q6_K and three of Q3_K, whose unpacking costs the most, run the single-column
+  // GEMV for each from kTwoGemvs weights on (two columns, GEMVs and one product:
+  // Q6_K 11008 x 4096 18.6 and 22.5 us, 4096 x 11008 20.9 and 22.8, 3584 x 8192
+  // 16.3 and 13.9; Q3_K 16.7 and 27.5, 22.3 and 34.4, 4096 x 4096 9.8 and 9.6, three
+  // columns 24.8 and 28.3, 32.7 and 34.4, 14.6 and 10.0; the other types' product
+  // won at every size, Q4_K 11008 x 4096 13.1 and 12.6, Q8_0 18.3 and 15.1).  More
+  // columns run the GEMM on the stored blocks; Q3_K, Q6_K, Q8_K and the other IQ
+  // types are packed into the workspace first, one pass over W (the no-allocation
+  // variant runs the GEMM for Q4_0 and the packed_ahead types only).  The types
+  // the GEMV reads only as packed units are packed for every N.
   constexpr int kColsGemv = 16;
   constexpr long long kTwoGemvs = 32LL << 20;
   const int stored = gemm_stored_format((int)type, K);  // the GEMM's format on the stored blocks, -1: packed units
@@ -1292,7 +1295,8 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
       return CHATNET_OK;
     }
   }
-  if (N >= 2 && !pack && gemv_qcols_supports((int)type) && !(N <= (type == CHATNET_GGML_Q3_K ? 3 : 2) && (long long)M * K >= kTwoGemvs)) {
+  const int gemvs = type == CHATNET_GGML_Q3_K ? 3 : type == CHATNET_GGML_Q6_K ? 2 : 1;
+  if (N >= 2 && !pack && gemv_qcols_supports((int)type) && !(N <= gemvs && (long long)M * K >= kTwoGemvs)) {
     // x staged once in the stream's workspace where there is one and it pays
     const size_t need = noalloc ? 0 : gemv_qcols_workspace((int)type, M, K, N, cus);
     char* ws = nullptr;

@@ -100,14 +100,15 @@ bool gemv_qcols_supports(int qtype) {
 // Few row groups and long rows (at most half a workgroup of 16 rows per CU, at
 // least 24 steps of 128 weights): K shared out over up to 16 workgroups per row
 // group, each wave keeping a step, and a launch that adds the shares: Q4_K 164 x
-// 11008 at 6 columns 21.2 -> 10.9 us, Q8_0 90 x 10432 at 2 11.3 -> 7.9.  At up to
-// two workgroups per CU it lost (4096 x 4096 at 5 columns 9.0 -> 11.1 us, 3000 x
-// 8192 at 8 16.1 -> 27.8; 1500 x 14336 won 1 to 3 us of 13 to 29).
-// Otherwise staging x costs a workgroup about 15 VALU instructions an element,
-// so from 22000 elements per CU on (columns x K, times the workgroups a CU runs)
-// it is done once ahead, a launch of 3 us: Q4_K 11008 x 4096 at 4 columns 20.8
-// us with every workgroup staging and 17.9 ahead, at 2 columns 16.6 and 17.8;
-// Q8_0 4096 x 4096 at 4 columns 8.8 and 11.7, at 7 columns 13.1 and 11.9.
+// 11008 at 6 columns 17.8 -> 8.8 us, 2048 x 11008 17.9 -> 15.3, 2048 x 4096 10.5 ->
+// 8.2 (at 2 columns 5.5 -> 6.5).  At a workgroup per CU it lost (4096 x 4096 at 6
+// columns 10.7 -> 11.2 us, at 12 12.3 -> 16.7).
+// Otherwise staging x costs a workgroup about 20 VALU instructions an element,
+// so from 32768 elements per CU on (columns x K, times the workgroups a CU runs)
+// it is done once ahead, a launch of 3 us.  Every workgroup staging, and ahead:
+// Q4_K 11008 x 4096 at 4 columns (22000) 14.4 and 16.0 us, 4096 x 4096 at 8 (32768)
+// 10.8 and 10.8, 2048 x 2048 at 16 14.4 and 9.4, Q8_0 10.1 and 9.3, 32000 x 4096 at
+// 4 36.9 and 38.1, Q4_K 4096 x 11008 at 4 (44000) 14.3 and 14.2, at 8 25.2 and 18.3.
 static int mcol_shares(int M, int K, int num_cus) {
   const int groups = (M + 15) / 16, nsteps = (K + 127) / 128;
   if (nsteps < 24 || 2 * groups > num_cus) return 1;
@@ -119,7 +120,7 @@ static int mcol_shares(int M, int K, int num_cus) {
 static bool mcol_ahead(int M, int K, int n, int num_cus) {
   const long long rows = M <= 16 * num_cus ? 16 : 32;
   const double wgs = (double)((M + rows - 1) / rows) / num_cus;
-  return (double)n * K * (wgs < 1 ? 1 : wgs > 2 ? 2 : wgs) >= 22000.0;
+  return (double)n * K * (wgs < 1 ? 1 : wgs > 2 ? 2 : wgs) >= 32768.0;
 }
 
 // Types whose x stays in fp32 up to kFp32Cols columns, as the single column's does

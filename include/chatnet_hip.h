@@ -258,11 +258,11 @@ CHATNET_API int chatnet_get_logits(chatnet_model* m, float* logits_host);
  * with x as two fp16 planes, summed with compensation in fp32 (its error
  * against float64 is the GEMV's, 1e-7).  Q4_1, Q5_0, Q5_1,
  * Q8_0, Q2_K .. Q6_K, IQ4_NL and IQ4_XS run up to 16 columns on their stored
- * blocks (one column, and two or three of a large matrix: the fused GEMV per
- * column): Q4_1, Q5_0, Q5_1, Q2_K, IQ4_NL and IQ4_XS up to 7 columns with x in
- * fp32, else with x to 31 bits of each 32 elements' largest; Q8_K and the other IQ
- * types below 8 columns run the GEMV once per column on the re-encoded copy,
- * made in the workspace first.  A GEMM whose grid of 128 x 128 tiles
+ * blocks (one column, two of a large Q6_K and two or three of a large Q3_K
+ * matrix: the fused GEMV per column): Q4_1, Q5_0, Q5_1, Q2_K, IQ4_NL and IQ4_XS
+ * up to 7 columns with x in fp32, else with x to 31 bits of each 32 elements'
+ * largest; Q8_K and the other IQ types below 8 columns run the GEMV once per
+ * column on the re-encoded copy, made in the workspace first.  A GEMM whose grid of 128 x 128 tiles
  * is just over one tile per CU (e.g. 11008 x 4096 at N = 512) runs as a
  * stream-K launch: one whole tile per CU, the other tiles' K chunks shared
  * out evenly, a shared tile summed in K order by its last contributor (the
