@@ -1133,12 +1133,14 @@ int run_prompt(chatnet_model* m, const int32_t* tokens, int n, int position) {
 }
 
 // F32 / F16 rows with several columns.  One launch of the multi-column GEMV takes
-// the columns whose fp32 x fits in LDS (8 up to K = 4864, 3 at 11008); F16 with
-// more of them runs the span kernel's exact-weight F16 product (W * xh + W *
-// xl, x as two fp16 planes, fp32 sums) out of the stream's workspace, three
-// launches whatever N is: F16 4096 x 4096 at 8 columns 20.5 us in one GEMV
-// launch and 25.1 us as a product, at 24 columns 140 us column by column and
-// 26 us; 2048 x 11008 at 7 columns 44 us in three GEMV launches.  F32, a
+// the columns whose fp32 x fits in LDS (8 up to K = 4864, 3 at 11008), each the
+// single-column result bit for bit; F16 with more of them runs the matrix-core
+// product of the exact weights with x in three fp16 planes (GEMM_W_F16_X3) out of
+// the stream's workspace, three launches whatever N is: F16 4096 x 4096 at 24
+// columns 20.0 us (140 column by column), 4096 x 11008 at 6 33 (51 in two GEMV
+// launches).  At 8 columns that one GEMV launch holds the two take 20.5 and 19.8 us
+// for 4096 x 4096, 8.1 and 17.3 for 2048 x 2048, 51.7 and 27.4 for 11008 x 4096:
+// the line lies where the GEMV's bits end, not where the product is faster.  F32, a
 // capturing stream whose workspace is too small and the no-allocation variant
 // (which takes these types without scratch, so overlapping calls are safe) run
 // the multi-column GEMV for any N.
@@ -1148,20 +1150,20 @@ int matmul_float(int type, const void* w, const float* x, float* y, int M, int K
     std::lock_guard<std::mutex> lk(g_enqueue_mu);
     const size_t plane = ((size_t)N * K * sizeof(uint16_t) + 255) & ~(size_t)255;
     const size_t scales = ((size_t)N * sizeof(float) + 255) & ~(size_t)255;
-    const size_t part = gemm_workspace_bytes(M, N, K, cus, true, GEMM_W_F16);
+    const size_t part = gemm_workspace_bytes(M, N, K, cus, true, GEMM_W_F16_X3);
     char* ws = nullptr;
     bool ok = true;
-    const int rc = matmul_workspace(dev, st, kMatmulCounterBytes + 2 * plane + scales + part, &ws, &ok);
+    const int rc = matmul_workspace(dev, st, kMatmulCounterBytes + 3 * plane + scales + part, &ws, &ok);
     if (rc) return rc;
     if (ok) {
       uint16_t* xh = (uint16_t*)(ws + kMatmulCounterBytes);
-      uint16_t* xl = (uint16_t*)((char*)xh + plane);
-      float* xinv = (float*)((char*)xl + plane);
-      HIP_TRY(to_f16_planes_launch(x, xh, xl, xinv, N, K, st));
+      const size_t elems = plane / sizeof(uint16_t);
+      float* xinv = (float*)((char*)xh + 3 * plane);
+      HIP_TRY(to_f16_planes_launch(x, xh, elems, xinv, N, K, st));
       GemmArgs g;
       memset(&g, 0, sizeof(g));
       g.qtype = type;
-      g.packed = GEMM_W_F16;
+      g.packed = GEMM_W_F16_X3;
       g.precise = 1;
       g.w[0] = g.w[1] = g.w[2] = (const uint8_t*)w;
       g.seg_rows[0] = M;
@@ -1170,7 +1172,8 @@ int matmul_float(int type, const void* w, const float* x, float* y, int M, int K
       g.K = K;
       g.N = N;
       g.xb = xh;
-      g.xb_lo = xl;
+      g.xb_lo = xh + elems;
+      g.xb_ll = xh + 2 * elems;
       g.xinv = xinv;
       g.x32 = x;
       g.epi = GEMV_EPI_STORE;

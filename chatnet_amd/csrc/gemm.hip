@@ -96,13 +96,13 @@ __global__ __launch_bounds__(CN_BLOCK) void to_f16_scaled_kernel(const float* __
   }
 }
 
-// x [N][K] fp32 -> the span kernel's two planes with the per-column scaling of
-// to_f16_scaled_kernel (the largest finite |x| in [2^14, 2^15)): hi = fp16(x *
-// 2^e), lo = fp16(x * 2^e - hi), together within 2^-24 of the element (lo's own
-// subnormals start 2^-39 below the column's largest).  An infinity keeps lo = 0.
+// x [N][K] fp32 -> GEMM_W_F16_X3's planes with the per-column scaling of
+// to_f16_scaled_kernel (the largest finite |x| in [2^14, 2^15)): y = x * 2^e, p0 =
+// fp16(y), p1 = fp16((y - p0) 2^11), p2 = fp16((y - p0 - p1 2^-11) 2^22), both
+// remainders exact in fp32 and below 2^15.
 template <int V>
 __global__ __launch_bounds__(CN_BLOCK) void to_f16_planes_kernel(const float* __restrict__ x,
-                                                                uint16_t* __restrict__ xh, uint16_t* __restrict__ xl,
+                                                                uint16_t* __restrict__ xp, size_t plane,
                                                                 float* __restrict__ xinv, int K) {
   __shared__ float red[4];
   const size_t n = blockIdx.x;
@@ -133,18 +133,20 @@ __global__ __launch_bounds__(CN_BLOCK) void to_f16_planes_kernel(const float* __
     const int i = (threadIdx.x + CN_BLOCK * j) * 4;
     if (i >= K) continue;
     const f32x4 y = v[j] * sc;  // 2^e is a normal float for e in [-125, 125]
-    _Float16 hi[4], lo[4];
+    _Float16 pl[3][4];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-      hi[q] = (_Float16)y[q];
-      const float r = y[q] - (float)hi[q];
-      lo[q] = fabsf(y[q]) <= 3.402823466e38f ? (_Float16)r : (_Float16)0.f;
+      const bool fin = fabsf(y[q]) <= 3.402823466e38f;
+      pl[0][q] = (_Float16)y[q];
+      const float r = fin ? (y[q] - (float)pl[0][q]) * 2048.0f : 0.f;
+      pl[1][q] = (_Float16)r;
+      pl[2][q] = (_Float16)((r - (float)pl[1][q]) * 2048.0f);
     }
     const size_t o = n * K + cn_span_pos(i);  // four adjacent elements stay adjacent
-    *reinterpret_cast<uint2*>(xh + o) = make_uint2(__builtin_bit_cast(uint32_t, (cn_half2){hi[0], hi[1]}),
-                                                   __builtin_bit_cast(uint32_t, (cn_half2){hi[2], hi[3]}));
-    *reinterpret_cast<uint2*>(xl + o) = make_uint2(__builtin_bit_cast(uint32_t, (cn_half2){lo[0], lo[1]}),
-                                                   __builtin_bit_cast(uint32_t, (cn_half2){lo[2], lo[3]}));
+#pragma unroll
+    for (int p = 0; p < 3; p++)
+      *reinterpret_cast<uint2*>(xp + p * plane + o) = make_uint2(__builtin_bit_cast(uint32_t, (cn_half2){pl[p][0], pl[p][1]}),
+                                                                 __builtin_bit_cast(uint32_t, (cn_half2){pl[p][2], pl[p][3]}));
   }
 }
 
@@ -541,7 +543,8 @@ __global__ __launch_bounds__(CN_BLOCK) void gemm_pack16_kernel(const uint8_t* __
 // (at least 8 chunks of 64 per split).  Span kernel: 32 or 64 columns; a tile grid of more than two workgroups per CU
 // takes the 2-stage ring (44 KB for raw Q4_0 at 64 columns, three workgroups
 // per CU; 56 KB for packed units and Q8_0, two), a smaller one the 3-stage ring
-// (two per CU), unless three stages leave one workgroup per CU (packed units,
+// (two per CU), unless three stages leave one workgroup per CU (F16 against three
+// planes, at 32 columns too: 11008 x 4096 at 24 39.8 -> 29.5 us; packed units,
 // Q8_0, F16: 7B-shaped Q4_K_M 2 layers, 333 tokens 1428 -> 1363 us; F16 200
 // tokens 887 -> 818), and a K split into the largest count that keeps the grid
 // within one round of resident workgroups with at least 8 chunks per split (a
@@ -561,6 +564,7 @@ int span_ring_bytes(int tn, int stages, int wf) {
   switch (wf) {
     case GEMM_W_PACKED: return span_ring_bytes_t<GEMM_W_PACKED>(tn, stages);
     case GEMM_W_F16: return span_ring_bytes_t<GEMM_W_F16>(tn, stages);
+    case GEMM_W_F16_X3: return span_ring_bytes_t<GEMM_W_F16_X3>(tn, stages);
     case GEMM_W_F32: return span_ring_bytes_t<GEMM_W_F32>(tn, stages);
     case GEMM_W_Q4_K: return span_ring_bytes_t<GEMM_W_Q4_K>(tn, stages);
     case GEMM_W_Q8_0: return span_ring_bytes_t<GEMM_W_Q8_0>(tn, stages);
@@ -583,7 +587,7 @@ GemmShape pick_gemm(int M, int N, int K, int num_cus, bool precise, int wf, bool
   if (precise) {
     s.tn = N <= 32 ? 1 : 2;
     const long long tiles = (long long)((M + 127) / 128) * ((N + 32 * s.tn - 1) / (32 * s.tn));
-    s.stages = tiles > 2LL * num_cus || (s.tn == 2 && span_ring_bytes(2, 3, wf) > 80 * 1024) ? 2 : 3;
+    s.stages = tiles > 2LL * num_cus || ((s.tn == 2 || wf == GEMM_W_F16_X3) && span_ring_bytes(s.tn, 3, wf) > 80 * 1024) ? 2 : 3;
     const int per_cu = std::max(1, std::min(3, 160 * 1024 / span_ring_bytes(s.tn, s.stages, wf)));
     const long long slots = (long long)per_cu * num_cus;
     while (s.splits < 16 && tiles * (s.splits + 1) <= slots &&
@@ -640,6 +644,7 @@ hipError_t launch_kernel(const GemmArgs& a, const GemmShape& s, bool precise, in
     case GEMM_W_Q4_0: return precise ? gemm_q4_0_span(a, s.tn, s.stages, grid, st) : gemm_q4_0_plane(a, s.tn, s.mt, grid, st);
     case GEMM_W_PACKED: return precise ? gemm_packed_span(a, s.tn, s.stages, grid, st) : gemm_packed_plane(a, s.tn, s.mt, grid, st);
     case GEMM_W_F16: return precise ? gemm_f16_span(a, s.tn, s.stages, grid, st) : hipErrorInvalidValue;
+    case GEMM_W_F16_X3: return precise ? gemm_f16_x3_span(a, s.tn, s.stages, grid, st) : hipErrorInvalidValue;
     case GEMM_W_F32: return precise ? gemm_f32_span(a, s.tn, s.stages, grid, st) : hipErrorInvalidValue;
     case GEMM_W_Q4_K: return precise ? gemm_q4_k_span(a, s.tn, s.stages, grid, st) : gemm_q4_k_plane(a, s.tn, s.mt, grid, st);
     case GEMM_W_Q8_0: return precise ? gemm_q8_0_span(a, s.tn, s.stages, grid, st) : gemm_q8_0_plane(a, s.tn, s.mt, grid, st);
@@ -738,8 +743,9 @@ size_t gemm_workspace_bytes(int M, int N, int K, int num_cus, bool precise, int 
 
 hipError_t gemm_launch(const GemmArgs& a_in, int num_cus, hipStream_t st, int* splits_left) {
   if (a_in.packed < GEMM_W_Q4_0 || a_in.packed >= GEMM_W_COUNT) return hipErrorInvalidValue;
-  if ((a_in.packed == GEMM_W_F16 || a_in.packed == GEMM_W_F32) && !a_in.precise)
+  if ((a_in.packed == GEMM_W_F16 || a_in.packed == GEMM_W_F16_X3 || a_in.packed == GEMM_W_F32) && !a_in.precise)
     return hipErrorInvalidValue;  // float rows only in the span kernel
+  if (a_in.packed == GEMM_W_F16_X3 && (!a_in.xb_ll || !a_in.x32)) return hipErrorInvalidValue;
   const bool blocks = a_in.packed == GEMM_W_Q4_K || a_in.packed == GEMM_W_Q5_K || a_in.packed == GEMM_W_IQ4_XS ||
                       a_in.packed == GEMM_W_Q2_K;
   if (a_in.K <= 0 || a_in.K % (blocks ? 256 : 64) || a_in.M <= 0 || a_in.N <= 0) return hipErrorInvalidValue;
@@ -770,7 +776,7 @@ hipError_t gemm_launch(const GemmArgs& a_in, int num_cus, hipStream_t st, int* s
   }
   const long long work = (long long)((a.M + 3) / 4) * a.N;
   const dim3 rgrid((unsigned)((work + CN_BLOCK - 1) / CN_BLOCK));
-  if (a.x32) hipLaunchKernelGGL((gemm_reduce_kernel<true>), rgrid, dim3(CN_BLOCK), 0, st, a);
+  if (a.packed == GEMM_W_F16_X3) hipLaunchKernelGGL((gemm_reduce_kernel<true>), rgrid, dim3(CN_BLOCK), 0, st, a);
   else hipLaunchKernelGGL((gemm_reduce_kernel<false>), rgrid, dim3(CN_BLOCK), 0, st, a);
   return hipGetLastError();
 }
@@ -786,14 +792,14 @@ hipError_t to_f16_scaled_launch(const float* x, uint16_t* xh, float* xinv, int N
   return hipGetLastError();
 }
 
-hipError_t to_f16_planes_launch(const float* x, uint16_t* xh, uint16_t* xl, float* xinv, int N, int K, hipStream_t st) {
+hipError_t to_f16_planes_launch(const float* x, uint16_t* xp, size_t plane, float* xinv, int N, int K, hipStream_t st) {
   if (N <= 0 || K <= 0 || K % 32 || K > 16384) return hipErrorInvalidValue;
   const int v = (K + 4 * CN_BLOCK - 1) / (4 * CN_BLOCK);  // float4 per thread
   const dim3 grid(N), block(CN_BLOCK);
-  if (v <= 2) hipLaunchKernelGGL((to_f16_planes_kernel<2>), grid, block, 0, st, x, xh, xl, xinv, K);
-  else if (v <= 4) hipLaunchKernelGGL((to_f16_planes_kernel<4>), grid, block, 0, st, x, xh, xl, xinv, K);
-  else if (v <= 8) hipLaunchKernelGGL((to_f16_planes_kernel<8>), grid, block, 0, st, x, xh, xl, xinv, K);
-  else hipLaunchKernelGGL((to_f16_planes_kernel<16>), grid, block, 0, st, x, xh, xl, xinv, K);
+  if (v <= 2) hipLaunchKernelGGL((to_f16_planes_kernel<2>), grid, block, 0, st, x, xp, plane, xinv, K);
+  else if (v <= 4) hipLaunchKernelGGL((to_f16_planes_kernel<4>), grid, block, 0, st, x, xp, plane, xinv, K);
+  else if (v <= 8) hipLaunchKernelGGL((to_f16_planes_kernel<8>), grid, block, 0, st, x, xp, plane, xinv, K);
+  else hipLaunchKernelGGL((to_f16_planes_kernel<16>), grid, block, 0, st, x, xp, plane, xinv, K);
   return hipGetLastError();
 }
 

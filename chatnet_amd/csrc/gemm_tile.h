@@ -62,8 +62,8 @@ __device__ __forceinline__ void write_h(const GemmArgs& a, int n, int j, float v
 }
 
 // Outputs of chatnet_matmul's F16 rows (rows m..m+3 of column n) that came out
-// NaN, summed again from the fp32 x: in two planes an infinite weight meets x's
-// low part too (inf * 0 or inf - inf), where the plain product is infinite.
+// NaN, summed again from the fp32 x: in planes an infinite weight meets x's
+// low parts too (inf * 0 or inf - inf), where the plain product is infinite.
 // Never taken for finite operands.  Only the compensated instances call it (a
 // loop in every instance's epilogue cost the others registers).
 __device__ __forceinline__ void f16_dot_again(const GemmArgs& a, int n, int m, f32x4& v) {
@@ -333,6 +333,7 @@ template <> struct WFmt<GEMM_W_F16> {  // rows of the float type, pieces XOR-swi
   static constexpr int UNIT = 128, WP = 8, SB = 0, MASK = -1, WD = 16;
   static constexpr int OFF[WP] = {0, 16, 32, 48, 64, 80, 96, 112}, STEP[WP] = {};
 };
+template <> struct WFmt<GEMM_W_F16_X3> : WFmt<GEMM_W_F16> {};
 template <> struct WFmt<GEMM_W_F32> {
   static constexpr int UNIT = 256, WP = 16, SB = 0, MASK = -1, WD = 32;
   static constexpr int OFF[WP] = {0, 16, 32, 48, 64, 80, 96, 112, 128, 144, 160, 176, 192, 208, 224, 240}, STEP[WP] = {};
@@ -373,7 +374,9 @@ template <> struct WFmt<GEMM_W_Q2_K> {  // the scales, the half's 32 qs bytes, d
 // Formats read through u8 codes with an fp32 scale and offset per 16 weights,
 // weight = fmaf(code, scale, offset): the values gemm_pack_kernel's units hold.
 template <int WF>
-constexpr bool coded_format() { return WF != GEMM_W_Q4_0 && WF != GEMM_W_F16 && WF != GEMM_W_F32; }
+constexpr bool float_format() { return WF == GEMM_W_F16 || WF == GEMM_W_F16_X3 || WF == GEMM_W_F32; }
+template <int WF>
+constexpr bool coded_format() { return WF != GEMM_W_Q4_0 && !float_format<WF>(); }
 
 // The scales and offsets of a lane's 32 weights of chunk c (first and last 16), and
 // their fifth bits.
@@ -485,11 +488,11 @@ template <bool PRECISE, int TN, int S, int WF, int MT = 1, int WNC = 1>
 struct PipeCfg {
   using F = WFmt<WF>;
   static constexpr int FMT = WF;
-  static constexpr int PL = PRECISE ? 2 : 1;
+  static constexpr int PL = WF == GEMM_W_F16_X3 ? 3 : PRECISE ? 2 : 1;  // x planes
   static constexpr int MTILES = MT;
   static constexpr int WN = WNC, WM = 4 / WNC;  // waves along N and M
   static constexpr int BM = 32 * WM * MT, BN = 32 * TN * WN;
-  static constexpr bool FLT = WF == GEMM_W_F16 || WF == GEMM_W_F32;
+  static constexpr bool FLT = float_format<WF>();
   static constexpr int UNIT = F::UNIT;         // global bytes per row and chunk of 64
   static constexpr int WP = F::WP;             // 16-byte pieces per row and chunk
   static constexpr int WROW = 16 * WP;         // LDS bytes per row and chunk
@@ -551,7 +554,7 @@ struct TileIO {
         const int row = piece >> 3, ch = piece & 7;
         const int n = min(n0 + row, a.N - 1);
         const int logical = ch ^ ((row >> 1) & 7);
-        xsrc[p][j] = (p ? a.xb_lo : a.xb) + (size_t)n * a.K + 8 * logical;
+        xsrc[p][j] = (p == 2 ? a.xb_ll : p ? a.xb_lo : a.xb) + (size_t)n * a.K + 8 * logical;
       }
 #pragma unroll
     for (int j = 0; j < C::WI; j++) {
@@ -712,7 +715,7 @@ struct TileIO {
   }
 
   // Final tiles: K-split partials [splits][N][M] or the epilogue.
-  template <int TN, bool COMP = false>
+  template <int TN>
   __device__ __forceinline__ void store(const GemmArgs& a, const f32x16 (&acc)[TN], const float (&scl)[TN],
                                         int mt = 0) const {
 #pragma unroll
@@ -731,7 +734,7 @@ struct TileIO {
               for (int i = 0; i < 4 && m + i < a.M; i++) p[i] = v[i];
           }
         } else {
-          if constexpr (COMP) f16_dot_again(a, n, m, v);
+          if constexpr (C::FMT == GEMM_W_F16_X3) f16_dot_again(a, n, m, v);
           write_out4(a, a.epi, n, m, v);
         }
       }
@@ -974,12 +977,17 @@ __global__ __launch_bounds__(CN_BLOCK) __attribute__((amdgpu_waves_per_eu(SK ? 2
 // bits for packed units), x = xh + xl to ~2^-22; the dropped Wb*xl term is
 // below 2^-19 relative.
 //
-// COMP (chatnet_matmul's F16 rows): every chunk's eight MFMA steps start from
-// zero and the chunk sums are added with a running compensation (Kahan), so
-// the product rounds no worse than the fp32 GEMV whose place it takes
-// (relative error against float64 at K = 4096: GEMV 1.0e-7, one accumulator
-// 5.9e-7, this 0.8e-7).
-template <int TN, int S, int WF, bool COMP = false>
+// GEMM_W_F16_X3 (chatnet_matmul's F16 rows): x in three planes of 11 bits each, 2^11
+// apart and each in fp16's normal range, so that the fp32 elements down to 2^-28 of
+// their column's largest meet the weights exactly (the planes hold 24 bits down to
+// 2^-38; the matrix cores' sums keep about 2^-52 of the largest element.  Two planes
+// held 22 of the 24 bits, and 2^-39 of the largest at best).  Every chunk's MFMA steps start from zero, the lowest
+// plane's first, and the chunk sums are added with a running compensation (Kahan),
+// so the product rounds no worse than the fp32 GEMV whose place it takes (relative
+// error against float64 at K = 4096: GEMV 1.0e-7, one accumulator 5.9e-7, this
+// 0.86e-7).  The third plane's products and loads cost 2 us of 18 at 24 columns of
+// 4096 x 4096, 65 -> 88 at 512.
+template <int TN, int S, int WF>
 __global__ __launch_bounds__(CN_BLOCK) void gemm_s_kernel(GemmArgs a) {
   using C = PipeCfg<true, TN, S, WF>;
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -991,6 +999,7 @@ __global__ __launch_bounds__(CN_BLOCK) void gemm_s_kernel(GemmArgs a) {
   for (int cc = 0; cc < TN; cc++)
 #pragma unroll
     for (int v = 0; v < 16; v++) acc[cc][v] = 0.f;
+  constexpr bool COMP = WF == GEMM_W_F16_X3;
   f32x16 sum[COMP ? TN : 1], com[COMP ? TN : 1];
   if constexpr (COMP) {
 #pragma unroll
@@ -1040,10 +1049,10 @@ __global__ __launch_bounds__(CN_BLOCK) void gemm_s_kernel(GemmArgs a) {
         }
       };
       if constexpr (COMP) {
-        // the low plane's four products first, while the sum is still 2^-12 of
-        // the chunk's: their rounding then does not count
+        // the lower planes' products first, while the sum is still 2^-11 of the
+        // next one's: their rounding then does not count
 #pragma unroll
-        for (int p = 1; p >= 0; p--)
+        for (int p = 2; p >= 0; p--) {
 #pragma unroll
           for (int s = 0; s < 4; s++) {
             const f16x8 wa =
@@ -1052,6 +1061,11 @@ __global__ __launch_bounds__(CN_BLOCK) void gemm_s_kernel(GemmArgs a) {
             for (int cc = 0; cc < TN; cc++)
               acc[cc] = mma32(wa, __builtin_bit_cast(f16x8, io.xfrag(st, p, s, cc)), acc[cc]);
           }
+          if (p > 0) {
+#pragma unroll
+            for (int cc = 0; cc < TN; cc++) acc[cc] *= 0x1p-11f;
+          }
+        }
 #pragma unroll
         for (int cc = 0; cc < TN; cc++) {
           add_compensated(sum[cc], com[cc], acc[cc]);
@@ -1100,7 +1114,7 @@ __global__ __launch_bounds__(CN_BLOCK) void gemm_s_kernel(GemmArgs a) {
   }
   float sc[TN];
   io.template load_scales<TN>(a, sc);
-  if constexpr (COMP) io.template store<TN, true>(a, sum, sc);
+  if constexpr (COMP) io.template store<TN>(a, sum, sc);
   else io.template store<TN>(a, acc, sc);
 }
 
@@ -1128,19 +1142,16 @@ hipError_t launch_p_ring(const GemmArgs& a, int mt, int grid, hipStream_t st) {
   return launch_p<TN, S, WF, 1>(a, grid, st);
 }
 
-template <int TN, int S, int WF, bool COMP = false>
+template <int TN, int S, int WF>
 hipError_t launch_s(const GemmArgs& a, int grid, hipStream_t st) {
-  if constexpr (WF == GEMM_W_F16 && !COMP) {
-    if (a.x32) return launch_s<TN, S, WF, true>(a, grid, st);
-  }
   constexpr int lds = PipeCfg<true, TN, S, WF>::LDS;
   static_assert(lds <= 160 * 1024, "LDS ring exceeds the CU's 160 KB");
   static std::atomic<uint64_t> lds_done{0};
   if (lds > 64 * 1024) {
-    const hipError_t e = allow_full_lds(reinterpret_cast<const void*>(&gemm_s_kernel<TN, S, WF, COMP>), lds_done);
+    const hipError_t e = allow_full_lds(reinterpret_cast<const void*>(&gemm_s_kernel<TN, S, WF>), lds_done);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL((gemm_s_kernel<TN, S, WF, COMP>), dim3(grid), dim3(CN_BLOCK), lds, st, a);
+  hipLaunchKernelGGL((gemm_s_kernel<TN, S, WF>), dim3(grid), dim3(CN_BLOCK), lds, st, a);
   return hipGetLastError();
 }
 

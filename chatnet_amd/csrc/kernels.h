@@ -126,9 +126,10 @@ hipError_t gemv_float_launch(int qtype, int epi, const GemvArgs& a, int num_cus,
 enum { GEMM_SEG_SINGLE = 0, GEMM_SEG_CONCAT = 1, GEMM_SEG_INTERLEAVE = 2 };
 // How W is stored (GemmArgs::packed): gemm_pack_launch units (any packable
 // type), rows of F16 / F32 values (the span kernel only), or a type's own blocks.
+// GEMM_W_F16_X3: F16 rows against x in three planes (chatnet_matmul).
 enum { GEMM_W_Q4_0 = 0, GEMM_W_PACKED = 1, GEMM_W_F16 = 2, GEMM_W_F32 = 3, GEMM_W_Q4_K = 4, GEMM_W_Q8_0 = 5,
        GEMM_W_Q5_0 = 6, GEMM_W_Q4_1 = 7, GEMM_W_Q5_1 = 8, GEMM_W_IQ4_NL = 9, GEMM_W_Q5_K = 10, GEMM_W_IQ4_XS = 11,
-       GEMM_W_Q2_K = 12, GEMM_W_COUNT = 13 };
+       GEMM_W_Q2_K = 12, GEMM_W_F16_X3 = 13, GEMM_W_COUNT = 14 };
 // The format that reads matrices of `qtype` as they are stored, -1 if there is
 // none (Q3_K, Q6_K, Q8_K and the other IQ types, read as packed units).
 int gemm_stored_format(int qtype, int K);
@@ -142,6 +143,7 @@ struct GemmArgs {
   const uint16_t* xb;     // N x K, row stride K, fp16 in the cn_span_pos order: one plane scaled per
                           // column (one-plane kernel, to_f16_scaled_launch), or the high parts when precise
   const uint16_t* xb_lo;  // precise: fp16 low parts, x = xb + xb_lo
+  const uint16_t* xb_ll;  // GEMM_W_F16_X3: x 2^e = xb + xb_lo 2^-11 + xb_ll 2^-22
   const float* xinv;      // one-plane kernel: per-column 2^-e undoing the scale of xb (nullptr: 1)
   int precise;            // exact-weight two-plane kernel
   const float* x32;       // F16 rows from chatnet_matmul: the fp32 x, read to redo an output that came out NaN
@@ -187,17 +189,18 @@ hipError_t gemm_launch(const GemmArgs& a, int num_cus, hipStream_t st, int* spli
   CN_GEMM_SPAN(f)
 CN_GEMM_FMT(q4_0) CN_GEMM_FMT(packed) CN_GEMM_FMT(q4_k) CN_GEMM_FMT(q8_0) CN_GEMM_FMT(q5_0) CN_GEMM_FMT(q4_1)
 CN_GEMM_FMT(q5_1) CN_GEMM_FMT(iq4_nl) CN_GEMM_FMT(q5_k) CN_GEMM_FMT(iq4_xs) CN_GEMM_FMT(q2_k) CN_GEMM_SPAN(f16)
-CN_GEMM_SPAN(f32)
+CN_GEMM_SPAN(f16_x3) CN_GEMM_SPAN(f32)
 #undef CN_GEMM_FMT
 #undef CN_GEMM_SPAN
 // x [N][K] fp32 -> the one-plane GEMM's input: xh[n] = fp16(x[n] * 2^e_n) in
 // the cn_span_pos order, 2^e_n bringing max|x[n]| into [2^14, 2^15), and
 // xinv[n] = 2^-e_n.  K % 32 == 0, K <= 16384.
 hipError_t to_f16_scaled_launch(const float* x, uint16_t* xh, float* xinv, int N, int K, hipStream_t st);
-// x [N][K] fp32 -> the span kernel's input scaled per column as above: hi + lo
-// fp16 planes of x[n] * 2^e_n (max over the finite |x[n]|), about 2^-24 of each
-// element, and xinv[n] = 2^-e_n.  Infinities stay infinite with lo = 0.
-hipError_t to_f16_planes_launch(const float* x, uint16_t* xh, uint16_t* xl, float* xinv, int N, int K, hipStream_t st);
+// x [N][K] fp32 -> GEMM_W_F16_X3's three fp16 planes, `plane` elements apart at xp:
+// x[n] * 2^e_n = p0 + p1 2^-11 + p2 2^-22 (2^e_n as above, from the largest finite
+// |x[n]|), exact for every element down to 2^-38 of that largest, and xinv[n] =
+// 2^-e_n.  Infinities stay infinite with p1 = p2 = 0.
+hipError_t to_f16_planes_launch(const float* x, uint16_t* xp, size_t plane, float* xinv, int N, int K, hipStream_t st);
 // x[r] += the K-split partials part[0..splits)[r] (summed as the GEMM's reduce
 // does), then xb / xb_lo = RMSNorm(x[r]) * g as the span GEMM's input (fp16 hi
 // + lo planes in the cn_span_pos order); splits 0: the norm alone.  dim % 32

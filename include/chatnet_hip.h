@@ -255,8 +255,8 @@ CHATNET_API int chatnet_get_logits(chatnet_model* m, float* logits_host);
  * with several columns run a multi-column GEMV (each column the N = 1
  * product's exact arithmetic), F16 with more columns than one launch of it
  * holds (8 up to K = 4864, fewer above) an MFMA product of the exact weights
- * with x as two fp16 planes, summed with compensation in fp32 (its error
- * against float64 is the GEMV's, 1e-7).  Q4_1, Q5_0, Q5_1,
+ * with x as three fp16 planes (24 bits), summed with compensation in fp32 (its
+ * error against float64 is the GEMV's, 1e-7).  Q4_1, Q5_0, Q5_1,
  * Q8_0, Q2_K .. Q6_K, IQ4_NL and IQ4_XS run up to 16 columns on their stored
  * blocks (one column, two of a large Q6_K and two or three of a large Q3_K
  * matrix: the fused GEMV per column): Q4_1, Q5_0, Q5_1, Q2_K, IQ4_NL and IQ4_XS

@@ -28,8 +28,8 @@ def float_weights(qtype, M, K, seed):
 @pytest.mark.parametrize("qtype", [F32, F16])
 def test_float_columns_match_float64(qtype, M, K, N):
     """Bar: 32-bit sums in any order, |error| <= K * 2^-24 of sum |w x| at worst
-    (the F16 product's x carries 2^-24 of each element besides); measured about
-    1e-7 of the largest output."""
+    (the F16 product's x is exact down to 2^-28 of its column's largest); measured
+    about 1e-7 of the largest output."""
     announce(f"float columns type={qtype} M={M} K={K} N={N}")
     w = float_weights(qtype, M, K, 5)
     x = synth.normal(6, f"fcx{N}x{K}", N * K, 1.0).reshape(N, K)
@@ -64,6 +64,23 @@ def test_f16_columns_of_other_magnitudes_and_non_finite_values():
         assert np.array_equal(one[~fin & ~np.isnan(one)], y[n][~fin & ~np.isnan(one)]), n
         if fin.any():
             assert normwise(y[n][fin], one[fin]) <= 2e-6, n
+
+
+@pytest.mark.parametrize("M,K,N", [(512, 512, 12), (100, 4096, 40), (64, 11008, 5), (4096, 4096, 70)])
+def test_f16_columns_hold_x_in_fp32(M, K, N):
+    """Against single ones the product is x itself, all 24 bits, also beside an
+    element 2^20 times larger under zero weights; beside one 2^30 times larger, to
+    2^-50 of it (the matrix cores align the terms of a sum to about 2^-52 of the
+    largest operand there)."""
+    announce(f"f16 columns, x exact M={M} K={K} N={N}")
+    at = (np.arange(M) * 7 + 1) % (K - 1) + 1
+    w = np.zeros((M, K), np.float16)
+    w[np.arange(M), at] = 1.0
+    x = synth.normal(57, f"exx{N}x{K}", N * K, 1.0).reshape(N, K)
+    x += np.copysign(np.float32(0.125), x)
+    for big, tol in ((1.0, 0.0), (2.0 ** 20, 0.0), (2.0 ** 30, 2.0 ** -20)):
+        x[:, 0] = big
+        assert np.max(np.abs(gpu_matmul(F16, w.view(np.uint8).ravel(), x, M, K) - x[:, at])) <= tol, big
 
 
 @pytest.mark.parametrize("M,K,N", [(96, 512, 16), (96, 512, 3)])
