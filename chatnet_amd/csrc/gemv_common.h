@@ -19,7 +19,8 @@ __device__ __forceinline__ const int* stop_flag(const GemvArgs& a) { return a.st
 // max M_c, sum L_c and unnormalised output O_c of its positions, and
 //   x = sum_c O_c e^(M_c - M) / sum_c L_c e^(M_c - M),  M = max_c M_c
 // (attn_merge_kernel's combination).  Every chunk's loads are issued (their
-// addresses do not depend on the position); inactive ones are masked.  The
+// addresses do not depend on the position); inactive ones and those without
+// positions have a sum of 0 and are left out, a NaN sum is not.  The
 // weights e^(M_c - M) and the sum depend on the head only: the base-256
 // staging (16-element groups of one head) computes them once per group.
 struct MergeSrc {
@@ -53,13 +54,13 @@ __device__ __forceinline__ float4 merged_x4(const MergeSrc& m, int i) {
     ml[c] = *reinterpret_cast<const float2*>(m.ml + 2 * (base + cc));
     oc[c] = *reinterpret_cast<const float4*>(m.o + (base + cc) * m.hd + d);
     if (c >= m.s_eff) ml[c].y = 0.f;
-    if (ml[c].y > 0.f) M = fmaxf(M, ml[c].x);
+    if (ml[c].y != 0.f) M = fmaxf(M, ml[c].x);
   }
   float L = 0.f;
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
   for (int c = 0; c < NS; c++) {
-    if (ml[c].y > 0.f) {
+    if (ml[c].y != 0.f) {
       const float f = expf(ml[c].x - M);
       L += ml[c].y * f;
       acc.x += oc[c].x * f;
@@ -88,13 +89,13 @@ __device__ __forceinline__ MergeW<NS> merge_weights(const MergeSrc& m, int h) {
   for (int c = 0; c < NS; c++) {  // straight-line loads: chunks past splits re-read the last
     ml[c] = *reinterpret_cast<const float2*>(m.ml + 2 * (base + (c < m.splits ? c : m.splits - 1)));
     if (c >= m.s_eff) ml[c].y = 0.f;
-    if (ml[c].y > 0.f) M = fmaxf(M, ml[c].x);
+    if (ml[c].y != 0.f) M = fmaxf(M, ml[c].x);
   }
   MergeW<NS> w;
   w.L = 0.f;
 #pragma unroll
   for (int c = 0; c < NS; c++) {
-    w.f[c] = ml[c].y > 0.f ? expf(ml[c].x - M) : 0.f;
+    w.f[c] = ml[c].y != 0.f ? expf(ml[c].x - M) : 0.f;
     w.L += ml[c].y * w.f[c];
   }
   return w;

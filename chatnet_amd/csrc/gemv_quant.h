@@ -198,13 +198,13 @@ __device__ __forceinline__ void stage_merge(const MergeSrc& m, const XMerge<MAXT
     for (int c = 0; c < NS; c++) {
       ml[c] = r.ml[j][c];
       if (c >= m.s_eff) ml[c].y = 0.f;
-      if (ml[c].y > 0.f) M = fmaxf(M, ml[c].x);
+      if (ml[c].y != 0.f) M = fmaxf(M, ml[c].x);
     }
     float L = 0.f;
     float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
 #pragma unroll
     for (int c = 0; c < NS; c++) {
-      if (ml[c].y > 0.f) {
+      if (ml[c].y != 0.f) {
         const float f = expf(ml[c].x - M);
         L += ml[c].y * f;
         lo.x += r.lo[j][c].x * f; lo.y += r.lo[j][c].y * f; lo.z += r.lo[j][c].z * f; lo.w += r.lo[j][c].w * f;

@@ -90,3 +90,28 @@ def test_spans_deep_in_the_context_share_their_keys(heads, kv, hd, f16, pos, n):
     h = per_token(cfg, ck, toks[pos:], pos, toks[:pos])
     # each schedule's bound against the oracle, twice that for an fp16 cache
     assert float(np.max(np.abs(g - h))) <= 2 * LOGIT_TOL * (2 if f16 else 1)
+
+
+# The O projection merges the splits' partials: from fp32 records (Q4_1, IQ4_XS),
+# packed units (IQ3_S), F16 and F32 rows.  (The digit types' staging drops a NaN.)
+@pytest.mark.parametrize("seq", [20, 300, 1000])
+@pytest.mark.parametrize("mix", ["legacy_blocks", "iq_a", "iq_b", "f16", "f32"])
+def test_a_nan_key_reaches_the_logits_from_any_split(mix, seq):
+    """A token whose embedding is NaN leaves a NaN key and value at its position;
+    whichever split of the decode attention holds it, later logits are NaN."""
+    announce(f"NaN key, {mix}, {seq} tokens")
+    cfg = SPAN_SMALL.replace(n_layers=1)
+    ck = synth.llama_checkpoint(cfg, seed=67, mix=mix)
+    emb = ck["token_embd.weight"]
+    rows = emb.data.view(np.float32).reshape(cfg.vocab_size, cfg.dim).copy()
+    bad = 7
+    rows[bad] = np.nan
+    ck["token_embd.weight"] = synth.SynthTensor(emb.type, emb.dims, rows.reshape(-1).view(np.uint8))
+    toks = synth.tokens(67, "prompt", seq, cfg.vocab_size)
+    toks[toks == bad] = bad + 1
+    for at in {0, 9, seq // 2, seq - 2}:
+        t = toks.copy()
+        t[at] = bad
+        with HipLlamaModel(cfg, ck) as m:
+            m.forward(t[:-1], 0)
+            assert np.all(np.isnan(m.forward(t[-1:], seq - 1))), at
