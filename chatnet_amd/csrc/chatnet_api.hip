@@ -127,19 +127,25 @@ std::mutex g_enqueue_mu;
 // every launch leaves them zero.
 constexpr size_t kMatmulCounterBytes = (size_t)kGemmTileCounters * sizeof(unsigned);
 
-// With `grown`, a capturing stream whose workspace is too small is no error:
-// *grown is false and the caller runs a path without one.
-int matmul_workspace(int dev, hipStream_t st, size_t bytes, char** out, bool* grown = nullptr) {
+// With `have`, a workspace is a convenience: a capturing stream gets none (*have is
+// false) and the caller runs a path without one.  So a captured call of such a path
+// touches only its operands, whatever ran on the stream before, and its replays need
+// no order against other work on the stream.  (The null stream cannot be captured.)
+int matmul_workspace(int dev, hipStream_t st, size_t bytes, char** out, bool* have = nullptr) {
+  if (have && st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(st, &cs));
+    if (cs != hipStreamCaptureStatusNone) {
+      *have = false;
+      return CHATNET_OK;
+    }
+  }
   std::lock_guard<std::mutex> lk(g_ws_mu);
   auto& e = g_ws[{dev, st}];
   bytes = std::max(bytes, kMatmulCounterBytes);
   if (e.second < bytes) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     HIP_TRY(hipStreamIsCapturing(st, &cs));
-    if (cs != hipStreamCaptureStatusNone && grown) {
-      *grown = false;
-      return CHATNET_OK;
-    }
     if (cs != hipStreamCaptureStatusNone)
       return fail(CHATNET_ERR_INVALID_ARG,
                   "chatnet_matmul: the stream is capturing and its workspace (%zu bytes) is smaller than the %zu "
@@ -1141,7 +1147,7 @@ int run_prompt(chatnet_model* m, const int32_t* tokens, int n, int position) {
 // launches).  At 8 columns that one GEMV launch holds the two take 20.5 and 19.8 us
 // for 4096 x 4096, 8.1 and 17.3 for 2048 x 2048, 51.7 and 27.4 for 11008 x 4096:
 // the line lies where the GEMV's bits end, not where the product is faster.  F32, a
-// capturing stream whose workspace is too small and the no-allocation variant
+// capturing stream and the no-allocation variant
 // (which takes these types without scratch, so overlapping calls are safe) run
 // the multi-column GEMV for any N.
 int matmul_float(int type, const void* w, const float* x, float* y, int M, int K, int N, int dev, int cus,

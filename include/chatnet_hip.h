@@ -273,9 +273,11 @@ CHATNET_API int chatnet_get_logits(chatnet_model* m, float* logits_host);
  * on a stream under HIP graph capture cannot allocate: it fails with
  * CHATNET_ERR_INVALID_ARG if the stream's workspace is too small, so a
  * capturing caller first makes one uncaptured call of the largest size, or
- * uses chatnet_matmul_noalloc.  `stream` is a hipStream_t (NULL = default
- * stream).  F16 rows need no workspace there: their
- * calls then run the multi-column GEMV.  Asynchronous on `stream`. */
+ * uses chatnet_matmul_noalloc.  A captured GEMM's replays use that workspace
+ * too: they must be ordered with other chatnet_matmul work of the capturing
+ * stream.  F16 rows and the up-to-16-column products use none when captured
+ * (F16: the multi-column GEMV).  `stream` is a hipStream_t (NULL = default
+ * stream).  Asynchronous on `stream`. */
 CHATNET_API int chatnet_matmul(uint32_t ggml_type, const void* w_dev, const float* x_dev,
                    float* y_dev, int M, int K, int N, void* stream);
 
