@@ -115,23 +115,35 @@ const void* embed_w(const DevTensor& t) { return embed_raw_type(t.type) ? t.ptr 
 // a graph the caller captured earlier may still read it.  Growing needs a
 // hipMalloc, which a stream under capture cannot take: a capturing caller gets
 // an error unless an uncaptured call of the same or a larger size came first.
-std::mutex g_ws_mu;
-std::map<std::pair<int, hipStream_t>, std::pair<char*, size_t>> g_ws;
-std::vector<char*> g_ws_retired;
-// Held while a call enqueues the launches that share its stream's workspace, so
-// that calls from several threads on one stream do not interleave them.
-std::mutex g_enqueue_mu;
+struct Workspace {
+  // Held from the growth until the last launch that uses it is enqueued, so that
+  // calls from several threads on one stream do not interleave their launches;
+  // other streams have workspaces, and locks, of their own.
+  std::mutex mu;
+  char* p = nullptr;
+  size_t bytes = 0;
+  std::vector<char*> retired;
+};
+std::mutex g_ws_mu;  // the map's; a Workspace in it stays where it is
+std::map<std::pair<int, hipStream_t>, Workspace> g_ws;
+Workspace& workspace_of(int dev, hipStream_t st) {
+  std::lock_guard<std::mutex> lk(g_ws_mu);
+  return g_ws[{dev, st}];
+}
 
 // The first kMatmulCounterBytes of a stream's workspace are the one-plane
 // GEMM's stream-K tile counters: zeroed when the workspace is allocated, and
 // every launch leaves them zero.
 constexpr size_t kMatmulCounterBytes = (size_t)kGemmTileCounters * sizeof(unsigned);
 
-// With `have`, a workspace is a convenience: a capturing stream gets none (*have is
-// false) and the caller runs a path without one.  So a captured call of such a path
-// touches only its operands, whatever ran on the stream before, and its replays need
-// no order against other work on the stream.  (The null stream cannot be captured.)
-int matmul_workspace(int dev, hipStream_t st, size_t bytes, char** out, bool* have = nullptr) {
+// At least `bytes` of `st`'s workspace, its lock taken into `lk` for the caller to
+// hold over its launches.  With `have`, a workspace is a convenience: a capturing
+// stream gets none (*have is false) and the caller runs a path without one.  So a
+// captured call of such a path touches only its operands, whatever ran on the
+// stream before, and its replays need no order against other work on the stream.
+// (The null stream cannot be captured.)
+int matmul_workspace(int dev, hipStream_t st, size_t bytes, char** out, std::unique_lock<std::mutex>& lk,
+                     bool* have = nullptr) {
   if (have && st) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     HIP_TRY(hipStreamIsCapturing(st, &cs));
@@ -140,17 +152,17 @@ int matmul_workspace(int dev, hipStream_t st, size_t bytes, char** out, bool* ha
       return CHATNET_OK;
     }
   }
-  std::lock_guard<std::mutex> lk(g_ws_mu);
-  auto& e = g_ws[{dev, st}];
+  Workspace& e = workspace_of(dev, st);
+  lk = std::unique_lock<std::mutex>(e.mu);
   bytes = std::max(bytes, kMatmulCounterBytes);
-  if (e.second < bytes) {
+  if (e.bytes < bytes) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     HIP_TRY(hipStreamIsCapturing(st, &cs));
     if (cs != hipStreamCaptureStatusNone)
       return fail(CHATNET_ERR_INVALID_ARG,
                   "chatnet_matmul: the stream is capturing and its workspace (%zu bytes) is smaller than the %zu "
                   "this call needs; make one uncaptured call of this size first, or use chatnet_matmul_noalloc",
-                  e.second, bytes);
+                  e.bytes, bytes);
     char* p = nullptr;
     if (hipMalloc((void**)&p, bytes) != hipSuccess)
       return fail(CHATNET_ERR_OUT_OF_MEMORY, "hipMalloc of %zu bytes (matmul workspace) failed", bytes);
@@ -159,10 +171,11 @@ int matmul_workspace(int dev, hipStream_t st, size_t bytes, char** out, bool* ha
       (void)hipFree(p);
       return fail(CHATNET_ERR_HIP, "hipMemsetAsync of the matmul workspace's counters: %s", hipGetErrorString(z));
     }
-    if (e.first) g_ws_retired.push_back(e.first);
-    e = {p, bytes};
+    if (e.p) e.retired.push_back(e.p);
+    e.p = p;
+    e.bytes = bytes;
   }
-  *out = e.first;
+  *out = e.p;
   return CHATNET_OK;
 }
 
@@ -1153,13 +1166,13 @@ int run_prompt(chatnet_model* m, const int32_t* tokens, int n, int position) {
 int matmul_float(int type, const void* w, const float* x, float* y, int M, int K, int N, int dev, int cus,
                  hipStream_t st, bool noalloc) {
   if (type == CHATNET_GGML_F16 && N >= 4 && N > gemv_float_cols_max(K) && !noalloc) {
-    std::lock_guard<std::mutex> lk(g_enqueue_mu);
+    std::unique_lock<std::mutex> lk;
     const size_t plane = ((size_t)N * K * sizeof(uint16_t) + 255) & ~(size_t)255;
     const size_t scales = ((size_t)N * sizeof(float) + 255) & ~(size_t)255;
     const size_t part = gemm_workspace_bytes(M, N, K, cus, true, GEMM_W_F16_X3);
     char* ws = nullptr;
     bool ok = true;
-    const int rc = matmul_workspace(dev, st, kMatmulCounterBytes + 3 * plane + scales + part, &ws, &ok);
+    const int rc = matmul_workspace(dev, st, kMatmulCounterBytes + 3 * plane + scales + part, &ws, lk, &ok);
     if (rc) return rc;
     if (ok) {
       uint16_t* xh = (uint16_t*)(ws + kMatmulCounterBytes);
@@ -1249,7 +1262,7 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
                        (type == CHATNET_GGML_Q4_0 || ahead || (!noalloc && gemm_pack_supports((int)type, K)));
   const bool pack = must_pack || (batched && stored < 0);
   const uint8_t* wp = (const uint8_t*)w_dev;
-  std::unique_lock<std::mutex> lk(g_enqueue_mu, std::defer_lock);
+  std::unique_lock<std::mutex> lk;  // the stream's workspace
   if (batched || pack || (noalloc && ahead)) {
     // [stream-K tile counters | fp16 x | per-column x scales | K-split or
     // stream-K partials | packed W]: the counters in the per-stream workspace
@@ -1264,7 +1277,6 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
     const size_t need = xb_bytes + part_bytes + pack_bytes;
     char* ws = nullptr;
     int rc;
-    if (batched || pack) lk.lock();
     if (noalloc) {
       if (need > kNoAllocScratchBytes)
         return fail(CHATNET_ERR_INVALID_ARG,
@@ -1272,7 +1284,7 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
                     need, kNoAllocScratchBytes);
       rc = noalloc_scratch(dev, &ws);
     } else {
-      rc = matmul_workspace(dev, st, need, &ws);
+      rc = matmul_workspace(dev, st, need, &ws, lk);
     }
     if (rc) return rc;
     if (pack) {
@@ -1310,9 +1322,8 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
     const size_t need = noalloc ? 0 : gemv_qcols_workspace((int)type, M, K, N, cus);
     char* ws = nullptr;
     if (need) {
-      lk.lock();
       bool ok = true;
-      const int rc = matmul_workspace(dev, st, kMatmulCounterBytes + need, &ws, &ok);
+      const int rc = matmul_workspace(dev, st, kMatmulCounterBytes + need, &ws, lk, &ok);
       if (rc) return rc;
       ws = ok ? ws + kMatmulCounterBytes : nullptr;
     }

@@ -2,6 +2,8 @@
 dequantized weights, at the edges of each path: a few columns in one launch
 (multi-column GEMV), the matrix-core paths from 8 columns on, non-finite
 values, a capturing stream and the no-allocation variant."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -333,6 +335,50 @@ def test_few_columns_captured_without_a_workspace_and_noalloc(qtype, M, same_ord
     del graph
     for b in (w_d, x_d, y_d):
         b.free()
+
+
+def test_threads_on_shared_and_own_streams():
+    """Four threads, two of them on one stream, each with products that use and grow
+    the stream's workspace (a packing pass, K splits, F16 planes, K shares, x staged
+    ahead): every result is the single call's."""
+    announce("threads, shared and own streams")
+    work = []
+    for i, (qtype, M, K, N) in enumerate([(14, 300, 2048, 40), (F16, 512, 512, 24), (12, 96, 4096, 9), (8, 2100, 4096, 12),
+                                          (12, 1000, 4096, 100), (18, 200, 512, 3)]):
+        w = float_weights(qtype, M, K, 60).view(np.uint8).ravel() if qtype == F16 else synth.tensor(qtype, 60 + i, "thr", M, K).data
+        x = synth.normal(61 + i, "thrx", N * K, 1.0).reshape(N, K)
+        work.append((qtype, M, K, N, gpu_matmul(qtype, w, x, M, K), hiprt.DeviceBuffer.from_numpy(w, pad=256),
+                     hiprt.DeviceBuffer.from_numpy(x)))
+    shared = hiprt.Stream()
+    streams = [shared, shared, hiprt.Stream(), hiprt.Stream()]
+    outs = [[[hiprt.DeviceBuffer(4 * c[1] * c[3]) for c in work] for _ in range(3)] for _ in streams]
+    errors = []
+
+    def run(t):
+        try:
+            for r in range(3):
+                for i in range(len(work)):
+                    j = (i + t) % len(work)
+                    qtype, M, K, N, _, w_d, x_d = work[j]
+                    ops.matmul_ptr(qtype, w_d.ptr, x_d.ptr, outs[t][r][j].ptr, M, K, N, streams[t].h)
+        except Exception as e:  # reported below, in the test's own thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=run, args=(t,)) for t in range(len(streams))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    hiprt.synchronize()
+    assert not errors, errors
+    for per_thread in outs:
+        for per_round in per_thread:
+            for c, y in zip(work, per_round):
+                assert np.array_equal(y.to_numpy(np.float32, c[1] * c[3]).reshape(c[3], c[1]), c[4])
+                y.free()
+    for c in work:
+        c[5].free()
+        c[6].free()
 
 
 # Types whose GEMM reads the stored blocks: 32-, 64- and 128-column tiles, one
