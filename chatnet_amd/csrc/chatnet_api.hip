@@ -141,9 +141,14 @@ constexpr size_t kMatmulCounterBytes = (size_t)kGemmTileCounters * sizeof(unsign
 // stream gets none (*have is false) and the caller runs a path without one.  So a
 // captured call of such a path touches only its operands, whatever ran on the
 // stream before, and its replays need no order against other work on the stream.
-// (The null stream cannot be captured.)
+// (The null stream cannot be captured.)  Nor does hipStreamPerThread get one: its
+// handle means another stream in every thread.
 int matmul_workspace(int dev, hipStream_t st, size_t bytes, char** out, std::unique_lock<std::mutex>& lk,
                      bool* have = nullptr) {
+  if (have && st == hipStreamPerThread) {
+    *have = false;
+    return CHATNET_OK;
+  }
   if (have && st) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     HIP_TRY(hipStreamIsCapturing(st, &cs));

@@ -322,6 +322,10 @@ def test_few_columns_captured_without_a_workspace_and_noalloc(qtype, M, same_ord
     alone = y_d.to_numpy(np.float32, N * M).reshape(N, M)
     assert np.all(np.abs(alone - ref) <= bound)
     y_d.fill(0xFF)
+    ops.matmul_ptr(qtype, w_d.ptr, x_d.ptr, y_d.ptr, M, K, N, 2)  # hipStreamPerThread: one handle, many streams
+    hiprt.synchronize()
+    assert np.array_equal(y_d.to_numpy(np.float32, N * M).reshape(N, M), alone)
+    y_d.fill(0xFF)
     ops.matmul_ptr(qtype, w_d.ptr, x_d.ptr, y_d.ptr, M, K, N, stream.h)  # the stream has a workspace
     stream.synchronize()
     assert np.array_equal(y_d.to_numpy(np.float32, N * M).reshape(N, M), ref)
