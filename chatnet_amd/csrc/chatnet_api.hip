@@ -137,9 +137,9 @@ Workspace& workspace_of(int dev, hipStream_t st) {
 constexpr size_t kMatmulCounterBytes = (size_t)kGemmTileCounters * sizeof(unsigned);
 
 // At least `bytes` of `st`'s workspace, its lock taken into `lk` for the caller to
-// hold over its launches.  With `have`, a workspace is a convenience: a capturing
-// stream gets none (*have is false) and the caller runs a path without one.  So a
-// captured call of such a path touches only its operands, whatever ran on the
+// hold over its launches.  With `have`, a workspace is a convenience: where memory
+// for it cannot be had, and on a capturing stream, there is none (*have is false)
+// and the caller runs a path without one.  So a captured call of such a path touches only its operands, whatever ran on the
 // stream before, and its replays need no order against other work on the stream.
 // (The null stream cannot be captured.)  Nor does hipStreamPerThread get one: its
 // handle means another stream in every thread.
@@ -169,8 +169,14 @@ int matmul_workspace(int dev, hipStream_t st, size_t bytes, char** out, std::uni
                   "this call needs; make one uncaptured call of this size first, or use chatnet_matmul_noalloc",
                   e.bytes, bytes);
     char* p = nullptr;
-    if (hipMalloc((void**)&p, bytes) != hipSuccess)
+    if (hipMalloc((void**)&p, bytes) != hipSuccess) {
+      (void)hipGetLastError();  // else the next launch reports it
+      if (have) {
+        *have = false;
+        return CHATNET_OK;
+      }
       return fail(CHATNET_ERR_OUT_OF_MEMORY, "hipMalloc of %zu bytes (matmul workspace) failed", bytes);
+    }
     const hipError_t z = hipMemsetAsync(p, 0, kMatmulCounterBytes, st);
     if (z != hipSuccess) {
       (void)hipFree(p);

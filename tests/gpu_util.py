@@ -1,4 +1,6 @@
 """Shared helpers of the GPU tests (device buffers through chatnet_amd.hiprt)."""
+import os
+import subprocess
 import sys
 
 import numpy as np
@@ -33,6 +35,36 @@ def gpu_matmul(qtype: int, w_bytes: np.ndarray, x: np.ndarray, M: int, K: int) -
     for b in (w_d, x_d, y_d):
         b.free()
     return y
+
+
+# hipMalloc as the library sees it: found before the runtime's where this is loaded
+# first and globally.
+_FAILING_MALLOC = """
+#define _GNU_SOURCE
+#include <dlfcn.h>
+unsigned long limit = ~0ul;
+int hipMalloc(void** p, unsigned long n) {
+  void* rt = dlopen("libamdhip64.so.7", RTLD_NOW | RTLD_NOLOAD);
+  return n > limit ? 2 : ((int (*)(void**, unsigned long))dlsym(rt, "hipMalloc"))(p, n);
+}
+"""
+_LOAD_FIRST = """
+import ctypes, sys
+_shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+def malloc_limit(n):
+    ctypes.c_ulong.in_dll(_shim, "limit").value = n
+"""
+
+
+def run_with_failing_malloc(tmp_path, program: str) -> None:
+    """Runs the program in a process of its own, where malloc_limit(n) makes the
+    library's hipMalloc report no memory above n bytes; it must end well."""
+    (tmp_path / "m.c").write_text(_FAILING_MALLOC)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", tmp_path / "m.so", tmp_path / "m.c", "-ldl"], check=True)
+    r = subprocess.run([sys.executable, "-c", _LOAD_FIRST + program, tmp_path / "m.so"], capture_output=True, text=True,
+                       cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))), timeout=100)
+    print(r.stdout, r.stderr[-2000:], flush=True)
+    assert r.returncode == 0
 
 
 # Greedy-identity results of the GPU tests, printed in pytest's terminal

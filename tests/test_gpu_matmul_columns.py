@@ -9,7 +9,7 @@ import pytest
 
 import oracle
 from chatnet_amd import _native, hiprt, ops, synth
-from gpu_util import announce, gpu_matmul, normwise
+from gpu_util import announce, gpu_matmul, normwise, run_with_failing_malloc
 
 pytestmark = pytest.mark.gpu
 
@@ -339,6 +339,34 @@ def test_few_columns_captured_without_a_workspace_and_noalloc(qtype, M, same_ord
     del graph
     for b in (w_d, x_d, y_d):
         b.free()
+
+
+WITHOUT_MEMORY = """
+import numpy as np
+from chatnet_amd import _native, hiprt, ops, synth
+lib = _native.hip_lib()
+malloc_limit(1024)
+for qtype, M, K, N in [(1, 96, 512, 16), (12, 96, 4096, 9), (8, 2100, 4096, 12), (12, 96, 512, 40)]:
+    print("[gpu-case] no memory for a workspace", qtype, M, K, N, flush=True)
+    w = (synth.normal(70, "w", M * K, 0.05).astype(np.float16).view(np.uint8) if qtype == 1
+         else synth.tensor(qtype, 70, "w", M, K).data)
+    w_d = hiprt.DeviceBuffer.from_numpy(w, pad=256)
+    x_d = hiprt.DeviceBuffer.from_numpy(synth.normal(71, "x", N * K, 1.0))
+    y, z = hiprt.DeviceBuffer(4 * N * M), hiprt.DeviceBuffer(4 * N * M)
+    y.fill(0xFF)
+    rc = lib.chatnet_matmul(qtype, w_d.ptr, x_d.ptr, y.ptr, M, K, N, None)
+    assert rc == (0 if N <= 16 else _native.ERR_OUT_OF_MEMORY), rc  # the GEMM has no other path
+    if rc == 0:
+        _native.check(lib.chatnet_matmul_noalloc(qtype, w_d.ptr, x_d.ptr, z.ptr, M, K, N, None))
+        hiprt.synchronize()
+        assert np.array_equal(y.to_numpy(np.uint32, N * M), z.to_numpy(np.uint32, N * M))
+"""
+
+
+def test_without_memory_for_a_workspace(tmp_path):
+    """Products that only gain by a workspace run without one where its allocation
+    fails, with the no-allocation variant's bits; the GEMM reports the failure."""
+    run_with_failing_malloc(tmp_path, WITHOUT_MEMORY)
 
 
 def test_threads_on_shared_and_own_streams():
