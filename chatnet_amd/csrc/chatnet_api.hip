@@ -956,15 +956,25 @@ int ensure_span_buffers(chatnet_model* m) {
   return CHATNET_OK;
 }
 
-// At least `need` bytes at sp_part, which the stream's kernels use in turn.
-int span_part(chatnet_model* m, size_t need) {
+// At least `need` bytes at sp_part, which the stream's kernels use in turn.  Where
+// they cannot be had beside the present ones: with `have`, *have is false and the
+// present ones stay; else they are given up first.
+int span_part(chatnet_model* m, size_t need, bool* have = nullptr) {
   if (need <= m->sp_part_bytes) return CHATNET_OK;
+  void* p = nullptr;
+  bool ok = hipMalloc(&p, need) == hipSuccess;
+  if (!ok) (void)hipGetLastError();  // else the next launch reports it
+  if (!ok && have) {
+    *have = false;
+    return CHATNET_OK;
+  }
   HIP_TRY(hipStreamSynchronize(m->stream));
   if (m->sp_part) (void)hipFree(m->sp_part);
   m->sp_part = nullptr;
   m->sp_part_bytes = 0;
-  if (hipMalloc(&m->sp_part, need) != hipSuccess)
+  if (!ok && hipMalloc(&p, need) != hipSuccess)
     return fail(CHATNET_ERR_OUT_OF_MEMORY, "hipMalloc of %zu bytes failed", need);
+  m->sp_part = (float*)p;
   m->sp_part_bytes = need;
   return CHATNET_OK;
 }
@@ -1070,7 +1080,9 @@ int run_span(chatnet_model* m, const int32_t* tokens, int n, int position, const
       at.scale = 1.0f / sqrtf((float)c.head_dim);  // LlamaModel.cs:248
       // the QKV GEMM's partials at sp_part are read by now (RoPE, in stream order)
       at.splits = attn_prefill_splits(cn, p0, c.n_heads, at.kv_mul, m->num_cus);
-      if ((rc = span_part(m, attn_prefill_workspace(cn, c.n_heads, c.head_dim, at.splits)))) return rc;
+      bool have = true;
+      if ((rc = span_part(m, attn_prefill_workspace(cn, c.n_heads, c.head_dim, at.splits), &have))) return rc;
+      if (!have) at.splits = 1;
       at.part = m->sp_part;
       HIP_TRY(attn_prefill_launch(at, st));
 

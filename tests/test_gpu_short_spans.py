@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from chatnet_amd import QWEN2_0_5B, HipLlamaModel, _native, synth
-from gpu_util import announce
+from gpu_util import announce, run_with_failing_malloc
 from test_gpu_model import LOGIT_TOL, SPAN_SMALL, span_case
 
 pytestmark = pytest.mark.gpu
@@ -115,3 +115,33 @@ def test_a_nan_key_reaches_the_logits_from_any_split(mix, seq):
         with HipLlamaModel(cfg, ck) as m:
             m.forward(t[:-1], 0)
             assert np.all(np.isnan(m.forward(t[-1:], seq - 1))), at
+
+
+SHARED_KEYS_WITHOUT_MEMORY = """
+import os
+import numpy as np
+from chatnet_amd import HipLlamaModel, TINY_TEST, synth
+cfg = TINY_TEST.replace(n_layers=2, dim=256, hidden_dim=512, n_heads=2, n_kv_heads=1, head_dim=128, context_length=2048)
+ck = synth.llama_checkpoint(cfg, seed=68, mix="q4_0")
+toks = synth.tokens(68, "prompt", 1512, cfg.vocab_size)
+def run(limit):
+    print("[gpu-case] shared keys, allocation limit", limit, flush=True)
+    with HipLlamaModel(cfg, ck) as m:
+        m.forward(toks[:12], 0)  # the span buffers and the GEMMs' partials
+        os.environ["CHATNET_SPAN_BATCH"] = "0"
+        m.forward(toks[12:1500], 12)
+        del os.environ["CHATNET_SPAN_BATCH"]
+        malloc_limit(limit)
+        g = m.forward(toks[1500:], 1500).copy()
+        malloc_limit(2 ** 62)
+        return g
+a, b = run(2 ** 62), run(1024)
+assert np.all(np.isfinite(b)) and np.max(np.abs(a - b)) <= 1e-4, np.max(np.abs(a - b))
+assert not np.array_equal(a, b)  # one share a row sums in another order
+"""
+
+
+def test_spans_without_memory_for_key_shares(tmp_path):
+    """A span whose keys would be shared runs without shares where their partial
+    results have no memory."""
+    run_with_failing_malloc(tmp_path, SHARED_KEYS_WITHOUT_MEMORY)
