@@ -661,8 +661,6 @@ hipError_t launch_kernel(const GemmArgs& a, const GemmShape& s, bool precise, in
 
 }  // namespace
 
-bool gemm_supports(int qtype, int K) { return qtype == 2 && K > 0 && K % 64 == 0; }
-
 int gemm_stored_format(int qtype, int K) {
   if (K <= 0 || K % 64) return -1;
   const bool sb = K % 256 == 0;

@@ -163,7 +163,6 @@ struct GemmArgs {
 };
 // Arrival counters a stream-K launch may use (one per tile).
 constexpr int kGemmTileCounters = 1024;
-bool gemm_supports(int qtype, int K);
 // Packed weights: every 64 weights of a row become one 96-byte unit of 64 u8
 // codes, 4 fp32 scales and 4 fp32 offsets (one pair per 16 weights), with
 // weight k = fmaf(code[k], scale[k/16], offset[k/16]) equal to the block

@@ -283,21 +283,21 @@ CHATNET_API int chatnet_matmul(uint32_t ggml_type, const void* w_dev, const floa
 
 /* chatnet_matmul without any allocation, for callers that cannot allocate
  * device memory: code under HIP graph capture, tight serving loops, harnesses
- * that forbid hipMalloc.  No counterpart in the reference.  Same arguments,
- * kernels and results as chatnet_matmul for Q4_0, Q4_1, Q5_0, Q5_1, Q2_K,
- * Q8_K and the IQ types (Q8_K's and the re-encoded IQ types' copy of W,
- * M*(K/64)*96 bytes, goes into the scratch; the size limit below counts such a
- * copy for each of these types but Q4_0), except
- * that it runs no stream-K launch: where chatnet_matmul shares tiles it runs
- * the plain tile grid, the same product summed in another order.  Q8_0,
- * Q3_K, Q4_K, Q5_K and Q6_K run the fused GEMV once per column on their stored
- * blocks, F32 and F16 the multi-column GEMV, without scratch.  The scratch (fp16 x, its per-column scales, the K-split partials
- * and the packed W) lives
- * in a fixed 64 MiB array per device, held by the library from load to
- * process exit, instead of a per-stream workspace.  Calls needing more
- * scratch than that (N*K*2 bytes of x for N >= 8 and N*4 bytes of scales,
- * each rounded up to 256, plus the partials, plus the packed W) fail with CHATNET_ERR_INVALID_ARG before
- * launching anything.  Every call on one device shares that device's array:
+ * that forbid hipMalloc.  No counterpart in the reference.  Same arguments and
+ * kernels as chatnet_matmul for Q4_0, Q4_1, Q5_0, Q5_1, Q2_K, Q8_K and the IQ
+ * types (Q8_K's and the re-encoded IQ types' copy of W, M*(K/64)*96 bytes, goes
+ * into the scratch; the size limit below counts such a copy for each of these
+ * types but Q4_0), except that it runs no stream-K launch and shares no K out:
+ * where chatnet_matmul does it runs the plain grid, the same product summed in
+ * another order.  Q8_0, Q3_K, Q4_K, Q5_K and Q6_K run the up-to-16-column product
+ * of their stored blocks in groups of columns, F32 and F16 the multi-column
+ * GEMV, for any N and without scratch.  The scratch (fp16 x, its per-column
+ * scales, the K-split partials and the packed W) lives in a fixed 64 MiB array
+ * per device, held by the library from load to process exit, instead of a
+ * per-stream workspace.  Calls needing more scratch than that (N*K*2 bytes of x
+ * where the GEMM runs and N*4 bytes of scales, each rounded up to 256, plus the
+ * partials, plus the packed W or its count) fail with CHATNET_ERR_INVALID_ARG
+ * before launching anything.  Every call on one device shares that device's array:
  * calls that may overlap on one device (different streams, threads) race and
  * must be serialized by the caller. */
 CHATNET_API int chatnet_matmul_noalloc(uint32_t ggml_type, const void* w_dev, const float* x_dev,
