@@ -871,7 +871,7 @@ LayerMats layer_mats(Layer& L) { return {{&L.wq, &L.wk, &L.wv, &L.wo, &L.wg, &L.
 // O, gate/up, down): F16 and F32 matrices as their own rows (GEMM_W_F16 /
 // GEMM_W_F32), block types from their stored blocks when every matrix of that
 // GEMM in every layer has one type that has such a format
-// (gemm_stored_format), else as packed units (block types mixed freely, made
+// (gemm_span_format), else as packed units (block types mixed freely, made
 // once per model).  The matrices one GEMM concatenates (q|k|v) or interleaves
 // (gate/up) must share a class (float type or block type); a span whose layers
 // cannot (ffn_gate Q4_0 with ffn_up F16, a type neither packable nor float)
@@ -908,7 +908,7 @@ SpanPlan span_plan(chatnet_model* m, int n) {
       int& g = gcls[gi];
       if (g == 0) g = k;
       else if (g != k) return p;
-      const int f = gemm_stored_format((int)t->type, (int)t->ne0);
+      const int f = gemm_span_format((int)t->type, (int)t->ne0);
       if (fmt[gi] == -2) fmt[gi] = f;
       else if (fmt[gi] != f) fmt[gi] = -1;
     }

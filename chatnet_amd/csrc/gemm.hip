@@ -572,9 +572,7 @@ int span_ring_bytes(int tn, int stages, int wf) {
     case GEMM_W_Q4_1: return span_ring_bytes_t<GEMM_W_Q4_1>(tn, stages);
     case GEMM_W_Q5_1: return span_ring_bytes_t<GEMM_W_Q5_1>(tn, stages);
     case GEMM_W_IQ4_NL: return span_ring_bytes_t<GEMM_W_IQ4_NL>(tn, stages);
-    case GEMM_W_Q5_K: return span_ring_bytes_t<GEMM_W_Q5_K>(tn, stages);
     case GEMM_W_IQ4_XS: return span_ring_bytes_t<GEMM_W_IQ4_XS>(tn, stages);
-    case GEMM_W_Q2_K: return span_ring_bytes_t<GEMM_W_Q2_K>(tn, stages);
     default: return span_ring_bytes_t<GEMM_W_Q4_0>(tn, stages);
   }
 }
@@ -652,9 +650,9 @@ hipError_t launch_kernel(const GemmArgs& a, const GemmShape& s, bool precise, in
     case GEMM_W_Q4_1: return precise ? gemm_q4_1_span(a, s.tn, s.stages, grid, st) : gemm_q4_1_plane(a, s.tn, s.mt, grid, st);
     case GEMM_W_Q5_1: return precise ? gemm_q5_1_span(a, s.tn, s.stages, grid, st) : gemm_q5_1_plane(a, s.tn, s.mt, grid, st);
     case GEMM_W_IQ4_NL: return precise ? gemm_iq4_nl_span(a, s.tn, s.stages, grid, st) : gemm_iq4_nl_plane(a, s.tn, s.mt, grid, st);
-    case GEMM_W_Q5_K: return precise ? gemm_q5_k_span(a, s.tn, s.stages, grid, st) : gemm_q5_k_plane(a, s.tn, s.mt, grid, st);
+    case GEMM_W_Q5_K: return precise ? hipErrorInvalidValue : gemm_q5_k_plane(a, s.tn, s.mt, grid, st);
     case GEMM_W_IQ4_XS: return precise ? gemm_iq4_xs_span(a, s.tn, s.stages, grid, st) : gemm_iq4_xs_plane(a, s.tn, s.mt, grid, st);
-    case GEMM_W_Q2_K: return precise ? gemm_q2_k_span(a, s.tn, s.stages, grid, st) : gemm_q2_k_plane(a, s.tn, s.mt, grid, st);
+    case GEMM_W_Q2_K: return precise ? hipErrorInvalidValue : gemm_q2_k_plane(a, s.tn, s.mt, grid, st);
     default: return hipErrorInvalidValue;
   }
 }
@@ -679,6 +677,20 @@ int gemm_stored_format(int qtype, int K) {
     case 23: return sb ? GEMM_W_IQ4_XS : -1;
     default: return -1;
   }
+}
+
+// The span kernel is bound by VALU instructions, of which packed units take the
+// fewest, and at 2.3 to 3.4 times the bytes the stored blocks win where those are
+// cheap to unpack.  Q5_K and Q2_K are not (layers of a 7B shape, packed and stored,
+// us: Q5_K 512 tokens 876 and 937, 64 230 and 238; of a 1.1B shape, 3 layers, 748 and
+// 786, 64 294 and 341; Q2_K 857 and 986, 734 and 823); IQ4 is for rows of 4096 and
+// more (IQ4_XS, 7B shape, 200 tokens 532 and 488, 16 185 and 176) and below 2048,
+// where K splits go deeper (IQ4_NL, K = 896, 64 tokens 381 and 303), but not between
+// (1.1B shape, 512 tokens 759 and 739, 64 292 and 311, 16 249 and 269).
+int gemm_span_format(int qtype, int K) {
+  if (qtype == 10 || qtype == 13) return -1;
+  if ((qtype == 20 || qtype == 23) && K >= 2048 && K < 4096) return -1;
+  return gemm_stored_format(qtype, K);
 }
 
 bool gemm_pack_supports(int qtype, int K) {

@@ -4,7 +4,3 @@
 hipError_t gemm_q2_k_plane(const GemmArgs& a, int tn, int mt, int grid, hipStream_t st) {
   return launch_one_plane<GEMM_W_Q2_K>(a, tn, mt, grid, st);
 }
-
-hipError_t gemm_q2_k_span(const GemmArgs& a, int tn, int stages, int grid, hipStream_t st) {
-  return launch_span<GEMM_W_Q2_K>(a, tn, stages, grid, st);
-}

@@ -611,13 +611,6 @@ struct TileIO {
     if constexpr (WF == GEMM_W_Q4_K || WF == GEMM_W_IQ4_XS) {
       run(0, 0, 4);
       run(4, 4 + 4 * h, 4);
-    } else if constexpr (WF == GEMM_W_Q5_K) {
-      run(0, 0, 4);
-      run(4, 8 + 4 * h, 4);
-      w[8] = wb[4 + 2 * (c & 1) + h];
-    } else if constexpr (WF == GEMM_W_Q2_K) {
-      run(0, 0, 12);
-      w[12] = wb[15];
     } else if constexpr (WF == GEMM_W_Q8_0) {
       run(0, 12 * h, 8);
       w[8] = wb[12 * h + 11];
@@ -642,7 +635,8 @@ struct TileIO {
       run(0, 8 * h, 8);
       run(8, 16 + 2 * h, 2);
       run(10, 20 + 2 * h, 2);
-    } else {  // Q4_0, IQ4_NL
+    } else {
+      static_assert(WF == GEMM_W_Q4_0 || WF == GEMM_W_IQ4_NL, "not a format of the span kernel");
       run(0, 8 * h, 4);
       w[4] = wb[4];
     }

@@ -133,6 +133,8 @@ enum { GEMM_W_Q4_0 = 0, GEMM_W_PACKED = 1, GEMM_W_F16 = 2, GEMM_W_F32 = 3, GEMM_
 // The format that reads matrices of `qtype` as they are stored, -1 if there is
 // none (Q3_K, Q6_K, Q8_K and the other IQ types, read as packed units).
 int gemm_stored_format(int qtype, int K);
+// The same for the span kernel, where unpacking costs more than packed units do (-1).
+int gemm_span_format(int qtype, int K);
 struct GemmArgs {
   int qtype;
   int packed;             // GEMM_W_*: how w is stored
@@ -183,12 +185,12 @@ hipError_t gemm_launch(const GemmArgs& a, int num_cus, hipStream_t st, int* spli
 // One format's instances (gemm_<format>.hip): column tiles per wave, then row
 // tiles per wave (one-plane kernel) or ring stages (span kernel).
 #define CN_GEMM_SPAN(f) hipError_t gemm_##f##_span(const GemmArgs& a, int tn, int stages, int grid, hipStream_t st);
-#define CN_GEMM_FMT(f) \
-  hipError_t gemm_##f##_plane(const GemmArgs& a, int tn, int mt, int grid, hipStream_t st); \
-  CN_GEMM_SPAN(f)
+#define CN_GEMM_PLANE(f) hipError_t gemm_##f##_plane(const GemmArgs& a, int tn, int mt, int grid, hipStream_t st);
+#define CN_GEMM_FMT(f) CN_GEMM_PLANE(f) CN_GEMM_SPAN(f)
 CN_GEMM_FMT(q4_0) CN_GEMM_FMT(packed) CN_GEMM_FMT(q4_k) CN_GEMM_FMT(q8_0) CN_GEMM_FMT(q5_0) CN_GEMM_FMT(q4_1)
-CN_GEMM_FMT(q5_1) CN_GEMM_FMT(iq4_nl) CN_GEMM_FMT(q5_k) CN_GEMM_FMT(iq4_xs) CN_GEMM_FMT(q2_k) CN_GEMM_SPAN(f16)
+CN_GEMM_FMT(q5_1) CN_GEMM_FMT(iq4_nl) CN_GEMM_FMT(iq4_xs) CN_GEMM_PLANE(q5_k) CN_GEMM_PLANE(q2_k) CN_GEMM_SPAN(f16)
 CN_GEMM_SPAN(f16_x3) CN_GEMM_SPAN(f32)
+#undef CN_GEMM_PLANE
 #undef CN_GEMM_FMT
 #undef CN_GEMM_SPAN
 // x [N][K] fp32 -> the one-plane GEMM's input: xh[n] = fp16(x[n] * 2^e_n) in

@@ -161,8 +161,8 @@ CHATNET_API int chatnet_upload_tensor(chatnet_model* m, const char* name, uint32
  * products per step, exact weights), F32 rows split into fp16 hi + lo as
  * read (three products, ~22 bits), block types from their stored blocks when
  * every matrix of that GEMM is of one type (Q4_0: each weight exact as two
- * fp16 planes; Q4_1, Q5_0, Q5_1, Q8_0, Q2_K, Q4_K, Q5_K, IQ4_NL, IQ4_XS: ~22
- * bits), otherwise re-encoded once into packed units kept for the model's
+ * fp16 planes; Q4_1, Q5_0, Q5_1, Q8_0, Q4_K, and IQ4_NL and IQ4_XS but for rows
+ * of 2048 to 4095: ~22 bits), otherwise re-encoded once into packed units kept for the model's
  * lifetime (~22 bits).  Shorter spans, and models whose
  * layers give one GEMM matrices of both a float and a block type (ffn_gate
  * Q4_0 with ffn_up F16), run token by token. */
