@@ -1278,7 +1278,12 @@ int matmul_impl(uint32_t type, const void* w_dev, const float* x_dev, float* y_d
   // the GEMV reads only as packed units are packed for every N.
   constexpr int kColsGemv = 16;
   constexpr long long kTwoGemvs = 32LL << 20;
-  const int stored = gemm_stored_format((int)type, K);  // the GEMM's format on the stored blocks, -1: packed units
+  // The GEMM's format on the stored blocks, -1: packed units.  Q2_K's blocks are
+  // unpacked anew by every 128-column tile and cost the most: from the fourth on the
+  // packing pass and packed units are faster (32000 x 4096, packed and stored, us: 384
+  // columns 214 and 211, 448 232 and 288, 1024 389 and 575; 4096 x 11008 91 and 79,
+  // 116 and 124, 192 and 228).
+  const int stored = type == CHATNET_GGML_Q2_K && N > 384 ? -1 : gemm_stored_format((int)type, K);
   const bool must_pack = gemv_needs_pack((int)type);
   const bool ahead = packed_ahead(type);
   const bool batched = N >= 8 && !(N <= kColsGemv && gemv_qcols_supports((int)type)) &&

@@ -249,7 +249,7 @@ CHATNET_API int chatnet_get_logits(chatnet_model* m, float* logits_host);
  * run the dequant-to-LDS fp16 MFMA GEMM (x
  * rounded to fp16 after scaling each column by a power of two that keeps it
  * inside fp16's range, each weight rounded once to fp16; the blocks read as
- * stored, Q3_K, Q6_K, Q8_K and the other IQ types first re-encoded
+ * stored, Q3_K, Q6_K, Q8_K, the other IQ types and beyond 384 columns Q2_K first re-encoded
  * into the workspace as u8 codes with an fp32 scale and offset per 16 weights,
  * M*(K/64)*96 bytes, giving the same dequantized values).  F32 and F16 rows
  * with several columns run a multi-column GEMV (each column the N = 1

@@ -437,3 +437,18 @@ def test_stored_block_gemm_edges(qtype, M, K, N):
 def test_repacked_gemm_edges(qtype, M, K, N):
     """The bound of the stored blocks' test: one fp16 rounding of each operand."""
     test_stored_block_gemm_edges(qtype, M, K, N)
+
+
+@pytest.mark.parametrize("N", [384, 385])
+def test_q2_k_gemm_on_either_side_of_its_packing_line(N):
+    """The stored blocks' bound, and the no-allocation variant's bits."""
+    test_stored_block_gemm_edges(10, 130, 768, N)
+    M, K = 130, 768
+    t = synth.tensor(10, 72, "q2line", M, K)
+    x = synth.normal(73, "q2linex", N * K, 1.0).reshape(N, K)
+    ref = gpu_matmul(10, t.data, x, M, K)
+    w_d, x_d = hiprt.DeviceBuffer.from_numpy(t.data, pad=256), hiprt.DeviceBuffer.from_numpy(x)
+    y_d = hiprt.DeviceBuffer(4 * N * M)
+    _native.check(_native.hip_lib().chatnet_matmul_noalloc(10, w_d.ptr, x_d.ptr, y_d.ptr, M, K, N, None))
+    hiprt.synchronize()
+    assert np.array_equal(y_d.to_numpy(np.float32, N * M).reshape(N, M), ref)
