@@ -15,7 +15,8 @@
 //
 // What bounds it: joining, scaling and adding the digits (7 VALU instructions for 16
 // rows x 32 weights x 4 columns); dot4 on packed digits took 21 per 16 weights and
-// column, one launch per column the weight stream N times (18.9 us at 5 columns of
+// column, one launch per column the weight stream N times (per library call, calls
+// back to back: 18.9 us at 5 columns of
 // Q8_0 4864 x 896, here 5.3; the MFMA GEMM behind its packing pass 67.7 at 16 of Q4_K
 // 11008 x 4096, here 24.5).  Three digits, whose
 // results met a column at a time in fp32, took 12 for 5 columns: Q4_K 4096 x 4096 at

@@ -4,7 +4,8 @@
 // The columns' fp32 records (stage_fp32's) lie in LDS together and every group of
 // 16 weights, unpacked once, meets all of them: one pass over W, where one launch
 // per column reads and unpacks it again each time.  Bound by the fma per weight and
-// column and by the LDS reads of x, which two rows share: Q5_0 11008 x 4096 at 3
+// column and by the LDS reads of x, which two rows share (per library call, calls back
+// to back): Q5_0 11008 x 4096 at 3
 // columns 13.8 us, at 7 26.9; a packing pass and a GEMV per column took 103 and 200,
 // the matrix-core product of x in 23-bit digits 14.9 and 21.7.  Rows whose columns do
 // not fit in LDS together run in groups: 4096 x 11008 at 7 columns 41.7 us.  Error
